@@ -2,7 +2,7 @@
 //
 // One step_forward_backward stage (time_schemes_mod.F90:102-118) of the SW
 // path is three launches:
-//   k_tend   an LDS-tiled stencil over 58 x 11 cells: the pole sums (in the
+//   k_tend   an LDS-tiled stencil over 60 x 11 cells: the pole sums (in the
 //            tiles next to the poles), m, mass fluxes, pv,
 //            ke, tangential winds, upwind pv on edges, then the forward
 //            tendencies du, dv and the updated, unfiltered gz
@@ -28,17 +28,15 @@ namespace gmc {
 
 namespace {
 
-// k_tend tile: one wavefront per tile row, lane q <-> column C0 - 3 + q
+// k_tend tile: one wavefront per tile row, lane q <-> column C0 - 2 + q
 constexpr int LC = kWave;               // 64 tile columns
-constexpr int HXL = 3;                  // column halo
-constexpr int TX = LC - 2 * HXL - 0;    // 58 output columns (q = 3 .. 60)
+constexpr int HXL = 2;                  // column halo: the west of pv_lat's four columns
+constexpr int TX = LC - 2 * HXL;        // 60 output columns (q = 2 .. 61)
+constexpr int LX = LC + 1;              // m and v_f rows in LDS: lane 63 also holds the column east of it
 // launch-shape parameters (the defaults are the measured best on MI355X;
 // the macros let a sweep build other shapes)
-#ifndef GMC_RPW_MAIN
-#define GMC_RPW_MAIN 1
-#endif
 #ifndef GMC_TY_MAIN
-#define GMC_TY_MAIN (GMC_RPW_MAIN == 2 ? 27 : 11)
+#define GMC_TY_MAIN 11
 #endif
 #ifndef GMC_FILTER_THREADS
 #define GMC_FILTER_THREADS 256
@@ -50,25 +48,17 @@ constexpr int TX = LC - 2 * HXL - 0;    // 58 output columns (q = 3 .. 60)
 #define GMC_NARROW_CHUNK (2 * GMC_FILTER_THREADS)
 #endif
 constexpr int TY_MAIN = GMC_TY_MAIN;    // output rows of the single-member k_tend tile
-constexpr int RPW_MAIN = GMC_RPW_MAIN;  // its tile rows per wavefront
 constexpr int NF = GMC_FILTER_THREADS;  // threads per workgroup of the filter kernels
 constexpr int NXCD = 8;                 // XCDs of an MI355X
 // A k_tend tile with TY output rows: LR = TY + 5 tile rows (r = R0-2 ..
-// R0+TY+2), RPW tile rows per wavefront: wavefront w owns the tile rows
-// w, w + NW, .. (NW = LR / RPW wavefronts).
-template <int TY_, int RPW_ = 1> struct Tile {
+// R0+TY+2), one wavefront each.
+template <int TY_> struct Tile {
   static constexpr int TY = TY_;
-  static constexpr int RPW = RPW_;
   static constexpr int LR = TY + 5;
-  static_assert(LR % RPW == 0, "the tile rows split evenly over the wavefronts");
-  static constexpr int NW = LR / RPW;
-  static constexpr int NT = NW * kWave;
-  static constexpr int NE = LR * LC;
-  static constexpr int SH_TILES = 7 * NE;                 // LDS field tiles
-  static constexpr int SH_MESH = LR * kRowRec;            // metric row records of the tile
-  static constexpr int NREC = (SH_MESH + NT - 1) / NT;    // record words per thread
-  static constexpr int SH_ALL = SH_TILES + SH_MESH + 8;
-  static constexpr int kMaxPoleLon = SH_TILES / 3;        // the pole sums keep 3 row terms in the tile area
+  static constexpr int NT = LR * kWave;
+  static constexpr int SH_TILES = LR * (2 * LX + 5 * LC);   // LDS field tiles
+  static constexpr int SH_ALL = SH_TILES + 8;
+  static constexpr int kMaxPoleLon = SH_TILES / 3;          // the pole sums keep 3 row terms in the tile area
 };
 
 struct StagePtrs {
@@ -127,93 +117,106 @@ __device__ void pole_sums(const Grid &g, const MT &M, double grav, double rgrav,
     t2[i] = north ? ul * le : -ul * le;
   }
   __syncthreads();
-  if (tid < kWave) {
-    const double ske = wave_zonal_sum(n, tid, [&](int i) { return t0[i]; });
-    const double smf = wave_zonal_sum(n, tid, [&](int i) { return t1[i]; });
-    const double svo = wave_zonal_sum(n, tid, [&](int i) { return t2[i]; });
-    if (tid == 0) {
+  // one wavefront per sum (workgroups here have at least three)
+  const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
+  if (w < 3) {
+    const double s = wave_zonal_sum_batched(n, tid % kWave, scratch + w * n);
+    if (tid % kWave == 0) {
       const double nl = (double)n;
-      pole[north] = ske / nl;
-      pole[2 + north] = smf * le / nl / ac;
-      pole[4 + north] = svo / nl / ac;
+      pole[2 * w + north] = w == 0 ? s / nl : (w == 1 ? s * le / nl / ac : s / nl / ac);
     }
   }
   __syncthreads();
 }
 
-// Metric rows of one tile in LDS (row records, tile row k = r - r0):
-// M(f, r) is a broadcast LDS read for a wave-uniform r.  The records carry
-// the reciprocals of the divisor fields, so M.div divides through div_rn.
-struct MeshTile {
-  const double *s;
-  int r0;
-  __device__ __forceinline__ double operator()(int f, int r) const { return s[(r - r0) * kRowRec + f]; }
-  __device__ __forceinline__ double div(double x, int f, int r) const {
-    const double *rec = s + (r - r0) * kRowRec;
-    return div_rn(x, rec[f], rec[GMC_MESH_NFIELDS + recip_slot(f)]);
+// Row records of the metric table in the constant address space: a record
+// index uniform over the wavefront makes every access a scalar load, so the
+// metric terms sit in scalar registers and take neither LDS nor vector ones.
+typedef const __attribute__((address_space(4))) double *RecPtr;
+
+// The records of rows r - 1, r, r + 1 for the point formulas: M(f, r') and
+// M.div(x, f, r'), which divides through the record's reciprocal.  Rows
+// beyond the table read its zero records.  (Forcing a phase's terms to be
+// loaded ahead of its barrier spilled scalar registers and was slower.)
+struct MeshRow {
+  RecPtr m1, c0, p1;
+  int r;
+  __device__ __forceinline__ MeshRow(RecPtr base, int nlat, int r_) : r(r_) {
+    auto rec = [&](int rr) { return base + (min(max(rr, -1), nlat) + 1) * kRowRec; };
+    m1 = rec(r - 1);
+    c0 = rec(r);
+    p1 = rec(r + 1);
+  }
+  __device__ __forceinline__ RecPtr at(int rr) const { return rr == r ? c0 : rr > r ? p1 : m1; }
+  __device__ __forceinline__ double operator()(int f, int rr) const { return at(rr)[f]; }
+  __device__ __forceinline__ double div(double x, int f, int rr) const {
+    return div_rn(x, at(rr)[f], at(rr)[GMC_MESH_NFIELDS + recip_slot(f)]);
   }
 };
 
-// The global loads of one tile, per lane and tile row of its wavefront: gz,
-// gzs, u_f, v_f of its tile point and gz_old of its output point; and its
-// words of the metric records.
-template <class S> struct TileIn {
-  double gz[S::RPW], gzs[S::RPW], uf[S::RPW], vf[S::RPW], gz_old[S::RPW];
-  double rec[S::NREC];
+// Pointers typed in the global address space, and element i of a row whose
+// base is uniform over the wavefront through a 32-bit byte offset: the access
+// takes the scalar base and one vector register (a row is far below 4 GiB).
+template <class T> using gptr = __attribute__((address_space(1))) T *;
+template <class T> __device__ __forceinline__ gptr<T> glb(T *p) { return (gptr<T>)p; }
+template <class PT> __device__ __forceinline__ double row_ld(PT row, unsigned i) {
+  return *(gptr<const double>)((gptr<const char>)row + i * 8u);
+}
+template <class PT> __device__ __forceinline__ void row_st(PT row, unsigned i, double v) {
+  *(gptr<double>)((gptr<char>)row + i * 8u) = v;
+}
+
+// The value of the lane west (east) of this one, by a wavefront shift of the
+// vector registers: every lane must be active; lane 0 (63) gets 0.
+template <int CTRL> __device__ __forceinline__ double lane_shift(double x) {
+  union { double d; int i[2]; } u{x};
+  u.i[0] = __builtin_amdgcn_update_dpp(0, u.i[0], CTRL, 0xf, 0xf, true);
+  u.i[1] = __builtin_amdgcn_update_dpp(0, u.i[1], CTRL, 0xf, 0xf, true);
+  return u.d;
+}
+__device__ __forceinline__ double lane_west(double x) { return lane_shift<0x138>(x); }   // wave_shr:1
+__device__ __forceinline__ double lane_east(double x) { return lane_shift<0x130>(x); }   // wave_shl:1
+
+// The global loads of one tile row per lane: gz, gzs, u_f, v_f of its tile
+// point, and on lane 63 gz, gzs and v_f of the column east of the tile.
+struct TileIn {
+  double gz, gzs, uf, vf, gz_x, gzs_x, vf_x;
 };
 
-template <class S, class PT, class RT>
-__device__ __forceinline__ TileIn<S> tile_fetch(const Grid &g, RT mrows, const PT &P, int C0, int R0) {
+template <class S, class PT>
+__device__ __forceinline__ TileIn tile_fetch(const Grid &g, const PT &P, int C0, int R0) {
   const int64_t p = g.pitch;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int q = threadIdx.x % kWave;
-  const int i = wrap(C0 - HXL + q, g.nlon);
+  const int k = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int q = threadIdx.x % kWave, r = R0 - 2 + k;
   const int ic = C0 + q - HXL;
-  TileIn<S> in;
-#pragma unroll
-  for (int h = 0; h < S::RPW; h++) {
-    const int k = w + h * S::NW, r = R0 - 2 + k;
-    in.gz[h] = in.gzs[h] = in.uf[h] = in.vf[h] = in.gz_old[h] = 0.0;
-    if (k >= 2 && k < S::TY + 2 && q >= HXL && q < HXL + TX && ic < g.nlon && r < g.nlat)
-      in.gz_old[h] = P.gz_old[r * p + ic];
-    if (r >= 0 && r < g.nlat) {
-      in.gz[h] = P.gz_star[r * p + i];
-      in.gzs[h] = P.gzs[r * p + i];
-      in.uf[h] = P.u_f[r * p + i];
-    }
-    if (r >= 0 && r < g.nhalf) in.vf[h] = P.v_f[r * p + i];
-  }
-#pragma unroll
-  for (int j = 0; j < S::NREC; j++) {
-    const int t = threadIdx.x + j * S::NT;
-    in.rec[j] = 0.0;
-    if (t < S::SH_MESH) {
-      const int rr = R0 - 2 + t / kRowRec;
-      if (rr >= 0 && rr < g.nlat) in.rec[j] = mrows[(int64_t)(rr + 1) * kRowRec + t % kRowRec];
+  // a lane beyond a narrow grid's east side only has to stay in its row
+  const int i = min(wrap(ic, g.nlon), g.nlon - 1);
+  TileIn in{};
+  if (r >= 0 && r < g.nlat) {
+    in.gz = row_ld(P.gz_star + r * p, i);
+    in.gzs = row_ld(P.gzs + r * p, i);
+    in.uf = row_ld(P.u_f + r * p, i);
+    if (r < g.nhalf) in.vf = row_ld(P.v_f + r * p, i);
+    if (q == LC - 1) {
+      const int ix = min(wrap(ic + 1, g.nlon), g.nlon - 1);
+      in.gz_x = row_ld(P.gz_star + r * p, ix);
+      in.gzs_x = row_ld(P.gzs + r * p, ix);
+      if (r < g.nhalf) in.vf_x = row_ld(P.v_f + r * p, ix);
     }
   }
   return in;
 }
 
 // Pole sums of the star state into the tile's pole slots, in the tiles that
-// read them (a uniform branch per workgroup).  Runs before the tile's loads
-// are fetched: it uses the tile's LDS as scratch.
+// read them (a uniform branch per workgroup); uses the tile's LDS as scratch.
 template <class S, class MT, class PT>
 __device__ __forceinline__ void tile_poles(const Grid &g, const MT &Mg, double grav, double rgrav, const PT &P, int R0,
                                            double *sh) {
-  double *pole = sh + S::SH_TILES + S::SH_MESH;
+  double *pole = sh + S::SH_TILES;
   if (R0 <= 2) pole_sums<S::NT>(g, Mg, grav, rgrav, P, 0, sh, pole);
   if (R0 + S::TY + 3 >= g.nlat - 1) pole_sums<S::NT>(g, Mg, grav, rgrav, P, 1, sh, pole);
 }
 
-// The stage's intermediates of the star state that the adjoint reads (the
-// fields operators_prepare leaves, on the rows it writes them): written by
-// the taping tile for its own output points.
-// One tile of the forward tendencies and the unfiltered gz update: output
-// columns C0 .. C0+TX-1, rows R0 .. R0+TY-1, LDS scratch sh[S::SH_ALL].  The
-// tile's pole slots hold its pole sums (tile_poles) and io its loads
-// (tile_fetch) on entry.  With TAPE the tile also writes the intermediates
-// of its output points to *tape.
 // the six upwind derivatives of one edge point into a tape
 __device__ __forceinline__ void tape_upwind(double *const *dst, int64_t o, const UpwD &d) {
   dst[0][o] = d.dt;
@@ -222,253 +225,198 @@ __device__ __forceinline__ void tape_upwind(double *const *dst, int64_t o, const
   for (int j = 0; j < 4; j++) dst[2 + j][o] = d.df[j];
 }
 
+// One tile of the forward tendencies and the unfiltered gz update: output
+// columns C0 .. C0+TX-1, rows R0 .. R0+TY-1, LDS scratch sh[S::SH_ALL].  The
+// tile's pole slots hold its pole sums (tile_poles) and io its loads
+// (tile_fetch) on entry.  With TAPE the tile also writes the star state's
+// intermediates of its output points to *tape.
+//
+// A wavefront owns one tile row in every phase and all its 64 lanes run every
+// formula, so the columns on either side come from wavefront shifts and only
+// the rows on either side from LDS (16 reads a point); the lanes whose stencil
+// leaves the tile form values that no output point reads.  Reading both kinds
+// of neighbour and the metric rows from LDS (90 reads a point) kept the LDS
+// pipe, which a CU's four SIMDs share, busy for half of the launch.
 template <class S, bool TAPE = false, class MT, class PT>
-__device__ __forceinline__ void tend_tile(const Grid &g, const MT &Mg, double grav, double rgrav,
+__device__ __forceinline__ void tend_tile(const Grid &g, const MT &Mg, RecPtr mrows, double grav, double rgrav,
                                           double dt, int stokes, int pv_scheme, int order, double wgt, int coriolis,
-                                          const PT &P, int C0, int R0, double *sh, const TileIn<S> &io,
+                                          const PT &P, int C0, int R0, double *sh, const TileIn &io,
                                           const TapeOut *tape = nullptr) {
-  double(*sm)[LC] = (double(*)[LC])(sh + 0 * S::NE);
-  double(*suf)[LC] = (double(*)[LC])(sh + 1 * S::NE);
-  double(*svf)[LC] = (double(*)[LC])(sh + 2 * S::NE);
-  double(*smfx)[LC] = (double(*)[LC])(sh + 3 * S::NE);
-  double(*smfy)[LC] = (double(*)[LC])(sh + 4 * S::NE);
-  double(*spv)[LC] = (double(*)[LC])(sh + 5 * S::NE);
-  double(*ske)[LC] = (double(*)[LC])(sh + 6 * S::NE);
-  double(*spl)[LC] = suf;  // pv_lon replaces u_f element by element (phase D)
-  double(*spt)[LC] = svf;  // pv_lat replaces v_f element by element (phase D)
-  double *sme = sh + S::SH_TILES;
-  const double *pole = sh + S::SH_TILES + S::SH_MESH;
+  double(*sm)[LX] = (double(*)[LX])sh;
+  double(*svf)[LX] = (double(*)[LX])(sh + S::LR * LX);
+  double *shc = sh + 2 * S::LR * LX;
+  double(*suf)[LC] = (double(*)[LC])shc;
+  double(*smfx)[LC] = (double(*)[LC])(shc + 1 * S::LR * LC);
+  double(*smfy)[LC] = (double(*)[LC])(shc + 2 * S::LR * LC);
+  double(*spv)[LC] = (double(*)[LC])(shc + 3 * S::LR * LC);
+  double(*ske)[LC] = (double(*)[LC])(shc + 4 * S::LR * LC);
+  double(*spl)[LC] = suf;  // pv_lon and pv_lat replace u_f and v_f, which
+  double(*spt)[LX] = svf;  // no row reads from LDS after phase B
+  const double *pole = sh + S::SH_TILES;
 
   const int64_t p = g.pitch;
   const int nlat = g.nlat, nhalf = g.nhalf;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // wavefront: tile rows w, w + NW, ..
+  const int k = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // tile row of this wavefront
   const int q = threadIdx.x % kWave;                                   // tile column of this lane
-  const int i = wrap(C0 - HXL + q, g.nlon);                            // global column
-  const int ic = C0 + q - HXL;                                         // output column of this lane (phase E)
-  // tile row k of the wavefront's h-th row, its global row (wave-uniform)
-  // and whether the lane holds an output point there
-#define TILE_ROW(h)                                   \
-  const int k = w + (h) * S::NW;                      \
-  const int r = R0 - 2 + k;                           \
+  const int r = R0 - 2 + k;                                            // global row
+  const int ic = C0 + q - HXL;                                         // output column
+  const int kn = min(k + 1, S::LR - 1), ks = max(k - 1, 0), kss = max(k - 2, 0);
   const bool out_pt = k >= 2 && k < S::TY + 2 && q >= HXL && q < HXL + TX && ic < g.nlon && r < nlat;
+  const bool u_row = r >= 1 && r <= nlat - 2, v_row = r >= 0 && r < nhalf;
+  const int64_t o = r * p + ic;
+  const MeshRow M(mrows, nlat, r);
 
-  // A: m, u_f, v_f of the wavefront's tile rows and the tile's metric rows
-#pragma unroll
-  for (int h = 0; h < S::RPW; h++) {
-    TILE_ROW(h)
-    sm[k][q] = (r >= 0 && r < nlat) ? div_rn(io.gz[h] - io.gzs[h], grav, rgrav) : 0.0;   // m_of
-    suf[k][q] = io.uf[h];
-    svf[k][q] = io.vf[h];
-    if (TAPE && out_pt && tape->u_f) {
-      tape->u_f[r * p + ic] = io.uf[h];
-      if (r < nhalf) tape->v_f[r * p + ic] = io.vf[h];
-    }
+  // A: m, u_f, v_f of the row
+  const double uf = io.uf, vf = io.vf;
+  const double m0 = div_rn(io.gz - io.gzs, grav, rgrav);   // m_of; 0 beyond the poles
+  sm[k][q] = m0;
+  svf[k][q] = vf;
+  suf[k][q] = uf;
+  if (q == LC - 1) {
+    sm[k][LC] = div_rn(io.gz_x - io.gzs_x, grav, rgrav);
+    svf[k][LC] = io.vf_x;
   }
-#pragma unroll
-  for (int j = 0; j < S::NREC; j++) {
-    const int t = threadIdx.x + j * S::NT;
-    if (t < S::SH_MESH) sme[t] = io.rec[j];
+  if (TAPE && out_pt && tape->u_f) {
+    tape->u_f[o] = uf;
+    if (v_row) tape->v_f[o] = vf;
   }
-  const MeshTile M{sme, R0 - 2};
   __syncthreads();
 
-  // B: mass fluxes (rows 1 .. TY+2), pv (rows 0 .. TY+3), ke (rows 2 .. TY+2).
-  // Tile rows that need all three away from the poles form them in one block,
-  // so that the compiler interleaves the three dependency chains; the lanes
-  // that block adds (mass fluxes on lane 1, ke on lanes 1, 2 and 62) write
-  // tile elements that no later phase reads.
-#pragma unroll
-  for (int h = 0; h < S::RPW; h++) {
-  TILE_ROW(h)
-  if (!TAPE && k >= 2 && k < S::TY + 3 && r >= 1 && r <= nlat - 3) {
-    if (q >= 1 && q < 63) {
-      const double m0 = sm[k][q], m1 = sm[k][q + 1], m2 = sm[k + 1][q], m3 = sm[k + 1][q + 1];
-      const double u0 = suf[k][q], u1 = suf[k + 1][q], uw = suf[k][q - 1];
-      const double v0 = svf[k][q], v1 = svf[k][q + 1], vs = svf[k - 1][q];
-      smfx[k][q] = (m0 + m1) * 0.5 * u0;
-      smfy[k][q] = (m0 + m2) * 0.5 * v0;
-      spv[k][q] = pv_of(vor_of(u0, u1, v1, v0, M, r), M, r, m_vtx_of(m0, m1, m2, m3, M, r));
-      ske[k][q] = ke_of(uw, u0, vs, v0, M, r);
+  // B: mass fluxes (rows 1 .. TY+2), pv (rows 0 .. TY+3), ke (rows 2 .. TY+2),
+  // the row's three chains in one block; then what the rows at and beyond the
+  // poles hold instead
+  const double m1 = sm[k][q + 1], m2 = sm[kn][q], m3 = sm[kn][q + 1];
+  const double u1 = suf[kn][q], v1 = svf[k][q + 1], vs = svf[ks][q], uw = lane_west(uf);
+  double mfx = (m0 + m1) * 0.5 * uf;
+  double mfy = (m0 + m2) * 0.5 * vf;
+  const double mv = m_vtx_of(m0, m1, m2, m3, M, r);
+  double pv = pv_of(vor_of(uf, u1, v1, vf, M, r), M, r, mv);
+  double ke = ke_of(uw, uf, vs, vf, M, r);
+  if (r < 2 || r > nlat - 3) {
+    if (!u_row) {
+      mfx = 0.0;
+      ke = r == 0 ? pole[0] : r == nlat - 1 ? pole[1] : 0.0;
     }
-  } else {
-  if (k >= 1 && k < S::TY + 3 && q >= 2 && q < 63) {
-    smfx[k][q] = (r >= 1 && r <= nlat - 2) ? (sm[k][q] + sm[k][q + 1]) * 0.5 * suf[k][q] : 0.0;
-    smfy[k][q] = (r >= 0 && r < nhalf) ? (sm[k][q] + sm[k + 1][q]) * 0.5 * svf[k][q] : 0.0;
-  }
-  if (k < S::TY + 4 && q >= 1 && q < 63) {
-    double v = 0.0;
-    if (r >= 0 && r < nhalf) {
-      double vor;
-      if (stokes && r == 0) vor = pole[4];
-      else if (stokes && r == nhalf - 1) vor = pole[5];
-      else vor = vor_of(suf[k][q], suf[k + 1][q], svf[k][q + 1], svf[k][q], M, r);
-      const double mv = m_vtx_of(sm[k][q], sm[k][q + 1], sm[k + 1][q], sm[k + 1][q + 1], M, r);
-      v = pv_of(vor, M, r, mv);
-      if (TAPE && out_pt) {
-        tape->m_vtx[r * p + ic] = mv;
-        tape->pv[r * p + ic] = v;
-        tape->mfy[r * p + ic] = smfy[k][q];
-        tape->m_lat[r * p + ic] = (sm[k][q] + sm[k + 1][q]) * 0.5;
+    if (!v_row) {
+      mfy = 0.0;
+      pv = 0.0;
+      if (r >= -2 && r <= nhalf + 1) {
+        int rr = r, ii = min(wrap(ic, g.nlon), g.nlon - 1);
+        mirror_half(rr, ii, g);
+        pv = pv_global(g, Mg, grav, rgrav, stokes, pole, P, rr, ii);
       }
-    } else if (r >= -2 && r <= nhalf + 1) {
-      int rr = r, ii = i;
-      mirror_half(rr, ii, g);
-      v = pv_global(g, Mg, grav, rgrav, stokes, pole, P, rr, ii);
+    } else if (stokes && (r == 0 || r == nhalf - 1)) {
+      pv = pv_of(r == 0 ? pole[4] : pole[5], M, r, mv);
     }
-    spv[k][q] = v;
   }
-  if (k >= 2 && k < S::TY + 3 && q >= 3 && q < 62) {
-    double v = 0.0;
-    if (r == 0) v = pole[0];
-    else if (r == nlat - 1) v = pole[1];
-    else if (r > 0 && r < nlat - 1) v = ke_of(suf[k][q - 1], suf[k][q], svf[k - 1][q], svf[k][q], M, r);
-    ske[k][q] = v;
-  }
-  }
+  smfx[k][q] = mfx;
+  smfy[k][q] = mfy;
+  spv[k][q] = pv;
+  ske[k][q] = ke;
+  if (TAPE && out_pt && v_row) {
+    tape->m_vtx[o] = mv;
+    tape->pv[o] = pv;
+    tape->mfy[o] = mfy;
+    tape->m_lat[o] = (m0 + m2) * 0.5;
   }
   __syncthreads();
 
-  // D: tangential winds and pv on the edges.  v_lon (U rows 2 .. TY+2) and
-  // u_lat (V rows 1 .. TY+1) are each read only by the lane that forms them,
-  // so they stay in registers; pv_lon replaces u_f and pv_lat replaces v_f
-  // element by element (each lane reads only its own u_f / v_f here, in each
-  // of its rows).
-#pragma unroll
-  for (int h = 0; h < S::RPW; h++) {
-  TILE_ROW(h)
+  // D: tangential winds and pv on the edges (U rows 2 .. TY+2, V rows 1 ..
+  // TY+1); phase E's gz_old is on its way meanwhile
+  double gz_old = 0.0;
+  if (out_pt) gz_old = row_ld(P.gz_old + r * p, ic);
+  const double mfy_s = smfy[ks][q], mfx_n = smfx[kn][q];
   double pl = 0.0, pt = 0.0;
-  if (!TAPE && k >= 2 && k < S::TY + 2 && r >= 1 && r <= nlat - 2) {
-    // both edges in one block (interleaved chains); lane 2 forms a pv_lat
-    // that is replaced by the 0 the edge loop below leaves there
-    if (q >= 2 && q < 62) {
-      const double tl = tangent_sum(M(GMC_FULL_TANGENT_WGT1, r), M(GMC_FULL_TANGENT_WGT2, r), smfy[k - 1][q],
-                                    smfy[k - 1][q + 1], smfy[k][q], smfy[k][q + 1]);
-      const double tu = tangent_sum(M(GMC_HALF_TANGENT_WGT1, r), M(GMC_HALF_TANGENT_WGT2, r), smfx[k][q - 1],
-                                    smfx[k][q], smfx[k + 1][q - 1], smfx[k + 1][q]);
-      const double vl = tl / ((sm[k][q] + sm[k][q + 1]) * 0.5);
-      const double ul = tu / ((sm[k][q] + sm[k + 1][q]) * 0.5);
-      const double el = pv_edge(pv_scheme, order, wgt, vl, suf[k][q], 0, dt, M(GMC_LE_LON, r), spv[k - 2][q],
-                                spv[k - 1][q], spv[k][q], spv[k + 1][q]);
-      const double et = pv_edge(pv_scheme, order, wgt, ul, svf[k][q], 1, dt, M(GMC_LE_LAT, r), spv[k][q - 2],
-                                spv[k][q - 1], spv[k][q], spv[k][q + 1]);
-      pl = el;
-      pt = q >= 3 ? et : 0.0;
+  if (k >= 1 && k < S::TY + 3) {
+    const double pss = spv[kss][q], ps = spv[ks][q], pn = spv[kn][q];
+    const double pw = lane_west(pv), pww = lane_west(pw), pe = lane_east(pv);
+    const double tl = tangent_sum(M(GMC_FULL_TANGENT_WGT1, r), M(GMC_FULL_TANGENT_WGT2, r), mfy_s, lane_east(mfy_s),
+                                  mfy, lane_east(mfy));
+    const double tu = tangent_sum(M(GMC_HALF_TANGENT_WGT1, r), M(GMC_HALF_TANGENT_WGT2, r), lane_west(mfx), mfx,
+                                  lane_west(mfx_n), mfx_n);
+    const double vl = div_mid(tl, (m0 + m1) * 0.5);
+    const double ul = div_mid(tu, (m0 + m2) * 0.5);
+    if (pv_scheme == GMC_PV_UPWIND && order == 3) {   // both edges in one block
+      pl = pv_upwind_edge(3, wgt, vl, uf, 0, pss, ps, pv, pn);
+      pt = pv_upwind_edge(3, wgt, ul, vf, 1, pww, pw, pv, pe);
+    } else {
+      pl = pv_edge(pv_scheme, order, wgt, vl, uf, 0, dt, M(GMC_LE_LON, r), pss, ps, pv, pn);
+      pt = pv_edge(pv_scheme, order, wgt, ul, vf, 1, dt, M(GMC_LE_LAT, r), pww, pw, pv, pe);
     }
-  } else {
-  if (k >= 2 && k < S::TY + 3 && q >= 2 && q < 62 && r >= 1 && r <= nlat - 2) {
-    const double tt = tangent_sum(M(GMC_FULL_TANGENT_WGT1, r), M(GMC_FULL_TANGENT_WGT2, r), smfy[k - 1][q],
-                                  smfy[k - 1][q + 1], smfy[k][q], smfy[k][q + 1]);
-    const double vl = tt / ((sm[k][q] + sm[k][q + 1]) * 0.5);
-    const double a1 = spv[k - 2][q], a2 = spv[k - 1][q], a3 = spv[k][q], a4 = spv[k + 1][q];
-    pl = pv_edge(pv_scheme, order, wgt, vl, suf[k][q], 0, dt, M(GMC_LE_LON, r), a1, a2, a3, a4);
+    if (!u_row) pl = 0.0;
+    if (!v_row) pt = 0.0;
     if (TAPE && out_pt) {
-      tape->m_lon[r * p + ic] = (sm[k][q] + sm[k][q + 1]) * 0.5;
-      tape->mfx[r * p + ic] = smfx[k][q];
-      if (tape->mfy_lon) tape->mfy_lon[r * p + ic] = tt;
-      tape->v_lon[r * p + ic] = vl;
-      tape->pv_lon[r * p + ic] = pl;
-      if (tape->dlon[0]) tape_upwind(tape->dlon, r * p + ic,
-                                     upwind_deriv(pv_scheme, order, wgt, vl, suf[k][q], 0, a1, a2, a3, a4));
+      if (u_row) {
+        tape->m_lon[o] = (m0 + m1) * 0.5;
+        tape->mfx[o] = mfx;
+        if (tape->mfy_lon) tape->mfy_lon[o] = tl;
+        tape->v_lon[o] = vl;
+        tape->pv_lon[o] = pl;
+        if (tape->dlon[0]) tape_upwind(tape->dlon, o, upwind_deriv(pv_scheme, order, wgt, vl, uf, 0, pss, ps, pv, pn));
+      }
+      if (v_row) {
+        if (tape->mfx_lat) tape->mfx_lat[o] = tu;
+        tape->u_lat[o] = ul;
+        tape->pv_lat[o] = pt;
+        if (tape->dlat[0]) tape_upwind(tape->dlat, o, upwind_deriv(pv_scheme, order, wgt, ul, vf, 1, pww, pw, pv, pe));
+      }
     }
-  }
-  if (k >= 1 && k < S::TY + 2 && q >= 3 && q < 62 && r >= 0 && r < nhalf) {
-    const double tt = tangent_sum(M(GMC_HALF_TANGENT_WGT1, r), M(GMC_HALF_TANGENT_WGT2, r), smfx[k][q - 1],
-                                  smfx[k][q], smfx[k + 1][q - 1], smfx[k + 1][q]);
-    const double ul = tt / ((sm[k][q] + sm[k + 1][q]) * 0.5);
-    const double a1 = spv[k][q - 2], a2 = spv[k][q - 1], a3 = spv[k][q], a4 = spv[k][q + 1];
-    pt = pv_edge(pv_scheme, order, wgt, ul, svf[k][q], 1, dt, M(GMC_LE_LAT, r), a1, a2, a3, a4);
-    if (TAPE && out_pt) {
-      if (tape->mfx_lat) tape->mfx_lat[r * p + ic] = tt;
-      tape->u_lat[r * p + ic] = ul;
-      tape->pv_lat[r * p + ic] = pt;
-      if (tape->dlat[0]) tape_upwind(tape->dlat, r * p + ic,
-                                     upwind_deriv(pv_scheme, order, wgt, ul, svf[k][q], 1, a1, a2, a3, a4));
-    }
-  }
   }
   spl[k][q] = pl;
   spt[k][q] = pt;
-  }
   __syncthreads();
 
-  // E: du, dv (forward pass) and gz_new = gz_old + dt dgz on the output rows;
-  // rows away from the poles in one block
-#pragma unroll
-  for (int h = 0; h < S::RPW; h++) {
-  TILE_ROW(h)
-  const double gz_old = io.gz_old[h];
-  if (r >= 1 && r <= nlat - 2) {
-    if (out_pt) {
-      const int64_t o = r * p + ic;
-      const double qhv = coriolis == 1
-          ? qhv_of(M, r, spl[k][q], smfy[k - 1][q], spt[k - 1][q], smfy[k - 1][q + 1], spt[k - 1][q + 1],
-                   smfy[k][q], spt[k][q], smfy[k][q + 1], spt[k][q + 1])
-          : tangent_sum(M(GMC_FULL_TANGENT_WGT1, r), M(GMC_FULL_TANGENT_WGT2, r), smfy[k - 1][q],
-                        smfy[k - 1][q + 1], smfy[k][q], smfy[k][q + 1]) * spl[k][q];
-      const double dku = M.div(ske[k][q + 1] - ske[k][q], GMC_DE_LON, r);
-      const double qhu = coriolis == 1
-          ? qhu_of(M, r, spt[k][q], smfx[k][q - 1], spl[k][q - 1], smfx[k][q], spl[k][q],
-                   smfx[k + 1][q - 1], spl[k + 1][q - 1], smfx[k + 1][q], spl[k + 1][q])
-          : tangent_sum(M(GMC_HALF_TANGENT_WGT1, r), M(GMC_HALF_TANGENT_WGT2, r), smfx[k][q - 1], smfx[k][q],
-                        smfx[k + 1][q - 1], smfx[k + 1][q]) * spt[k][q];
-      const double dkv = M.div(ske[k + 1][q] - ske[k][q], GMC_DE_LAT, r);
-      const double dgz = -(dmfdlon_of(smfx[k][q], smfx[k][q - 1], M, r) +
-                           dmfdlat_of(smfy[k][q], smfy[k - 1][q], M, r)) * grav;
-      P.du[o] = qhv - dku;
-      P.dv[o] = -qhu - dkv;
-      P.gz_new[o] = gz_old + dt * dgz;
-    }
-    continue;
-  }
-  // the pole rows: v on the southern pole edge row, gz from the pole sums
-  if (out_pt) {
-    const int64_t o = r * p + ic;
-    if (r < nhalf) {
-      const double qhu = coriolis == 1
-          ? qhu_of(M, r, spt[k][q], smfx[k][q - 1], spl[k][q - 1], smfx[k][q], spl[k][q],
-                   smfx[k + 1][q - 1], spl[k + 1][q - 1], smfx[k + 1][q], spl[k + 1][q])
-          : tangent_sum(M(GMC_HALF_TANGENT_WGT1, r), M(GMC_HALF_TANGENT_WGT2, r), smfx[k][q - 1], smfx[k][q],
-                        smfx[k + 1][q - 1], smfx[k + 1][q]) * spt[k][q];
-      const double dk = M.div(ske[k + 1][q] - ske[k][q], GMC_DE_LAT, r);
-      P.dv[o] = -qhu - dk;
-    }
+  // E: du, dv (forward pass) and gz_new = gz_old + dt dgz on the output rows
+  if (k < 2 || k >= S::TY + 2) return;
+  const double pt_s = spt[ks][q], pt_se = lane_east(pt_s), pt_e = lane_east(pt);
+  const double pl_n = spl[kn][q], pl_nw = lane_west(pl_n), pl_w = lane_west(pl);
+  const double mfy_e = lane_east(mfy), mfy_se = lane_east(mfy_s), mfx_w = lane_west(mfx), mfx_nw = lane_west(mfx_n);
+  const double ke_0 = ske[k][q], ke_e = lane_east(ke_0), ke_n = ske[kn][q];
+  const double qhv = coriolis == 1
+      ? qhv_of(M, r, pl, mfy_s, pt_s, mfy_se, pt_se, mfy, pt, mfy_e, pt_e)
+      : tangent_sum(M(GMC_FULL_TANGENT_WGT1, r), M(GMC_FULL_TANGENT_WGT2, r), mfy_s, mfy_se, mfy, mfy_e) * pl;
+  const double qhu = coriolis == 1
+      ? qhu_of(M, r, pt, mfx_w, pl_w, mfx, pl, mfx_nw, pl_nw, mfx_n, pl_n)
+      : tangent_sum(M(GMC_HALF_TANGENT_WGT1, r), M(GMC_HALF_TANGENT_WGT2, r), mfx_w, mfx, mfx_nw, mfx_n) * pt;
+  const double dku = M.div(ke_e - ke_0, GMC_DE_LON, r);
+  const double dkv = M.div(ke_n - ke_0, GMC_DE_LAT, r);
+  double dgz = -(dmfdlon_of(mfx, mfx_w, M, r) + dmfdlat_of(mfy, mfy_s, M, r)) * grav;
+  if (!u_row) {   // the pole rows: gz from the pole sums
     const double dmfdlon = 0.0, dmfdlat = r == 0 ? pole[2] : pole[3];
-    const double dgz = -(dmfdlon + dmfdlat) * grav;
-    P.gz_new[o] = gz_old + dt * dgz;
+    dgz = -(dmfdlon + dmfdlat) * grav;
   }
+  if (out_pt) {
+    if (u_row) row_st(P.du + r * p, ic, qhv - dku);
+    if (v_row) row_st(P.dv + r * p, ic, -qhu - dkv);
+    row_st(P.gz_new + r * p, ic, gz_old + dt * dgz);
   }
-#undef TILE_ROW
 }
 
-// Forward tendencies and the unfiltered gz update on a 58 x TY_MAIN tile.
-// Wavefront w owns tile rows k = w, w + NW, .. (global row R0 - 2 + k) in
-// every phase and lane q the column C0 - 3 + q, so metric terms are
-// wave-uniform (broadcast LDS reads of the tile's metric rows) and each phase
-// is one pass over each of its rows.  Blocks are dealt to the XCDs
-// round-robin; each XCD gets a contiguous run of tiles (row-major), so
-// vertically adjacent tiles share that XCD's L2.  The XCD holding the north
-// pole walks its run backwards so that the polar tiles, which also form the
-// pole sums, start first.
-constexpr int kTendThreads = Tile<TY_MAIN, RPW_MAIN>::NT;
+// Forward tendencies and the unfiltered gz update on a 60 x TY_MAIN tile.
+// Wavefront k owns tile row k (global row R0 - 2 + k) in every phase and lane
+// q the column C0 - 2 + q, so metric terms are wave-uniform.  Blocks are
+// dealt to the XCDs round-robin; each XCD gets a contiguous run of tiles
+// (row-major), so vertically adjacent tiles share that XCD's L2.  The XCD
+// holding the north pole walks its run backwards so that the polar tiles,
+// which also form the pole sums, start first.
+constexpr int kTendThreads = Tile<TY_MAIN>::NT;
 template <bool TAPE>
-__global__ void __launch_bounds__(kTendThreads, 8 / RPW_MAIN) k_tend(Grid g, Mesh Mg, const double *__restrict__ mrows,
-                                                             double grav, double rgrav, double dt, int stokes,
-                                                             int pv_scheme, int order, double wgt, int coriolis,
-                                                             StagePtrs P, TapeOut tape) {
-  using S = Tile<TY_MAIN, RPW_MAIN>;
+__global__ void __launch_bounds__(kTendThreads, 8) k_tend(Grid g, Mesh Mg, const double *__restrict__ mrows,
+                                                          double grav, double rgrav, double dt, int stokes,
+                                                          int pv_scheme, int order, double wgt, int coriolis,
+                                                          StagePtrs P, TapeOut tape) {
+  using S = Tile<TY_MAIN>;
   __shared__ double sh[S::SH_ALL];
   // tile of this block
   const int nx = (g.nlon + TX - 1) / TX, ny = (g.nlat + S::TY - 1) / S::TY, T = nx * ny;
-  const int b = blockIdx.x, x = b % NXCD, s = b / NXCD;
-  int start = 0;
-  for (int y = 0; y < x; y++) start += (T - y + NXCD - 1) / NXCD;
-  const int cnt = (T - x + NXCD - 1) / NXCD;
-  const int t = start + (x == NXCD - 1 ? cnt - 1 - s : s);
+  const int b = blockIdx.x, x = b % NXCD;
+  const int t = x == NXCD - 1 ? T - 1 - b / NXCD : xcd_item(b, T);
   const int C0 = (t % nx) * TX, R0 = (t / nx) * S::TY;
 
+  const TileIn io = tile_fetch<S>(g, P, C0, R0);
   tile_poles<S>(g, Mg, grav, rgrav, P, R0, sh);
-  const TileIn<S> io = tile_fetch<S>(g, mrows, P, C0, R0);
-  tend_tile<S, TAPE>(g, Mg, grav, rgrav, dt, stokes, pv_scheme, order, wgt, coriolis, P, C0, R0, sh, io, &tape);
+  tend_tile<S, TAPE>(g, Mg, (RecPtr)mrows, grav, rgrav, dt, stokes, pv_scheme, order, wgt, coriolis, P, C0, R0, sh, io,
+                     &tape);
 }
 
 // ---------------------------------------------------------------------------
@@ -629,8 +577,6 @@ struct EnsMember {
 // ensemble kernels therefore hand the shared tile and item code pointers
 // typed in the global address space, so that it emits global loads and
 // stores as it does for pointers passed as kernel arguments.
-template <class T> using gptr = __attribute__((address_space(1))) T *;
-template <class T> __device__ __forceinline__ gptr<T> glb(T *p) { return (gptr<T>)p; }
 struct MeshG {
   gptr<const double> m;
   int nlat;
@@ -685,10 +631,10 @@ __global__ void __launch_bounds__(S::NT, 8) k_tend_ens(const EnsMember *__restri
     const int lt = t - d.tile0;
     const int C0 = (lt % d.nx) * TX, R0 = (lt / d.nx) * S::TY;
     const StagePtrsG sp = glb(d.sp);
+    const TileIn io = tile_fetch<S>(d.g, sp, C0, R0);
     tile_poles<S>(d.g, glb(d.M), d.grav, d.rgrav, sp, R0, sh);
-    const TileIn<S> io = tile_fetch<S>(d.g, glb(d.mrows), sp, C0, R0);
-    tend_tile<S>(d.g, glb(d.M), d.grav, d.rgrav, d.dt, d.stokes, d.pv_scheme, d.order, d.wgt, d.coriolis, sp, C0,
-                 R0, sh, io);
+    tend_tile<S>(d.g, glb(d.M), (RecPtr)d.mrows, d.grav, d.rgrav, d.dt, d.stokes, d.pv_scheme, d.order, d.wgt,
+                 d.coriolis, sp, C0, R0, sh, io);
     __syncthreads();
   }
 }
@@ -809,7 +755,7 @@ static int build_plan(gmc_ctx *c) {
     if (nb_lon[r] > g.nlon) return set_error(c, GMC_EINVAL, "filter wider than a latitude circle");
   for (int r = 0; r < g.nhalf; r++)
     if (nb_lat[r] > g.nlon) return set_error(c, GMC_EINVAL, "filter wider than a latitude circle");
-  if (g.nlon > Tile<TY_MAIN, RPW_MAIN>::kMaxPoleLon) return set_error(c, GMC_EINVAL, "nlon too large for the fused stage kernels");
+  if (g.nlon > Tile<TY_MAIN>::kMaxPoleLon) return set_error(c, GMC_EINVAL, "nlon too large for the fused stage kernels");
   std::vector<Item> items;
   FusedPlan *P = new FusedPlan();
 
@@ -894,7 +840,7 @@ static void fused_stage(gmc_ctx *c, int o, int s, int n, double dt, bool tape = 
   TapeOut T{S[S_M_LON], S[S_M_LAT], S[S_M_VTX], S[S_MFX_LON], S[S_MFY_LAT], S[S_MFX_LAT], S[S_MFY_LON],
             S[S_U_LAT], S[S_V_LON], S[S_PV], S[S_PV_LON], S[S_PV_LAT], nullptr, nullptr};
   if (dst) T = *dst;
-  stage_launch(c, tape ? k_tend<true> : k_tend<false>, dim3(tiles), dim3(Tile<TY_MAIN, RPW_MAIN>::NT), 0, g, M,
+  stage_launch(c, tape ? k_tend<true> : k_tend<false>, dim3(tiles), dim3(Tile<TY_MAIN>::NT), 0, g, M,
                c->d_mrows, c->cfg.g, 1.0 / c->cfg.g, dt, c->cfg.pv_pole_stokes, c->cfg.pv_scheme,
                pv_order(c->cfg), c->cfg.upwind_wgt_pv, c->cfg.coriolis_scheme, sp, T);
   stage_launch(c, k_gzf, dim3(PL->n_gz), dim3(NF), PL->lds_gz, g, c->big, c->small1, PL->d_items, gz_new,
@@ -1004,11 +950,11 @@ struct EnsShape {
   const char *name;
 };
 constexpr EnsShape kEnsShapes[] = {
-    {11, 0, "tile 58x11, one workgroup per tile"}, {7, 0, "tile 58x7, one workgroup per tile"},
-    {5, 0, "tile 58x5, one workgroup per tile"},   {11, 4, "tile 58x11, 1024 persistent workgroups"},
-    {7, 4, "tile 58x7, 1024 persistent workgroups"}, {5, 4, "tile 58x5, 1024 persistent workgroups"},
-    {11, 8, "tile 58x11, 2048 persistent workgroups"}, {7, 8, "tile 58x7, 2048 persistent workgroups"},
-    {5, 8, "tile 58x5, 2048 persistent workgroups"}};
+    {11, 0, "tile 60x11, one workgroup per tile"}, {7, 0, "tile 60x7, one workgroup per tile"},
+    {5, 0, "tile 60x5, one workgroup per tile"},   {11, 4, "tile 60x11, 1024 persistent workgroups"},
+    {7, 4, "tile 60x7, 1024 persistent workgroups"}, {5, 4, "tile 60x5, 1024 persistent workgroups"},
+    {11, 8, "tile 60x11, 2048 persistent workgroups"}, {7, 8, "tile 60x7, 2048 persistent workgroups"},
+    {5, 8, "tile 60x5, 2048 persistent workgroups"}};
 constexpr int kNumEnsShapes = sizeof(kEnsShapes) / sizeof(kEnsShapes[0]);
 
 int stage_count(int scheme) { return scheme == GMC_TIME_EULER ? 1 : 3; }
