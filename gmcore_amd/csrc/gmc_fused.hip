@@ -1,20 +1,22 @@
 // gmc_fused.hip -- fused stage kernels used by gmc_step / gmc_time_integrate.
 //
 // One step_forward_backward stage (time_schemes_mod.F90:102-118) of the SW
-// path is three launches:
-//   k_tend   an LDS-tiled stencil over 60 x 11 cells: the pole sums (in the
-//            tiles next to the poles), m, mass fluxes, pv,
-//            ke, tangential winds, upwind pv on edges, then the forward
-//            tendencies du, dv and the updated, unfiltered gz
-//            (operators_prepare_2 forward + calc_grad_mf + calc_coriolis +
-//            calc_grad_ke + the gz part of update_state);
-//   k_gzf    the big and small zonal filters of the new gz;
-//   k_uvf    the backward pass (pgf from gz_f), the u/v update with the
-//            pole-row smoothing, and the big filters to u_f, v_f.
-// The filter kernels run over a host-built work list of (row, column chunk)
-// items so that polar rows with hundreds of taps are spread over many
-// workgroups.  Every expression is the same point formula as the
-// operator-level kernels (gmc_point.hpp), so both paths give the same bits.
+// path is three steps:
+//   tendencies  an LDS-tiled stencil: the pole sums (in the tiles next to the
+//               poles), m, mass fluxes, pv, ke, tangential winds, upwind pv on
+//               edges, then the forward tendencies du, dv and the updated,
+//               unfiltered gz (operators_prepare_2 forward + calc_grad_mf +
+//               calc_coriolis + calc_grad_ke + the gz part of update_state);
+//   gz filters  the big and small zonal filters of the new gz;
+//   u and v     the backward pass (pgf from gz_f), the u/v update with the
+//               pole-row smoothing, and the big filters to u_f, v_f.
+// k_tend, k_gzf and k_uvf are those three over the whole grid.  k_stage, which
+// gmc_step runs, takes the rows of short filters through all three in one
+// tile, and the polar rows in bands of whole circles or in three launches.
+// The filter items are (row, column chunk) pieces from a host-built list, so
+// that polar rows with hundreds of taps are spread over many workgroups.
+// Every expression is the same point formula as the operator-level kernels
+// (gmc_point.hpp), so all paths give the same bits.
 #include <hip/hip_ext.h>
 
 #include <algorithm>
@@ -177,6 +179,12 @@ template <int CTRL> __device__ __forceinline__ double lane_shift(double x) {
 __device__ __forceinline__ double lane_west(double x) { return lane_shift<0x138>(x); }   // wave_shr:1
 __device__ __forceinline__ double lane_east(double x) { return lane_shift<0x130>(x); }   // wave_shl:1
 
+// What a tile owns: output columns c0 .. c0+nc-1 on the lanes from hl on, rows
+// r0 .. r1-1 (at most TY; the tile's local row k is global row r0 - 2 + k).
+struct TileGeo {
+  int c0, nc, hl, r0, r1;
+};
+
 // The global loads of one tile row per lane: gz, gzs, u_f, v_f of its tile
 // point, and on lane 63 gz, gzs and v_f of the column east of the tile.
 struct TileIn {
@@ -184,11 +192,11 @@ struct TileIn {
 };
 
 template <class S, class PT>
-__device__ __forceinline__ TileIn tile_fetch(const Grid &g, const PT &P, int C0, int R0) {
+__device__ __forceinline__ TileIn tile_fetch(const Grid &g, const PT &P, const TileGeo &G) {
   const int64_t p = g.pitch;
   const int k = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int q = threadIdx.x % kWave, r = R0 - 2 + k;
-  const int ic = C0 + q - HXL;
+  const int q = threadIdx.x % kWave, r = G.r0 - 2 + k;
+  const int ic = G.c0 + q - G.hl;
   // a lane beyond a narrow grid's east side only has to stay in its row
   const int i = min(wrap(ic, g.nlon), g.nlon - 1);
   TileIn in{};
@@ -225,11 +233,49 @@ __device__ __forceinline__ void tape_upwind(double *const *dst, int64_t o, const
   for (int j = 0; j < 4; j++) dst[2 + j][o] = d.df[j];
 }
 
-// One tile of the forward tendencies and the unfiltered gz update: output
-// columns C0 .. C0+TX-1, rows R0 .. R0+TY-1, LDS scratch sh[S::SH_ALL].  The
-// tile's pole slots hold its pole sums (tile_poles) and io its loads
-// (tile_fetch) on entry.  With TAPE the tile also writes the star state's
-// intermediates of its output points to *tape.
+// A short zonal filter (half width H) of a value held one column a lane, taps
+// in ascending order as filter_point.
+template <int H> __device__ __forceinline__ double lane_taps(double x, RecPtr w) {
+  double t[2 * H + 1];
+  t[H] = x;
+#pragma unroll
+  for (int j = 1; j <= H; j++) {
+    t[H - j] = lane_west(t[H - j + 1]);
+    t[H + j] = lane_east(t[H + j - 1]);
+  }
+  double acc = 0.0;
+#pragma unroll
+  for (int j = 0; j < 2 * H + 1; j++) acc = acc + w[j] * t[j];
+  return acc;
+}
+constexpr int kLaneTaps = 9;   // widest filter the lanes take
+template <class WT> __device__ __forceinline__ double lane_filter(double x, int n, WT wgt) {
+  const RecPtr w = (RecPtr)wgt;
+  if (n == 5) return lane_taps<2>(x, w);
+  if (n == 3) return lane_taps<1>(x, w);
+  if (n == 7) return lane_taps<3>(x, w);
+  if (n == 9) return lane_taps<4>(x, w);
+  return x;
+}
+
+// What the rest of a stage reads and writes in a tile that does all of it.
+template <class FT, class CP, class WP> struct TileRest {
+  FT big, small;
+  CP u_old, v_old;
+  WP u, v, u_f, v_f, gz_f, gz;
+};
+
+// One tile of the forward tendencies and the unfiltered gz update of the
+// points G owns, LDS scratch sh[S::SH_ALL].  The tile's pole slots hold its
+// pole sums (tile_poles) and io its loads (tile_fetch) on entry.  With TAPE
+// the tile also writes the star state's intermediates of its output points to
+// *tape.  With FULL the tile, on rows of short filters (at most kLaneTaps)
+// away from the poles, does the rest of the stage as well: the filters of gz
+// by lane shifts, the gz_f of the row north through LDS, u and v and their
+// filters.  A lane's filtered u takes 1 + h + h' columns either side (h, h'
+// the half widths of the filters of gz and of u), 54 of 64 lanes at h = 2;
+// what that recomputes is less than the gz, du, dv and gz_f that three
+// kernels pass through memory.
 //
 // A wavefront owns one tile row in every phase and all its 64 lanes run every
 // formula, so the columns on either side come from wavefront shifts and only
@@ -237,11 +283,12 @@ __device__ __forceinline__ void tape_upwind(double *const *dst, int64_t o, const
 // leaves the tile form values that no output point reads.  Reading both kinds
 // of neighbour and the metric rows from LDS (90 reads a point) kept the LDS
 // pipe, which a CU's four SIMDs share, busy for half of the launch.
-template <class S, bool TAPE = false, class MT, class PT>
+struct NoRest {};
+template <class S, bool TAPE, bool FULL, class MT, class PT, class RT>
 __device__ __forceinline__ void tend_tile(const Grid &g, const MT &Mg, RecPtr mrows, double grav, double rgrav,
                                           double dt, int stokes, int pv_scheme, int order, double wgt, int coriolis,
-                                          const PT &P, int C0, int R0, double *sh, const TileIn &io,
-                                          const TapeOut *tape = nullptr) {
+                                          const PT &P, const TileGeo &G, double *sh, const TileIn &io,
+                                          const TapeOut *tape, const RT &rest) {
   double(*sm)[LX] = (double(*)[LX])sh;
   double(*svf)[LX] = (double(*)[LX])(sh + S::LR * LX);
   double *shc = sh + 2 * S::LR * LX;
@@ -258,10 +305,10 @@ __device__ __forceinline__ void tend_tile(const Grid &g, const MT &Mg, RecPtr mr
   const int nlat = g.nlat, nhalf = g.nhalf;
   const int k = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // tile row of this wavefront
   const int q = threadIdx.x % kWave;                                   // tile column of this lane
-  const int r = R0 - 2 + k;                                            // global row
-  const int ic = C0 + q - HXL;                                         // output column
+  const int r = G.r0 - 2 + k;                                          // global row
+  const int ic = G.c0 + q - G.hl;                                      // output column
   const int kn = min(k + 1, S::LR - 1), ks = max(k - 1, 0), kss = max(k - 2, 0);
-  const bool out_pt = k >= 2 && k < S::TY + 2 && q >= HXL && q < HXL + TX && ic < g.nlon && r < nlat;
+  const bool out_pt = k >= 2 && r < G.r1 && q >= G.hl && q < G.hl + G.nc;
   const bool u_row = r >= 1 && r <= nlat - 2, v_row = r >= 0 && r < nhalf;
   const int64_t o = r * p + ic;
   const MeshRow M(mrows, nlat, r);
@@ -324,7 +371,8 @@ __device__ __forceinline__ void tend_tile(const Grid &g, const MT &Mg, RecPtr mr
   // D: tangential winds and pv on the edges (U rows 2 .. TY+2, V rows 1 ..
   // TY+1); phase E's gz_old is on its way meanwhile
   double gz_old = 0.0;
-  if (out_pt) gz_old = row_ld(P.gz_old + r * p, ic);
+  const int il = min(wrap(ic, g.nlon), g.nlon - 1);
+  if (FULL ? k >= 2 && r <= G.r1 : out_pt) gz_old = row_ld(P.gz_old + r * p, FULL ? il : ic);
   const double mfy_s = smfy[ks][q], mfx_n = smfx[kn][q];
   double pl = 0.0, pt = 0.0;
   if (k >= 1 && k < S::TY + 3) {
@@ -367,7 +415,14 @@ __device__ __forceinline__ void tend_tile(const Grid &g, const MT &Mg, RecPtr mr
   __syncthreads();
 
   // E: du, dv (forward pass) and gz_new = gz_old + dt dgz on the output rows
-  if (k < 2 || k >= S::TY + 2) return;
+  // (FULL: gz also on the row north of them)
+  if (!FULL && (k < 2 || k >= S::TY + 2)) return;
+  double u_old = 0.0, v_old = 0.0;
+  if constexpr (FULL)
+    if (k >= 2 && r < G.r1) {
+      u_old = row_ld(rest.u_old + r * p, il);
+      v_old = row_ld(rest.v_old + r * p, il);
+    }
   const double pt_s = spt[ks][q], pt_se = lane_east(pt_s), pt_e = lane_east(pt);
   const double pl_n = spl[kn][q], pl_nw = lane_west(pl_n), pl_w = lane_west(pl);
   const double mfy_e = lane_east(mfy), mfy_se = lane_east(mfy_s), mfx_w = lane_west(mfx), mfx_nw = lane_west(mfx_n);
@@ -381,15 +436,51 @@ __device__ __forceinline__ void tend_tile(const Grid &g, const MT &Mg, RecPtr mr
   const double dku = M.div(ke_e - ke_0, GMC_DE_LON, r);
   const double dkv = M.div(ke_n - ke_0, GMC_DE_LAT, r);
   double dgz = -(dmfdlon_of(mfx, mfx_w, M, r) + dmfdlat_of(mfy, mfy_s, M, r)) * grav;
-  if (!u_row) {   // the pole rows: gz from the pole sums
+  if (!FULL && !u_row) {   // the pole rows: gz from the pole sums
     const double dmfdlon = 0.0, dmfdlat = r == 0 ? pole[2] : pole[3];
     dgz = -(dmfdlon + dmfdlat) * grav;
   }
-  if (out_pt) {
-    if (u_row) row_st(P.du + r * p, ic, qhv - dku);
-    if (v_row) row_st(P.dv + r * p, ic, -qhu - dkv);
-    row_st(P.gz_new + r * p, ic, gz_old + dt * dgz);
+  const double gz_new = gz_old + dt * dgz;
+  if constexpr (!FULL) {
+    if (out_pt) {
+      if (u_row) row_st(P.du + r * p, ic, qhv - dku);
+      if (v_row) row_st(P.dv + r * p, ic, -qhu - dkv);
+      row_st(P.gz_new + r * p, ic, gz_new);
+    }
+  } else {
+    // F: the filters of gz; the row's gz_f to the row south of it, over pv
+    double gz_f = 0.0;
+    if (k >= 2 && r <= G.r1) {
+      const auto nb = *((const __attribute__((address_space(4))) int32_t *)rest.big.ngrid_lon + r);
+      gz_f = lane_filter(gz_new, nb, rest.big.wgt_lon + (int64_t)r * rest.big.max_taps);
+      spv[k][q] = gz_f;
+    }
+    __syncthreads();
+    if (k < 2 || r >= G.r1) return;
+    const auto ns = *((const __attribute__((address_space(4))) int32_t *)rest.small.ngrid_lon + r);
+    const auto nu = *((const __attribute__((address_space(4))) int32_t *)rest.big.ngrid_lon + r);
+    const auto nv = *((const __attribute__((address_space(4))) int32_t *)rest.big.ngrid_lat + r);
+    const double gz_s = lane_filter(gz_new, ns, rest.small.wgt_lon + (int64_t)r * rest.small.max_taps);
+    // G: u, v and their filters
+    const double u = u_old + dt * ((qhv - dku) - pgf_lon_of(lane_east(gz_f), gz_f, M, r));
+    const double v = v_old + dt * ((-qhu - dkv) - pgf_lat_of(spv[kn][q], gz_f, M, r));
+    const double u_f = lane_filter(u, nu, rest.big.wgt_lon + (int64_t)r * rest.big.max_taps);
+    const double v_f = lane_filter(v, nv, rest.big.wgt_lat + (int64_t)r * rest.big.max_taps);
+    if (out_pt) {
+      row_st(rest.gz_f + r * p, ic, gz_f);
+      row_st(rest.gz + r * p, ic, gz_s);
+      row_st(rest.u + r * p, ic, u);
+      row_st(rest.v + r * p, ic, v);
+      row_st(rest.u_f + r * p, ic, u_f);
+      row_st(rest.v_f + r * p, ic, v_f);
+    }
   }
+}
+
+// tile (tx, ty) of a cover of the grid by 60 x TY tiles
+template <class S> __device__ __forceinline__ TileGeo tile_geo(const Grid &g, int tx, int ty) {
+  const int c0 = tx * TX, r0 = ty * S::TY;
+  return TileGeo{c0, min(TX, g.nlon - c0), HXL, r0, min(r0 + S::TY, g.nlat)};
 }
 
 // Forward tendencies and the unfiltered gz update on a 60 x TY_MAIN tile.
@@ -411,12 +502,11 @@ __global__ void __launch_bounds__(kTendThreads, 8) k_tend(Grid g, Mesh Mg, const
   const int nx = (g.nlon + TX - 1) / TX, ny = (g.nlat + S::TY - 1) / S::TY, T = nx * ny;
   const int b = blockIdx.x, x = b % NXCD;
   const int t = x == NXCD - 1 ? T - 1 - b / NXCD : xcd_item(b, T);
-  const int C0 = (t % nx) * TX, R0 = (t / nx) * S::TY;
-
-  const TileIn io = tile_fetch<S>(g, P, C0, R0);
-  tile_poles<S>(g, Mg, grav, rgrav, P, R0, sh);
-  tend_tile<S, TAPE>(g, Mg, (RecPtr)mrows, grav, rgrav, dt, stokes, pv_scheme, order, wgt, coriolis, P, C0, R0, sh, io,
-                     &tape);
+  const TileGeo G = tile_geo<S>(g, t % nx, t / nx);
+  const TileIn io = tile_fetch<S>(g, P, G);
+  tile_poles<S>(g, Mg, grav, rgrav, P, G.r0, sh);
+  tend_tile<S, TAPE, false>(g, Mg, (RecPtr)mrows, grav, rgrav, dt, stokes, pv_scheme, order, wgt, coriolis, P, G, sh,
+                            io, &tape, NoRest{});
 }
 
 // ---------------------------------------------------------------------------
@@ -437,16 +527,16 @@ __device__ __forceinline__ int wrap2(int c, int n) { return c < 0 ? c + n : (c >
 // row window are staged in LDS: xs = [weights big | weights small | window].
 template <class FT, class CP, class WP>
 __device__ __forceinline__ void gzf_item(const Grid &g, const FT &big, const FT &small, const Item &it, CP gz_new,
-                                         WP gz_f, WP gz, double *xs) {
+                                         WP gz_f, WP gz, double *xs, int tid) {
   const int r = it.row;
   const int64_t o = r * g.pitch;
   const int nb = it.n, ns = it.n2;
   const int hb = nb > 1 ? (nb - 1) / 2 : 0, hs = ns > 1 ? (ns - 1) / 2 : 0, hw = hb > hs ? hb : hs;
   double *wb = xs, *ws = xs + big.max_taps, *x0 = xs + big.max_taps + small.max_taps;
   const int len = it.c1 - it.c0 + 2 * hw;
-  for (int k = threadIdx.x; k < nb; k += NF) wb[k] = big.wgt_lon[(int64_t)r * big.max_taps + k];
-  for (int k = threadIdx.x; k < ns; k += NF) ws[k] = small.wgt_lon[(int64_t)r * small.max_taps + k];
-  for (int t = threadIdx.x; t < len; t += 4 * NF) {
+  for (int k = tid; k < nb; k += NF) wb[k] = big.wgt_lon[(int64_t)r * big.max_taps + k];
+  for (int k = tid; k < ns; k += NF) ws[k] = small.wgt_lon[(int64_t)r * small.max_taps + k];
+  for (int t = tid; t < len; t += 4 * NF) {
     double v[4];
 #pragma unroll
     for (int u = 0; u < 4; u++)
@@ -456,7 +546,7 @@ __device__ __forceinline__ void gzf_item(const Grid &g, const FT &big, const FT 
       if (t + u * NF < len) x0[t + u * NF] = v[u];
   }
   __syncthreads();
-  for (int c = it.c0 + threadIdx.x; c < it.c1; c += NF) {
+  for (int c = it.c0 + tid; c < it.c1; c += NF) {
     const double *x = x0 + (c - it.c0);      // x[hw] is column c
     gz_f[o + c] = nb > 1 ? filter_point(wb, nb, x + hw - hb) : x[hw];
     gz[o + c] = ns > 1 ? filter_point(ws, ns, x + hw - hs) : x[hw];
@@ -466,7 +556,7 @@ __device__ __forceinline__ void gzf_item(const Grid &g, const FT &big, const FT 
 __global__ void __launch_bounds__(NF) k_gzf(Grid g, FilterDev big, FilterDev small, const Item *__restrict__ items,
                                             const double *__restrict__ gz_new, double *gz_f, double *gz) {
   extern __shared__ double xs[];
-  gzf_item(g, big, small, items[xcd_item(blockIdx.x, gridDim.x)], gz_new, gz_f, gz, xs);
+  gzf_item(g, big, small, items[xcd_item(blockIdx.x, gridDim.x)], gz_new, gz_f, gz, xs, threadIdx.x);
 }
 
 struct UVPtrs {
@@ -479,23 +569,22 @@ struct UVPtrs {
 // window of the updated row].
 template <class MT, class FT, class PT>
 __device__ __forceinline__ void uvf_item(const Grid &g, const MT &M, double dt, const FT &big,
-                                         const Item &it, const PT &P, double *xs) {
+                                         const Item &it, const PT &P, double *xs, int tid) {
   const int r = it.row;
   const int64_t p = g.pitch, o = r * p;
   const int nl = g.nlon;
   double *w = xs, *x0 = xs + big.max_taps;
-  if (it.kind == 1 && (r == 0 || r == g.nlat - 1)) {   // pole U rows: not updated, copied to u_f
-    for (int c = it.c0 + threadIdx.x; c < it.c1; c += NF) P.u_f[o + c] = P.u[o + c];
-    return;
-  }
-  const int n = it.n;
+  const bool pole_u = it.kind == 1 && (r == 0 || r == g.nlat - 1);   // not updated, copied to u_f
+  const int n = pole_u ? 0 : it.n;
   const int h = n > 1 ? (n - 1) / 2 : 0;
   const int len = it.c1 - it.c0 + 2 * h;
   const auto wg = (it.kind == 1 ? big.wgt_lon : big.wgt_lat) + (int64_t)r * big.max_taps;
-  for (int k = threadIdx.x; k < n; k += NF) w[k] = wg[k];
-  if (it.kind == 1) {
+  for (int k = tid; k < n; k += NF) w[k] = wg[k];
+  if (pole_u) {
+    for (int c = it.c0 + tid; c < it.c1; c += NF) P.u_f[o + c] = P.u[o + c];
+  } else if (it.kind == 1) {
     const double de = M(GMC_DE_LON, r), rde = 1.0 / de;
-    for (int t = threadIdx.x; t < len; t += 4 * NF) {
+    for (int t = tid; t < len; t += 4 * NF) {
       double uo[4], du[4], ge[4], gw[4];
 #pragma unroll
       for (int u = 0; u < 4; u++)
@@ -514,7 +603,7 @@ __device__ __forceinline__ void uvf_item(const Grid &g, const MT &M, double dt, 
     const int pole = r == 0 ? 1 : (r == g.nhalf - 1 ? -1 : 0);   // neighbour row of the smoothing
     const double de0 = M(GMC_DE_LAT, r), de1 = pole ? M(GMC_DE_LAT, r + pole) : 1.0;
     const double rde0 = 1.0 / de0, rde1 = 1.0 / de1;
-    for (int t = threadIdx.x; t < len; t += 2 * NF) {
+    for (int t = tid; t < len; t += 2 * NF) {
       double a[2][8];
 #pragma unroll
       for (int u = 0; u < 2; u++)
@@ -536,9 +625,10 @@ __device__ __forceinline__ void uvf_item(const Grid &g, const MT &M, double dt, 
     }
   }
   __syncthreads();
+  if (pole_u) return;
   const auto out = it.kind == 1 ? P.u : P.v;
   const auto out_f = it.kind == 1 ? P.u_f : P.v_f;
-  for (int c = it.c0 + threadIdx.x; c < it.c1; c += NF) {
+  for (int c = it.c0 + tid; c < it.c1; c += NF) {
     const double *x = x0 + (c - it.c0);
     out[o + c] = x[h];
     out_f[o + c] = n > 1 ? filter_point(w, n, x) : x[h];
@@ -548,9 +638,603 @@ __device__ __forceinline__ void uvf_item(const Grid &g, const MT &M, double dt, 
 __global__ void __launch_bounds__(NF) k_uvf(Grid g, Mesh M, double dt, FilterDev big, const Item *__restrict__ items,
                                             UVPtrs P) {
   extern __shared__ double xs[];
-  uvf_item(g, M, dt, big, items[xcd_item(blockIdx.x, gridDim.x)], P, xs);
+  uvf_item(g, M, dt, big, items[xcd_item(blockIdx.x, gridDim.x)], P, xs, threadIdx.x);
 }
 
+
+// ---------------------------------------------------------------------------
+// A whole stage of a band of rows in one workgroup, for rows whose filters
+// are too wide for a tile's lanes, on grids whose latitude circles fit a band
+// into LDS.
+//
+// The workgroup owns up to TY v rows over whole circles, so every stencil and
+// filter of the stage stays inside it: it forms the tendencies of its rows and
+// of the rows around them, filters gz on its rows and the next one north,
+// updates u and v and filters them, with a barrier where the three kernels
+// have a launch.  The expressions and their order are theirs, so both forms
+// give the same bits.
+//
+// Band b: v rows r0 .. r0+nv-1, the cell and U rows of the same numbers, and
+// in the last band the pole row north of them.  Local row k is global row
+// r0 - 2 + k.  The two v rows next to a pole share a band (the smoothing of
+// the pole row reads both).
+constexpr int NB_T = 1024;              // threads of a band's workgroup
+constexpr int NB_W = NB_T / kWave;
+constexpr int kBandTY = 2;              // v rows of a band
+constexpr int kBandRows = kBandTY + 5;  // local rows: two south, three north of the v rows
+constexpr int kBandLoads = 4;           // (row, 64-column) tasks per wavefront: loads of the local rows,
+constexpr int kBandOut = 2;             // and its output rows
+struct Band {
+  int r0, nv;
+  int part, parts;   // of several workgroups that form the same band, the columns part / parts
+};
+// LDS rows of nlon doubles: m, u_f, v_f; mfx and mfy (local rows 1 .. TY+2),
+// pv (0 .. TY+3), ke (2 .. TY+2)
+constexpr int kBandLdsRows = 3 * kBandRows + 2 * (kBandTY + 2) + (kBandTY + 4) + (kBandTY + 1);
+
+// The (row, segment) tasks of a wavefront, every nw-th from its own: a scalar
+// division per task would cost as much as the task's loads.
+struct Tasks {
+  int row, seg, segs, drow, dseg;
+  __device__ __forceinline__ Tasks(int w, int segs_, int nw) : segs(segs_) {
+    row = w / segs;
+    seg = w - row * segs;
+    drow = nw / segs;
+    dseg = nw - drow * segs;
+  }
+  __device__ __forceinline__ void next() {
+    row += drow;
+    seg += dseg;
+    if (seg >= segs) {
+      seg -= segs;
+      row++;
+    }
+  }
+};
+
+// Two neighbouring outputs of a zonal filter of n taps (filter_point's sums):
+// x points at the even column's window.  Each tap needs one more value of the
+// window, read in 16-byte pairs: half of filter_point's LDS reads per output,
+// which bound a wide filter's workgroup.
+__device__ __forceinline__ void filter_pair(const double *w, int n, const double *x, double &o0, double &o1) {
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  double a0 = 0.0, a1 = 0.0, cur;
+  int k = 0;
+  if ((__builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)x) & 8) == 0) {   // x[0] on a pair's boundary
+    const d2 p = *(const d2 *)x;
+    a0 = a0 + w[0] * p.x;
+    a1 = a1 + w[0] * p.y;
+    cur = p.y;
+    k = 1;
+  } else {
+    cur = x[0];
+  }
+  for (; k + 8 <= n; k += 8) {
+    d2 p[4];
+    double wk[8];
+#pragma unroll
+    for (int u = 0; u < 4; u++) p[u] = *(const d2 *)(x + k + 1 + 2 * u);
+#pragma unroll
+    for (int u = 0; u < 8; u++) wk[u] = w[k + u];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      a0 = a0 + wk[2 * u] * cur;
+      a1 = a1 + wk[2 * u] * p[u].x;
+      a0 = a0 + wk[2 * u + 1] * p[u].x;
+      a1 = a1 + wk[2 * u + 1] * p[u].y;
+      cur = p[u].y;
+    }
+  }
+  for (; k < n; k++) {
+    const double nx = x[k + 1];
+    a0 = a0 + w[k] * cur;
+    a1 = a1 + w[k] * nx;
+    cur = nx;
+  }
+  o0 = a0;
+  o1 = a1;
+}
+
+struct BandOut {
+  double *gz_f, *gz;
+};
+
+template <bool TAPE>
+__device__ __forceinline__ void band_stage(const Grid &g, RecPtr mrows, double grav, double rgrav, double dt,
+                                           int stokes, int pv_scheme, int order, double wgt, int coriolis,
+                                           const FilterDev &big, const FilterDev &small, const Band bd,
+                                           const StagePtrs &P, const UVPtrs &U, const BandOut &G, const TapeOut &tape,
+                                           double *xs) {
+  const int n = g.nlon, nlat = g.nlat, nhalf = g.nhalf, segs = (n + kWave - 1) / kWave;
+  const int64_t p = g.pitch;
+  constexpr int TY = kBandTY, LR = kBandRows;
+  double *sm = xs, *suf = sm + LR * n, *svf = suf + LR * n;
+  double *smfx = svf + LR * n - n, *smfy = smfx + (TY + 2) * n;   // row k at + k n, from k = 1
+  double *spv = smfy + (TY + 2) * n + n;
+  double *ske = spv + (TY + 4) * n - 2 * n;                       // from k = 2
+  double *pole = spv + (TY + 4) * n + (TY + 1) * n, *wt = pole + 8;
+  double *spl = suf, *spt = svf;   // pv on the edges replaces u_f and v_f element by element
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid / kWave), q = tid % kWave;
+  const int r0 = bd.r0, nv = bd.nv;
+  const bool south = r0 == 0, north = r0 + nv == nhalf;
+  const int nu = nv + (north ? 1 : 0);         // cell rows the band writes
+  const int rows = nv + 5;                     // local rows in use
+
+  // ---- the band's loads, all on their way before the first use -----------
+  double a_gz[kBandLoads], a_gzs[kBandLoads], a_uf[kBandLoads], a_vf[kBandLoads];
+  Tasks T(w, segs, NB_W);
+#pragma unroll
+  for (int j = 0; j < kBandLoads; j++, T.next()) {
+    const int k = T.row, r = r0 - 2 + k, i = T.seg * kWave + q;
+    a_gz[j] = a_gzs[j] = a_uf[j] = a_vf[j] = 0.0;
+    if (k < rows && r >= 0 && r < nlat && i < n) {
+      a_gz[j] = row_ld(P.gz_star + r * p, i);
+      a_gzs[j] = row_ld(P.gzs + r * p, i);
+      a_uf[j] = row_ld(P.u_f + r * p, i);
+      if (r < nhalf) a_vf[j] = row_ld(P.v_f + r * p, i);
+    }
+  }
+  double gz_old[kBandOut], u_old[kBandOut], v_old[kBandOut];
+  T = Tasks(w, segs, NB_W);
+#pragma unroll
+  for (int j = 0; j < kBandOut; j++, T.next()) {
+    const int k = 2 + T.row, r = r0 - 2 + k, i = T.seg * kWave + q;
+    gz_old[j] = u_old[j] = v_old[j] = 0.0;
+    if (k <= nv + 2 && r < nlat && i < n) {
+      gz_old[j] = row_ld(P.gz_old + r * p, i);
+      if (k < nv + 2) {
+        u_old[j] = row_ld(U.u_old + r * p, i);
+        v_old[j] = row_ld(U.v_old + r * p, i);
+      }
+    }
+  }
+  double u_pole = 0.0;   // n <= NB_T
+  if ((south || north) && tid < n) u_pole = row_ld(U.u + (south ? 0 : nlat - 1) * p, tid);
+  // filter weights: table rows (zero beyond a row's taps, at most nlon <= NB_T
+  // of them) loaded whole, so that no load waits for the tap counts
+  double wr[3 * TY + 2];
+#pragma unroll
+  for (int j = 0; j <= TY; j++) {
+    const int r = min(r0 + j, nlat - 1), rv = min(r0 + j, nhalf - 1);
+    if (tid < big.max_taps) {
+      wr[j] = row_ld(big.wgt_lon + (int64_t)r * big.max_taps, tid);
+      if (j < TY) wr[2 * TY + 2 + j] = row_ld(big.wgt_lat + (int64_t)rv * big.max_taps, tid);
+    }
+    if (tid < small.max_taps) wr[TY + 1 + j] = row_ld(small.wgt_lon + (int64_t)r * small.max_taps, tid);
+  }
+  // taps of row r0 + j and where its weights sit: big and small filter of the
+  // cell (and U) rows, big filter of the v rows
+  typedef const __attribute__((address_space(4))) int32_t *TapPtr;
+  int nb[TY + 1], ns[TY + 1], nt[TY], ob[TY + 1], os[TY + 1], ot[TY], o = 0;
+#pragma unroll
+  for (int j = 0; j <= TY; j++) {
+    const int r = min(r0 + j, nlat - 1), rv = min(r0 + j, nhalf - 1);
+    nb[j] = ((TapPtr)big.ngrid_lon)[r];
+    ns[j] = ((TapPtr)small.ngrid_lon)[r];
+    ob[j] = o;
+    os[j] = ob[j] + max(nb[j], 0);
+    o = os[j] + max(ns[j], 0);
+    if (j < TY) {
+      nt[j] = ((TapPtr)big.ngrid_lat)[rv];
+      ot[j] = o;
+      o += max(nt[j], 0);
+    }
+  }
+  T = Tasks(w, segs, NB_W);
+#pragma unroll
+  for (int j = 0; j < kBandLoads; j++, T.next()) {
+    const int k = T.row, r = r0 - 2 + k, i = T.seg * kWave + q;
+    if (k < rows && i < n) {
+      const int e = k * n + i;
+      sm[e] = div_rn(a_gz[j] - a_gzs[j], grav, rgrav);   // m_of
+      suf[e] = a_uf[j];
+      svf[e] = a_vf[j];
+      if (TAPE && tape.u_f && k >= 2 && k < 2 + nu) {
+        row_st(tape.u_f + r * p, i, a_uf[j]);
+        if (r < nhalf) row_st(tape.v_f + r * p, i, a_vf[j]);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j <= TY; j++) {
+    if (tid < nb[j]) wt[ob[j] + tid] = wr[j];
+    if (tid < ns[j]) wt[os[j] + tid] = wr[TY + 1 + j];
+    if (j < TY && tid < nt[j]) wt[ot[j] + tid] = wr[2 * TY + 2 + j];
+  }
+  // the entry of a per-row array for a row index known at run time
+  auto pick = [](const int *v, int n_, int j) {
+    int x = v[0];
+    for (int e = 1; e < n_; e++) x = j == e ? v[e] : x;
+    return x;
+  };
+  __syncthreads();
+
+  // ---- pole sums (pole_sums' terms from LDS), one each for the last three
+  // wavefronts while the others form B; the rows that read them follow
+  // (the bands that read the vertex row next to a pole: its own, and with two
+  // rows a band the one beside it)
+  const bool sum_s = r0 <= 2, sum_n = r0 + nv >= nhalf - 2;
+  if (sum_s || sum_n) {
+    if (const int ws = w - (NB_W - 3); ws >= 0) {
+      const int vr = sum_s ? 0 : nhalf - 1, cr = sum_s ? 0 : nlat - 1;
+      const int kv = vr - r0 + 2, ku = sum_s ? kv + 1 : kv;
+      const MeshRow V(mrows, nlat, vr), Cc(mrows, nlat, cr);
+      const double le = V(GMC_LE_LAT, vr), ac = Cc(GMC_AREA_CELL, cr);
+      const double w1 = V(GMC_HALF_TANGENT_WGT1, vr), w2 = V(GMC_HALF_TANGENT_WGT2, vr);
+      auto term = [&](int i) {
+        const double v = svf[kv * n + i];
+        if (ws == 0) return v * v;
+        const double m_lat = (sm[kv * n + i] + sm[(kv + 1) * n + i]) * 0.5;
+        if (ws == 1) {
+          const double mfy = m_lat * v;
+          return sum_n ? -mfy : mfy;
+        }
+        const int im = wrap(i - 1, n), ip = wrap(i + 1, n);
+        const double *mu = sm + ku * n, *uu = suf + ku * n;
+        const double mfx_w = (mu[im] + mu[i]) * 0.5 * uu[im], mfx_e = (mu[i] + mu[ip]) * 0.5 * uu[i];
+        const double t = sum_n ? tangent_sum(w1, w2, mfx_w, mfx_e, 0.0, 0.0) : tangent_sum(w1, w2, 0.0, 0.0, mfx_w, mfx_e);
+        const double ul = t / m_lat;
+        return sum_n ? ul * le : -ul * le;
+      };
+      // wave_zonal_sum's order, three terms of a lane formed at a time
+      double sum = 0.0;
+      for (int i = q; i < n; i += 3 * kWave) {
+        double t[3];
+#pragma unroll
+        for (int u = 0; u < 3; u++) t[u] = i + u * kWave < n ? term(i + u * kWave) : 0.0;
+#pragma unroll
+        for (int u = 0; u < 3; u++)
+          if (i + u * kWave < n) sum = sum + t[u];
+      }
+      for (int x = 1; x < kWave; x <<= 1) sum = sum + __shfl_xor(sum, x, kWave);
+      const double nl = (double)n;
+      if (q == 0) pole[ws] = ws == 0 ? sum / nl : (ws == 1 ? sum * le / nl / ac : sum / nl / ac);
+    }
+  }
+
+  // ---- B: mass fluxes, pv, ke (as tend_tile) -----------------------------
+  const bool sums = sum_s || sum_n;
+  const int r_sum = sum_s ? 0 : nhalf - 1, c_sum = sum_s ? 0 : nlat - 1;   // vertex and cell row of the sums
+  const int nw_b = sums ? NB_W - 3 : NB_W;
+  for (T = Tasks(w < nw_b ? w : kBandRows * segs, segs, nw_b); T.row < nv + 4; T.next()) {
+    const int k = T.row, r = r0 - 2 + k, i = T.seg * kWave + q;
+    if (r < 0 || r >= nlat || i >= n) continue;
+    const MeshRow M(mrows, nlat, r);
+    const int ie = wrap(i + 1, n), iw = wrap(i - 1, n), ks = max(k - 1, 0);
+    const double *m_ = sm + k * n, *u_ = suf + k * n, *v_ = svf + k * n;
+    const double m0 = m_[i], m1 = m_[ie], m2 = m_[n + i], m3 = m_[n + ie];
+    const double uf = u_[i], u1 = u_[n + i], uw = u_[iw], vf = v_[i], v1 = v_[ie], vs = svf[ks * n + i];
+    const bool u_row = r >= 1 && r <= nlat - 2, v_row = r < nhalf;
+    const double mv = m_vtx_of(m0, m1, m2, m3, M, r);
+    // the vertex row of a pole sum keeps m_vtx until the sum is there
+    const double pv = stokes && sums && r == r_sum ? mv : pv_of(vor_of(uf, u1, v1, vf, M, r), M, r, mv);
+    const double mfx = (m0 + m1) * 0.5 * uf, mfy = (m0 + m2) * 0.5 * vf;
+    if (v_row) spv[k * n + i] = pv;
+    if (k >= 1 && k <= nv + 2) {
+      smfx[k * n + i] = u_row ? mfx : 0.0;
+      smfy[k * n + i] = v_row ? mfy : 0.0;
+      if (k >= 2 && u_row) ske[k * n + i] = ke_of(uw, uf, vs, vf, M, r);
+    }
+    if (TAPE && v_row && k >= 2 && k < 2 + nv) {
+      row_st(tape.m_vtx + r * p, i, mv);
+      if (!(stokes && r == r_sum)) row_st(tape.pv + r * p, i, pv);
+      row_st(tape.mfy + r * p, i, mfy);
+      row_st(tape.m_lat + r * p, i, (m0 + m2) * 0.5);
+    }
+  }
+  __syncthreads();
+
+  if (sums) {
+    const int kv = r_sum - r0 + 2, kc = c_sum - r0 + 2;
+    const MeshRow V(mrows, nlat, r_sum);
+    for (int i = tid; i < n; i += NB_T) {
+      if (stokes) {
+        const double pv = pv_of(pole[2], V, r_sum, spv[kv * n + i]);
+        spv[kv * n + i] = pv;
+        if (TAPE && kv >= 2 && kv < 2 + nv) row_st(tape.pv + r_sum * p, i, pv);
+      }
+      if (kc >= 2 && kc <= nv + 2) ske[kc * n + i] = pole[0];
+    }
+    __syncthreads();
+  }
+
+  // ---- D: tangential winds and pv on the edges ---------------------------
+  // (U rows 2 .. nv+2 and V rows 1 .. nv+1, a task each)
+  for (T = Tasks(w, segs, NB_W); T.row < 2 * (nv + 1); T.next()) {
+    const bool lon = T.row <= nv;
+    const int k = lon ? 2 + T.row : T.row - nv, r = r0 - 2 + k, i = T.seg * kWave + q;
+    if (r < 0 || r >= nlat || i >= n) continue;
+    const MeshRow M(mrows, nlat, r);
+    const int ie = wrap(i + 1, n), iw = wrap(i - 1, n), iww = wrap(i - 2, n), ih = wrap(i + g.half, n);
+    const bool u_row = r >= 1 && r <= nlat - 2, v_row = r < nhalf;
+    const double *m_ = sm + k * n;
+    const double m0 = m_[i];
+    const double *fx = smfx + k * n, *fy = smfy + k * n;
+    if (lon) {
+      if (!u_row) {
+        spl[k * n + i] = 0.0;
+        continue;
+      }
+      const double uf = suf[k * n + i];
+      double pl;
+      const double tl = tangent_sum(M(GMC_FULL_TANGENT_WGT1, r), M(GMC_FULL_TANGENT_WGT2, r), fy[i - n], fy[ie - n], fy[i], fy[ie]);
+      const double ml = (m0 + m_[ie]) * 0.5, vl = div_mid(tl, ml);
+      // rows beyond a pole are rows on its other side, half a circle away
+      const double *v0 = spv + k * n;
+      const double a1 = r == 1 ? v0[ih - n] : v0[i - 2 * n], a2 = v0[i - n], a3 = v0[i];
+      const double a4 = r == nhalf - 1 ? v0[ih] : v0[i + n];
+      if (pv_scheme == GMC_PV_UPWIND && order == 3) pl = pv_upwind_edge(3, wgt, vl, uf, 0, a1, a2, a3, a4);
+      else pl = pv_edge(pv_scheme, order, wgt, vl, uf, 0, dt, M(GMC_LE_LON, r), a1, a2, a3, a4);
+      if (TAPE && k < 2 + nu) {
+        row_st(tape.m_lon + r * p, i, ml);
+        row_st(tape.mfx + r * p, i, fx[i]);
+        if (tape.mfy_lon) row_st(tape.mfy_lon + r * p, i, tl);
+        row_st(tape.v_lon + r * p, i, vl);
+        row_st(tape.pv_lon + r * p, i, pl);
+        if (tape.dlon[0]) tape_upwind(tape.dlon, r * p + i, upwind_deriv(pv_scheme, order, wgt, vl, uf, 0, a1, a2, a3, a4));
+      }
+      spl[k * n + i] = pl;
+    }
+    if (!lon) {
+      if (!v_row) continue;
+      const double vf = svf[k * n + i];
+      double pt;
+      const double tu = tangent_sum(M(GMC_HALF_TANGENT_WGT1, r), M(GMC_HALF_TANGENT_WGT2, r), fx[iw], fx[i], fx[n + iw], fx[n + i]);
+      const double ul = div_mid(tu, (m0 + m_[n + i]) * 0.5);
+      const double *v0 = spv + k * n;
+      const double a1 = v0[iww], a2 = v0[iw], a3 = v0[i], a4 = v0[ie];
+      if (pv_scheme == GMC_PV_UPWIND && order == 3) pt = pv_upwind_edge(3, wgt, ul, vf, 1, a1, a2, a3, a4);
+      else pt = pv_edge(pv_scheme, order, wgt, ul, vf, 1, dt, M(GMC_LE_LAT, r), a1, a2, a3, a4);
+      if (TAPE && k >= 2) {
+        if (tape.mfx_lat) row_st(tape.mfx_lat + r * p, i, tu);
+        row_st(tape.u_lat + r * p, i, ul);
+        row_st(tape.pv_lat + r * p, i, pt);
+        if (tape.dlat[0]) tape_upwind(tape.dlat, r * p + i, upwind_deriv(pv_scheme, order, wgt, ul, vf, 1, a1, a2, a3, a4));
+      }
+      spt[k * n + i] = pt;
+    }
+  }
+  __syncthreads();
+
+  // ---- E: tendencies, the unfiltered gz into rows wrapped around the circle
+  // (column c of row j at x[j][c + n / 2], c in [-n/2, n + n/2)) over m
+  const int hw = n / 2;
+  auto put = [&](double *row, int i, double v) {
+    row[i + hw] = v;
+    row[i + hw + (i < n - hw ? n : -n)] = v;
+  };
+  double du[kBandOut], dv[kBandOut];
+  T = Tasks(w, segs, NB_W);
+#pragma unroll
+  for (int j = 0; j < kBandOut; j++, T.next()) {
+    const int k = 2 + T.row, r = r0 - 2 + k, i = T.seg * kWave + q;
+    du[j] = dv[j] = 0.0;
+    if (k > nv + 2 || r >= nlat || i >= n) continue;
+    const MeshRow M(mrows, nlat, r);
+    const int ie = wrap(i + 1, n), iw = wrap(i - 1, n);
+    const double *fx = smfx + k * n, *fy = smfy + k * n, *pl = spl + k * n, *pt = spt + k * n, *ke = ske + k * n;
+    const bool u_row = r >= 1 && r <= nlat - 2;
+    double dgz;
+    if (u_row) {
+      dgz = -(dmfdlon_of(fx[i], fx[iw], M, r) + dmfdlat_of(fy[i], fy[i - n], M, r)) * grav;
+    } else {
+      const double dmfdlon = 0.0, dmfdlat = pole[1];
+      dgz = -(dmfdlon + dmfdlat) * grav;
+    }
+    const double gz_new = gz_old[j] + dt * dgz;
+    put(sm + (k - 2) * 2 * n, i, gz_new);
+    if (k < nv + 2) {
+      if (u_row) {
+        const double qhv = coriolis == 1
+            ? qhv_of(M, r, pl[i], fy[i - n], pt[i - n], fy[ie - n], pt[ie - n], fy[i], pt[i], fy[ie], pt[ie])
+            : tangent_sum(M(GMC_FULL_TANGENT_WGT1, r), M(GMC_FULL_TANGENT_WGT2, r), fy[i - n], fy[ie - n], fy[i], fy[ie]) * pl[i];
+        du[j] = qhv - M.div(ke[ie] - ke[i], GMC_DE_LON, r);
+      }
+      const double qhu = coriolis == 1
+          ? qhu_of(M, r, pt[i], fx[iw], pl[iw], fx[i], pl[i], fx[n + iw], pl[n + iw], fx[n + i], pl[n + i])
+          : tangent_sum(M(GMC_HALF_TANGENT_WGT1, r), M(GMC_HALF_TANGENT_WGT2, r), fx[iw], fx[i], fx[n + iw], fx[n + i]) * pt[i];
+      dv[j] = -qhu - M.div(ke[n + i] - ke[i], GMC_DE_LAT, r);
+    }
+  }
+  __syncthreads();
+
+  // ---- F: the filters of gz, two columns a lane; gz_f also into LDS over ke
+  // (a band in parts stores only its part's columns)
+  const int segs2 = (n + 2 * kWave - 1) / (2 * kWave);
+  const int p0 = n / 2 * bd.part / bd.parts * 2, p1 = n / 2 * (bd.part + 1) / bd.parts * 2;
+  for (T = Tasks(w, segs2, NB_W); T.row < 2 * (nv + 1); T.next()) {
+    const int j = T.row >> 1, r = r0 + j, i = 2 * (T.seg * kWave + q);
+    if (r >= nlat || i >= n) continue;
+    const double *x = sm + j * 2 * n + i + hw;
+    const bool sml = T.row & 1, mine = i >= p0 && i < p1;
+    if (sml && (T.seg * 2 * kWave >= p1 || (T.seg + 1) * 2 * kWave <= p0)) continue;
+    const int nf = sml ? pick(ns, TY + 1, j) : pick(nb, TY + 1, j), of = sml ? pick(os, TY + 1, j) : pick(ob, TY + 1, j);
+    double f0 = x[0], f1 = x[1];
+    if (nf > 1) filter_pair(wt + of, nf, x - (nf - 1) / 2, f0, f1);
+    if (!sml) {
+      ske[(j + 2) * n + i] = f0;
+      ske[(j + 2) * n + i + 1] = f1;
+    }
+    if (j < nu && mine) {
+      double *out = (sml ? G.gz : G.gz_f) + r * p;
+      row_st(out, i, f0);
+      row_st(out, i + 1, f1);
+    }
+  }
+  __syncthreads();
+
+  // ---- G: u and v of the band into wrapped rows over m and u_f (u rows,
+  // then v rows), then the smoothing of the v row next to a pole -----------
+  T = Tasks(w, segs, NB_W);
+#pragma unroll
+  for (int j = 0; j < kBandOut; j++, T.next()) {
+    const int jr = T.row, r = r0 + jr, i = T.seg * kWave + q;
+    if (jr >= nv || i >= n) continue;
+    const MeshRow M(mrows, nlat, r);
+    const double *f = ske + (jr + 2) * n;
+    if (r >= 1) put(sm + jr * 2 * n, i, u_old[j] + dt * (du[j] - pgf_lon_of(f[wrap(i + 1, n)], f[i], M, r)));
+    put(sm + (TY + jr) * 2 * n, i, v_old[j] + dt * (dv[j] - pgf_lat_of(f[n + i], f[i], M, r)));
+  }
+  __syncthreads();
+  if (south || north) {
+    double *v0 = sm + (TY + (south ? 0 : nv - 1)) * 2 * n, *v1 = v0 + (south ? 2 * n : -2 * n);
+    for (int i = tid; i < n; i += NB_T) put(v0, i, pole_smooth(v0[i + hw], v1[i + hw]));
+    __syncthreads();
+  }
+
+  // ---- H: the big filters of u and v, two columns a lane -----------------
+  const int segs_p = (p1 - p0 + 2 * kWave - 1) / (2 * kWave);
+  for (T = Tasks(w, segs_p, NB_W); T.row < 2 * nv; T.next()) {
+    const int j = T.row >> 1, r = r0 + j, i = p0 + 2 * (T.seg * kWave + q);
+    const bool lat = !(T.row & 1);
+    if (i >= p1 || (!lat && r == 0)) continue;
+    const double *x = sm + ((lat ? TY : 0) + j) * 2 * n + i + hw;
+    const int nf = lat ? pick(nt, TY, j) : pick(nb, TY + 1, j), of = lat ? pick(ot, TY, j) : pick(ob, TY + 1, j);
+    double f0 = x[0], f1 = x[1];
+    double *out = (lat ? U.v : U.u) + r * p, *out_f = (lat ? U.v_f : U.u_f) + r * p;
+    row_st(out, i, f0);
+    row_st(out, i + 1, f1);
+    if (nf > 1) filter_pair(wt + of, nf, x - (nf - 1) / 2, f0, f1);
+    row_st(out_f, i, f0);
+    row_st(out_f, i + 1, f1);
+  }
+  if ((south || north) && tid < n && bd.part == 0)   // pole U rows: not updated, copied to u_f
+    row_st(U.u_f + (south ? 0 : nlat - 1) * p, tid, u_pole);
+}
+
+// ---------------------------------------------------------------------------
+// The stage as gmc_step runs it.
+//
+// Away from the poles the zonal filters have 3 to 9 taps, and one tile takes a
+// point through the whole stage (tend_tile with FULL).  Only the polar rows,
+// about an eighth of them, need the tendencies, the gz filters and the u / v
+// part one after the other:
+//   one launch    (kStageOne) where their circles fit into LDS: bands of the
+//                 polar rows beside the tiles;
+//   three launches (kStageTend, kStageGz, kStageUv) elsewhere: tiles of the
+//                 polar tendencies, then four filter items a workgroup, with
+//                 the tiles of the other rows spread over the three so that
+//                 none of them leaves compute units idle.
+// A polar v row next to the tiles reads their gz_f row, so the tiles beside
+// the polar rows go into the first launch.
+//
+// Measured per step with three models in flight on three streams (and alone),
+// three kernels a stage against this: 180 x 91 wrfrk3 17.9 (50) -> 13.5 (39)
+// us, 360 x 181 24.1 (62) -> 19.4 (55), 502 x 253 with damping 35 (90) -> 31
+// (85), 1440 x 721 149 (164) -> 134 (163).  A full tile takes 5 us from its
+// start to its last store; the band at a pole, 17 us at 360 columns, bounds
+// the small grids, the vector instructions and the loads of the tiles (two
+// workgroups a compute unit, 45 % of the issue slots) the large ones.
+//
+// A workgroup finds its work from its number and the kernel arguments alone: a
+// table would put one more trip to memory (about 1 us) before its first load.
+enum { kStageTend = 0, kStageGz = 1, kStageUv = 2, kStageOne = 3 };
+constexpr int kMaxSegs = 8;
+// Bands of the short rows whose tiles have the same width: from band b0 and
+// tile t0 on, nx tiles of w columns a band, first output lane hl; div = 2^32 /
+// nx rounded up (t * div >> 32 is t / nx for the few thousand tiles there are).
+struct TileSeg {
+  int b0, t0, nx, w, hl;
+  uint32_t div;
+};
+// What the launches of a stage share about its rows: [ra, rb) the rows of
+// short filters; the polar tendencies' nx_p tiles a band, tiles_s of them
+// south and tiles_p in all; bands_s polar bands south and bands_p in all.
+struct StageMap {
+  int ra, rb, nseg, ntiles;
+  TileSeg seg[kMaxSegs];
+  int nx_p, tiles_s, tiles_p, bands_s, bands_p;
+  uint32_t div_p;
+};
+struct StageArgs {
+  Grid g;
+  Mesh M;
+  const double *mrows;
+  double grav, rgrav, dt, wgt;
+  int stokes, pv_scheme, order, coriolis;
+  StagePtrs P;
+  UVPtrs U;
+  BandOut G;
+  FilterDev big, small;
+  StageMap S;
+  int polar;               // workgroups of this launch with polar work
+  int tile0, tiles;        // its tiles of the short rows, from tile0 on (counted around)
+  const Item *items;       // filter items, kItemsPerWg a workgroup
+  int item_lds;            // doubles of LDS per item
+  TapeOut tape;
+};
+using StageTile = Tile<11>;
+constexpr int kItemsPerWg = StageTile::NT / NF;
+
+__device__ __forceinline__ TileGeo short_tile(const StageMap &S, int nlon, int t) {
+  TileSeg s = S.seg[0];
+#pragma unroll
+  for (int k = 1; k < kMaxSegs; k++)
+    if (k < S.nseg && t >= S.seg[k].t0) s = S.seg[k];
+  const int e = t - s.t0, b = (int)(((uint64_t)(uint32_t)e * s.div) >> 32), x = e - b * s.nx;
+  const int r0 = S.ra + (s.b0 + b) * StageTile::TY, c0 = x * s.w;
+  return TileGeo{c0, min(s.w, nlon - c0), s.hl, r0, min(r0 + StageTile::TY, S.rb)};
+}
+
+// Tile e of the polar tendencies: bands from the south pole to row ra, then
+// from row rb to the north pole.
+__device__ __forceinline__ TileGeo polar_tile(const StageMap &S, const Grid &g, int e) {
+  const bool north = e >= S.tiles_s;
+  if (north) e -= S.tiles_s;
+  const int b = (int)(((uint64_t)(uint32_t)e * S.div_p) >> 32), x = e - b * S.nx_p;
+  const int r0 = (north ? S.rb : 0) + b * StageTile::TY, c0 = x * TX;
+  return TileGeo{c0, min(TX, g.nlon - c0), HXL, r0, min(r0 + StageTile::TY, north ? g.nlat : S.ra)};
+}
+
+// The work of polar workgroup e: kPoleParts workgroups for the band at each
+// pole, whose filters are twice as wide as the next one's, each filtering and
+// storing its share of the columns; then the other bands, numbered from the
+// poles, south first: kBandTY v rows each, the last of a zone what is left.
+constexpr int kPoleParts = 4;
+__device__ __forceinline__ Band polar_band(const StageMap &S, int nhalf, int e) {
+  const bool pole = e < 2 * kPoleParts;
+  const bool north = pole ? e >= kPoleParts : e - 2 * kPoleParts >= S.bands_s - 1;
+  const int part = pole ? e % kPoleParts : 0, parts = pole ? kPoleParts : 1;
+  const int j = pole ? 0 : e - 2 * kPoleParts + 1 - (north ? S.bands_s - 1 : 0);   // from the zone's pole
+  if (!north) return Band{kBandTY * j, min(kBandTY, S.ra - kBandTY * j), part, parts};
+  const int r1 = nhalf - kBandTY * j, r0 = max(r1 - kBandTY, S.rb);
+  return Band{r0, r1 - r0, part, parts};
+}
+
+template <int PHASE, bool TAPE>
+__global__ void __launch_bounds__(StageTile::NT, PHASE == kStageOne ? 4 : 8) k_stage(StageArgs A) {
+  extern __shared__ __attribute__((aligned(16))) double xs[];
+  using S = StageTile;
+  const int b = blockIdx.x;
+  if (b >= A.polar) {
+    int t = A.tile0 + xcd_item(b - A.polar, A.tiles);
+    t = t >= A.S.ntiles ? t - A.S.ntiles : t;
+    const TileGeo geo = short_tile(A.S, A.g.nlon, t);
+    const TileRest<FilterDev, const double *, double *> rest{A.big,  A.small, A.U.u_old, A.U.v_old, A.U.u,
+                                                             A.U.v,  A.U.u_f, A.U.v_f,   A.G.gz_f,  A.G.gz};
+    const TileIn io = tile_fetch<S>(A.g, A.P, geo);
+    tend_tile<S, TAPE, true>(A.g, A.M, (RecPtr)A.mrows, A.grav, A.rgrav, A.dt, A.stokes, A.pv_scheme, A.order, A.wgt,
+                             A.coriolis, A.P, geo, xs, io, &A.tape, rest);
+  } else if constexpr (PHASE == kStageTend) {
+    const TileGeo geo = polar_tile(A.S, A.g, b);
+    const TileIn io = tile_fetch<S>(A.g, A.P, geo);
+    tile_poles<S>(A.g, A.M, A.grav, A.rgrav, A.P, geo.r0, xs);
+    tend_tile<S, TAPE, false>(A.g, A.M, (RecPtr)A.mrows, A.grav, A.rgrav, A.dt, A.stokes, A.pv_scheme, A.order, A.wgt,
+                              A.coriolis, A.P, geo, xs, io, &A.tape, NoRest{});
+  } else if constexpr (PHASE == kStageOne) {
+    band_stage<TAPE>(A.g, (RecPtr)A.mrows, A.grav, A.rgrav, A.dt, A.stokes, A.pv_scheme, A.order, A.wgt, A.coriolis,
+                     A.big, A.small, polar_band(A.S, A.g.nhalf, b), A.P, A.U, A.G, A.tape, xs);
+  } else {
+    // an item per group of NF threads (the list is padded with empty items)
+    const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x / NF), tid = threadIdx.x % NF;
+    const Item &it = A.items[b * kItemsPerWg + grp];
+    double *x = xs + grp * A.item_lds;
+    if constexpr (PHASE == kStageGz)
+      gzf_item(A.g, A.big, A.small, it, A.P.gz_new, A.G.gz_f, A.G.gz, x, tid);
+    else
+      uvf_item(A.g, A.M, A.dt, A.big, it, A.U, x, tid);
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Batched ensembles: the same stage kernels over many contexts in one launch.
@@ -629,12 +1313,12 @@ __global__ void __launch_bounds__(S::NT, 8) k_tend_ens(const EnsMember *__restri
     }
     const EnsMember d = mem[lo];   // a private copy: no aliasing with the stores of the tile
     const int lt = t - d.tile0;
-    const int C0 = (lt % d.nx) * TX, R0 = (lt / d.nx) * S::TY;
+    const TileGeo G = tile_geo<S>(d.g, lt % d.nx, lt / d.nx);
     const StagePtrsG sp = glb(d.sp);
-    const TileIn io = tile_fetch<S>(d.g, sp, C0, R0);
-    tile_poles<S>(d.g, glb(d.M), d.grav, d.rgrav, sp, R0, sh);
-    tend_tile<S>(d.g, glb(d.M), (RecPtr)d.mrows, d.grav, d.rgrav, d.dt, d.stokes, d.pv_scheme, d.order, d.wgt,
-                 d.coriolis, sp, C0, R0, sh, io);
+    const TileIn io = tile_fetch<S>(d.g, sp, G);
+    tile_poles<S>(d.g, glb(d.M), d.grav, d.rgrav, sp, G.r0, sh);
+    tend_tile<S, false, false>(d.g, glb(d.M), (RecPtr)d.mrows, d.grav, d.rgrav, d.dt, d.stokes, d.pv_scheme, d.order,
+                               d.wgt, d.coriolis, sp, G, sh, io, nullptr, NoRest{});
     __syncthreads();
   }
 }
@@ -645,7 +1329,7 @@ __global__ void __launch_bounds__(NF) k_gzf_ens(const EnsMember *__restrict__ me
   for (int b = blockIdx.x; b < nitems; b += gridDim.x) {
     const Item it = items[b];
     const EnsMember d = mem[it.member];
-    gzf_item(d.g, glb(d.big), glb(d.small1), it, glb(d.sp.gz_new), glb(d.gz_f_out), glb(d.gz_out), xs);
+    gzf_item(d.g, glb(d.big), glb(d.small1), it, glb(d.sp.gz_new), glb(d.gz_f_out), glb(d.gz_out), xs, threadIdx.x);
     __syncthreads();
   }
 }
@@ -660,7 +1344,7 @@ __global__ void __launch_bounds__(NF) k_uvf_ens(const EnsMember *__restrict__ me
     const MeshG M = glb(d->M);
     const FilterDevG big = glb(d->big);
     const UVPtrsG up = glb(d->up);
-    uvf_item(g, M, d->dt, big, it, up, xs);
+    uvf_item(g, M, d->dt, big, it, up, xs, threadIdx.x);
     __syncthreads();
   }
 }
@@ -681,9 +1365,10 @@ static constexpr int kNarrowChunk = GMC_NARROW_CHUNK;
 // width; n (and n2) are the taps of the row's filters, the window of a chunk
 // is its columns and (n - 1) / 2 on either side (lds: the largest window).
 // Returns the number of chunks the row was cut into.
-static int add_row(std::vector<Item> &v, int row, int kind, int work, int nlon, size_t &lds, int n, int n2 = 0) {
+static int add_row(std::vector<Item> &v, int row, int kind, int work, int nlon, size_t &lds, int n, int n2 = 0,
+                   int chunk_work = kChunkWork) {
   int w = work <= 16 ? std::min(nlon, kNarrowChunk)
-                     : std::min(nlon, std::max(64, (kChunkWork / work + 63) / 64 * 64));
+                     : std::min(nlon, std::max(64, (chunk_work / work + 63) / 64 * 64));
   const int parts = (nlon + w - 1) / w;
   const int h = n > 1 ? (n - 1) / 2 : 0;
   for (int k = 0; k < parts; k++) {
@@ -699,9 +1384,27 @@ struct FusedPlan {
   int n_gz = 0, n_uv = 0;
   size_t lds_gz = 0, lds_uv = 0;
   int rows_split = 0, max_parts = 1, widest = 0;   // reported by gmc_filter_plan
+  // the stage as gmc_step runs it (launches of k_stage; none: the three kernels)
+  int n_stage = 0;
+  StageMap map{};
+  struct Launch {
+    int polar, tile0, tiles, item_lds;
+    Item *d_items;
+    size_t lds;
+  } stage[3] = {};
+  std::vector<void *> mem;   // their device allocations
 };
 
 static FusedPlan *plan_of(gmc_ctx *c) { return (FusedPlan *)c->fused_plan; }
+
+static void plan_free(gmc_ctx *c) {
+  FusedPlan *P = plan_of(c);
+  if (!P) return;
+  if (P->d_items) hip_note(hipFree(P->d_items), "plan free");
+  for (void *m : P->mem) hip_note(hipFree(m), "plan free");
+  delete P;
+  c->fused_plan = nullptr;
+}
 
 // Order a work list for a launch of one workgroup per item whose workgroup b
 // takes item xcd_item(b): each XCD works through one contiguous run of the
@@ -737,6 +1440,152 @@ static std::vector<Item> xcd_deal(const std::vector<Item> &v, W work) {
     for (int k : run[y]) out.push_back(v[k]);
   }
   return out;
+}
+
+template <class T> static int to_device(gmc_ctx *c, FusedPlan *P, const std::vector<T> &v, T *&d, const char *what) {
+  void *m = nullptr;
+  int rc = check_hip(c, hipMalloc(&m, sizeof(T) * std::max<size_t>(v.size(), 1)), what);
+  if (rc) return rc;
+  P->mem.push_back(m);
+  d = (T *)m;
+  return check_hip(c, hipMemcpy(m, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice), what);
+}
+
+// The rows [ra, rb) that tiles take through the whole stage: rows of short
+// filters (and the gz row rb that the last v row reads), at least three from
+// either pole, whose sums and mirrored rows the tiles then never read.
+static void short_rows(int nlat, const std::vector<int32_t> &nb, const std::vector<int32_t> &ns,
+                       const std::vector<int32_t> &nbv, int &ra, int &rb) {
+  const int nhalf = nlat - 1;
+  auto cell = [&](int r) { return nb[r] <= kLaneTaps && ns[r] <= kLaneTaps; };
+  const int mid = nlat / 2;
+  ra = rb = mid;
+  while (ra > 3 && cell(ra - 1) && nbv[ra - 1] <= kLaneTaps) ra--;
+  while (rb < nhalf - 3 && cell(rb) && nbv[rb] <= kLaneTaps && cell(rb + 1)) rb++;
+}
+
+// The launches of the stage.  Grids of at least 64 columns and 24 rows (below
+// that the polar zones are most of the grid) whose short rows are at least
+// half of all take it.
+static int build_stage(gmc_ctx *c, FusedPlan *P, const std::vector<int32_t> &nb, const std::vector<int32_t> &ns,
+                       const std::vector<int32_t> &nbv) {
+  using S = StageTile;
+  const Grid &g = c->grid;
+  const int nlon = g.nlon, nlat = g.nlat, nhalf = g.nhalf;
+  if (nlon < kWave || nlat < 24) return GMC_OK;
+  StageMap &m = P->map;
+  short_rows(nlat, nb, ns, nbv, m.ra, m.rb);
+  if (2 * (m.rb - m.ra) < nlat) return GMC_OK;
+  constexpr size_t kLds = 160 * 1024, kTileLds = sizeof(double) * S::SH_ALL;
+  auto half_width = [](int n) { return n > 1 ? (n - 1) / 2 : 0; };
+  auto divisor = [](int n) { return (uint32_t)((0xffffffffull + n) / n); };
+  // the short rows' tiles: bands of like width in segments (the last segment
+  // takes what does not fit the table at its widest filters)
+  const int nbands = (m.rb - m.ra + S::TY - 1) / S::TY;
+  std::vector<std::pair<int, int>> h(nbands);   // half widths of the filters of gz, and of u and v
+  for (int b = 0; b < nbands; b++) {
+    const int r0 = m.ra + S::TY * b, r1 = std::min(r0 + S::TY, m.rb);
+    for (int r = r0; r <= r1; r++) h[b].first = std::max({h[b].first, half_width(nb[r]), half_width(ns[r])});
+    for (int r = r0; r < r1; r++) h[b].second = std::max({h[b].second, half_width(nb[r]), half_width(nbv[r])});
+  }
+  for (int b = 0; b < nbands;) {
+    int e = b + 1;
+    std::pair<int, int> hh = h[b];
+    while (e < nbands && (h[e] == h[b] || m.nseg == kMaxSegs - 1)) {
+      hh = {std::max(hh.first, h[e].first), std::max(hh.second, h[e].second)};
+      e++;
+    }
+    TileSeg &s = m.seg[m.nseg++];
+    s.b0 = b;
+    s.t0 = m.ntiles;
+    s.hl = std::max(2, 1 + hh.first) + hh.second;
+    s.w = std::min(61, 62 - hh.first) - hh.second - s.hl + 1;
+    s.nx = (nlon + s.w - 1) / s.w;
+    s.w = (nlon + s.nx - 1) / s.nx;
+    s.div = divisor(s.nx);
+    m.ntiles += s.nx * (e - b);
+    b = e;
+  }
+  auto big_lds = [&](std::initializer_list<const void *> fs) {
+    int rc = GMC_OK;
+    for (const void *f : fs)
+      if (!rc) rc = check_hip(c, hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds), "lds");
+    return rc;
+  };
+  int rc;
+  // one launch: bands of the polar rows, if their circles and weights fit
+  const int segs = (nlon + kWave - 1) / kWave;
+  int weights = 0;
+  for (int r = 0; r < nhalf; r++) {
+    if (r >= m.ra && r < m.rb) continue;
+    int w = 0;
+    for (int j = 0; j <= kBandTY && r + j < nlat; j++) {
+      w += std::max(nb[r + j], 0) + std::max(ns[r + j], 0);
+      if (j < kBandTY && r + j < nhalf) w += std::max(nbv[r + j], 0);
+    }
+    weights = std::max(weights, w);
+  }
+  const size_t lds = sizeof(double) * ((size_t)kBandLdsRows * nlon + 8 + weights);
+  if (kBandRows * segs <= kBandLoads * NB_W && (kBandTY + 1) * segs <= kBandOut * NB_W && lds <= kLds) {
+    m.bands_s = (m.ra + kBandTY - 1) / kBandTY;
+    m.bands_p = m.bands_s + (nhalf - m.rb + kBandTY - 1) / kBandTY;
+    P->stage[0] = {m.bands_p + 2 * (kPoleParts - 1), 0, m.ntiles, 0, nullptr, std::max(lds, kTileLds)};
+    rc = big_lds({(const void *)k_stage<kStageOne, false>, (const void *)k_stage<kStageOne, true>});
+    if (!rc) P->n_stage = 1;
+    return rc;
+  }
+  // three launches
+  m.nx_p = (nlon + TX - 1) / TX;
+  m.div_p = divisor(m.nx_p);
+  m.tiles_s = m.nx_p * ((m.ra + S::TY - 1) / S::TY);
+  m.tiles_p = m.tiles_s + m.nx_p * ((nlat - m.rb + S::TY - 1) / S::TY);
+  // filter items of at most kStageWork tap-outputs: four share a workgroup's LDS
+  constexpr int kStageWork = 8192;
+  std::vector<Item> items[3];
+  size_t lgz = 0, luv = 0;
+  for (int r = 0; r < nlat; r++) {
+    if (r >= m.ra && r < m.rb) continue;
+    add_row(items[1], r, 0, nb[r] + std::max(1, nb[r] / 2), nlon, lgz, std::max(nb[r], ns[r]), 0, kStageWork);
+    add_row(items[2], r, 1, nb[r], nlon, luv, nb[r], 0, kStageWork);
+    if (r < nhalf) add_row(items[2], r, 2, nbv[r], nlon, luv, nbv[r], 0, kStageWork);
+  }
+  for (auto &it : items[1]) { it.n = nb[it.row]; it.n2 = ns[it.row]; }
+  for (int k = 1; k < 3; k++) {
+    // heavy and light items share a workgroup: item i of the order by work
+    // goes to workgroup i mod the number of workgroups
+    std::vector<Item> &v = items[k];
+    auto taps = [](const Item &it) { return (int64_t)(it.c1 - it.c0) * std::max(it.n + it.n2, 1); };
+    std::stable_sort(v.begin(), v.end(), [&](const Item &a, const Item &b) { return taps(a) > taps(b); });
+    while (v.size() % kItemsPerWg) v.push_back(Item{1, 0, 0, 1, 0, 0, 0, 0});   // no columns
+    const int n = (int)v.size() / kItemsPerWg;
+    std::vector<Item> dealt(v.size());
+    for (int i = 0; i < (int)v.size(); i++) dealt[i % n * kItemsPerWg + i / n] = v[i];
+    v = dealt;
+  }
+  const size_t item[3] = {0, lgz + sizeof(double) * (c->big.max_taps + c->small1.max_taps),
+                          luv + sizeof(double) * c->big.max_taps};
+  if (kItemsPerWg * std::max(item[1], item[2]) > kLds) return GMC_OK;
+  // the short rows' tiles: what fills the second and third launch up to two
+  // workgroups a compute unit, the two bands beside the polar rows (first and
+  // last in the numbering) in the first
+  constexpr int slots = 2 * 256;
+  const int keep = std::min(m.ntiles, m.seg[0].nx + m.seg[m.nseg - 1].nx);
+  int left = m.ntiles - keep;
+  for (int k = 1; k < 3; k++) {
+    const int polar = (int)items[k].size() / kItemsPerWg, take = std::min(left, std::max(0, slots - polar));
+    P->stage[k] = {polar, 0, take, (int)(item[k] / sizeof(double)), nullptr, std::max(kTileLds, kItemsPerWg * item[k])};
+    left -= take;
+  }
+  const int n0 = keep + left;   // the first launch's tiles, around the numbering's ends
+  P->stage[0] = {m.tiles_p, m.ntiles - (n0 + 1) / 2, n0, 0, nullptr, kTileLds};
+  P->stage[1].tile0 = n0 / 2;
+  P->stage[2].tile0 = n0 / 2 + P->stage[1].tiles;
+  rc = big_lds({(const void *)k_stage<kStageTend, false>, (const void *)k_stage<kStageTend, true>,
+                (const void *)k_stage<kStageGz, false>, (const void *)k_stage<kStageGz, true>,
+                (const void *)k_stage<kStageUv, false>, (const void *)k_stage<kStageUv, true>});
+  for (int k = 1; k < 3 && !rc; k++) rc = to_device(c, P, items[k], P->stage[k].d_items, "stage items alloc");
+  if (!rc) P->n_stage = 3;
+  return rc;
 }
 
 static int build_plan(gmc_ctx *c) {
@@ -791,19 +1640,16 @@ static int build_plan(gmc_ctx *c) {
   rc = check_hip(c, hipMalloc((void **)&P->d_items, sizeof(Item) * items.size()), "plan alloc");
   if (!rc) rc = check_hip(c, hipMemcpy(P->d_items, items.data(), sizeof(Item) * items.size(), hipMemcpyHostToDevice),
                           "plan copy");
-  if (rc) { delete P; return rc; }
+  if (!rc) rc = build_stage(c, P, nb_lon, ns_lon, nb_lat);
   c->fused_plan = P;
-  return GMC_OK;
+  if (rc) plan_free(c);
+  return rc;
 }
 
 void fused_release(gmc_ctx *c) {
   for (auto &sg : c->graphs) hip_note(hipGraphExecDestroy(sg.exec), "step graph destroy");
   c->graphs.clear();
-  if (FusedPlan *P = plan_of(c)) {
-    hip_note(hipFree(P->d_items), "plan free");
-    delete P;
-    c->fused_plan = nullptr;
-  }
+  plan_free(c);
 }
 
 const char *const kKernelNames[kKernelClasses] = {"k_tend", "k_gzf", "k_uvf"};
@@ -840,12 +1686,31 @@ static void fused_stage(gmc_ctx *c, int o, int s, int n, double dt, bool tape = 
   TapeOut T{S[S_M_LON], S[S_M_LAT], S[S_M_VTX], S[S_MFX_LON], S[S_MFY_LAT], S[S_MFX_LAT], S[S_MFY_LON],
             S[S_U_LAT], S[S_V_LON], S[S_PV], S[S_PV_LON], S[S_PV_LAT], nullptr, nullptr};
   if (dst) T = *dst;
+  UVPtrs up{O[S_U_LON], O[S_V_LAT], du, dv, N[S_GZ_F], N[S_U_LON], N[S_V_LAT], N[S_U_F], N[S_V_F]};
+  if (PL->n_stage && !c->prof_ev) {   // gmc_kernel_times times the three kernels on every grid
+    StageArgs A{g, M, c->d_mrows, c->cfg.g, 1.0 / c->cfg.g, dt, c->cfg.upwind_wgt_pv, c->cfg.pv_pole_stokes,
+                c->cfg.pv_scheme, pv_order(c->cfg), c->cfg.coriolis_scheme, sp, up, BandOut{N[S_GZ_F], N[S_GZ]},
+                c->big, c->small1, PL->map, 0, 0, 0, nullptr, 0, T};
+    for (int k = 0; k < PL->n_stage; k++) {
+      const FusedPlan::Launch &L = PL->stage[k];
+      A.polar = L.polar;
+      A.tile0 = L.tile0;
+      A.tiles = L.tiles;
+      A.items = L.d_items;
+      A.item_lds = L.item_lds;
+      auto fn = PL->n_stage == 1 ? (tape ? k_stage<kStageOne, true> : k_stage<kStageOne, false>)
+                : k == 0         ? (tape ? k_stage<kStageTend, true> : k_stage<kStageTend, false>)
+                : k == 1         ? (tape ? k_stage<kStageGz, true> : k_stage<kStageGz, false>)
+                                 : (tape ? k_stage<kStageUv, true> : k_stage<kStageUv, false>);
+      hipLaunchKernelGGL(fn, dim3(L.polar + L.tiles), dim3(StageTile::NT), L.lds, c->stream, A);
+    }
+    return;
+  }
   stage_launch(c, tape ? k_tend<true> : k_tend<false>, dim3(tiles), dim3(Tile<TY_MAIN>::NT), 0, g, M,
                c->d_mrows, c->cfg.g, 1.0 / c->cfg.g, dt, c->cfg.pv_pole_stokes, c->cfg.pv_scheme,
                pv_order(c->cfg), c->cfg.upwind_wgt_pv, c->cfg.coriolis_scheme, sp, T);
   stage_launch(c, k_gzf, dim3(PL->n_gz), dim3(NF), PL->lds_gz, g, c->big, c->small1, PL->d_items, gz_new,
                N[S_GZ_F], N[S_GZ]);
-  UVPtrs up{O[S_U_LON], O[S_V_LAT], du, dv, N[S_GZ_F], N[S_U_LON], N[S_V_LAT], N[S_U_F], N[S_V_F]};
   stage_launch(c, k_uvf, dim3(PL->n_uv), dim3(NF), PL->lds_uv, g, M, dt, c->big, PL->d_items + PL->n_gz, up);
 }
 

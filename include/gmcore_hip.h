@@ -171,7 +171,9 @@ int gmc_time_integrate(gmc_ctx *ctx, int32_t old_level, int32_t new_level, doubl
  * old/new swap of time_advance; repeated nsteps times.  Uses the fused
  * stage kernels, replayed from HIP graphs captured on first use for each
  * (old, new, dt): graphs of 8 steps while 8 or more remain, then graphs of
- * one step; device resident, nothing crosses PCIe. */
+ * one step; device resident, nothing crosses PCIe.  The tendency levels are
+ * its scratch: what they hold afterwards is undefined (as after
+ * gmc_time_integrate). */
 int gmc_step(gmc_ctx *ctx, double dt, int32_t nsteps);
 
 /* Current time level index of `old` (1..3) after gmc_step's swaps. */
@@ -218,7 +220,9 @@ int gmc_synchronize(gmc_ctx *ctx);
  * does (the state advances), launched one by one on the context's stream,
  * each launch with a start and an end HIP event that the dispatch itself
  * stamps (hipExtLaunchKernelGGL), so the figure is the kernel's own duration
- * without the gap before it.  out_ms[k] receives the mean duration in
+ * without the gap before it.  It launches the stage as its three kernels also
+ * on grids where gmc_step gives a stage one launch, or three that share its
+ * work differently; the states are the same, bit for bit.  out_ms[k] receives the mean duration in
  * milliseconds of kernel class k (at most cap classes, *n set to the count);
  * gmc_kernel_name(k) names them. */
 int gmc_kernel_times(gmc_ctx *ctx, double dt, int32_t nsteps, double *out_ms, int32_t cap, int32_t *n);
