@@ -187,41 +187,83 @@ struct InnerPtrs {
 // [0, npole) are the pole rows (2 per tracer, padded to a multiple of the
 // XCD count so that the interior items keep their XCD placement).  An
 // interior item covers the cell rows r0 .. r0 + 6 (r0 = 1 + 7 rb) over one
-// column segment: wavefront w forms the y-fluxes of V row r0 - 1 + w (into
-// LDS, each shared by the cells either side) and, for w < 7, the x-fluxes
-// and the update of cell row r0 + w.  Lane l sits on column 63 s - 1 + l;
-// lanes 1..63 own the cells 63 s .. 63 s + 62, the x-flux on a cell's west
-// face coming from the lane below.  Interior items are numbered (row block,
-// segment, tracer), the tracer fastest, and dealt to the XCDs in contiguous
-// runs, so the wind rows and the neighbouring tracer rows an item reads are
-// already in its XCD's L2.
+// column segment, for a group of up to kGroup tracers: wavefront w forms the
+// y-fluxes of V row r0 - 1 + w (into LDS, each shared by the cells either
+// side) and, for w < 7, the x-fluxes and the update of cell row r0 + w.  Lane
+// l sits on column 63 s - 1 + l; lanes 1..63 own the cells 63 s .. 63 s + 62,
+// the x-flux on a cell's west face coming from the lane below.  Interior items
+// are numbered (row block, segment, group), the group fastest, and dealt to
+// the XCDs in contiguous runs, so the wind rows and the neighbouring tracer
+// rows an item reads are already in its XCD's L2.
+//
+// The kernels are bound by instruction issue.  The wind's share of a face (its
+// weights, direction, stencil address, the reciprocal of its Courant number)
+// is half of a face's instructions and the same for every tracer, so a group
+// forms it once: 232 vector instructions per tracer and cell instead of 430,
+// 40 -> 28 us a kernel at 720 x 361 x 8 tracers.  Groups of 4 at four
+// wavefronts per SIMD: groups of 2 and 8 and six wavefronts took 2 to 10 %
+// longer, eight (spilling) 45 %.
 constexpr int NF = 512;
 constexpr int kSeg = kWave - 1;
 constexpr int kRowsPerItem = NF / kWave - 1;
+constexpr int kGroup = 4;
 struct FluxItem {
   int pole;    // 1: pole row item
-  int r, t;    // pole: cell row; interior: first cell row r0; tracer
+  int r, t;    // pole: cell row; interior: first cell row r0; (first) tracer
   int c0;      // first cell of the segment
+  int nt;      // tracers of the group
 };
-__device__ __forceinline__ FluxItem flux_item(const AdvGrid &g, int ntr) {
+int flux_items(const AdvGrid &g) {
+  return ((g.nlat - 2 + kRowsPerItem - 1) / kRowsPerItem) * ((g.nlon + kSeg - 1) / kSeg);
+}
+// Tracers per item: one where that does not even give every compute unit four
+// workgroups (then the group's serial loop would be the kernel's time), else
+// kGroup.
+int flux_group(const AdvGrid &g, int ntr) { return flux_items(g) * ntr <= 4 * 256 ? 1 : kGroup; }
+__device__ __forceinline__ FluxItem flux_item(const AdvGrid &g, int ntr, int group) {
   const int npole = (2 * ntr + kNumXcd - 1) / kNumXcd * kNumXcd;
   const int b = blockIdx.x;
-  FluxItem it{0, -1, 0, 0};
+  FluxItem it{0, -1, 0, 0, 1};
   if (b < npole) {
     if (b < 2 * ntr) { it.pole = 1; it.r = b % 2 ? g.nlat - 1 : 0; it.t = b / 2; }
     return it;
   }
-  const int nseg = (g.nlon + kSeg - 1) / kSeg, nrb = (g.nlat - 2 + kRowsPerItem - 1) / kRowsPerItem;
-  const int L = xcd_item(b - npole, nrb * nseg * ntr);
-  it.t = L % ntr;
-  const int rs = L / ntr, s = rs % nseg, rb = rs / nseg;
+  const int nseg = (g.nlon + kSeg - 1) / kSeg, ng = (ntr + group - 1) / group;
+  const int nrb = (g.nlat - 2 + kRowsPerItem - 1) / kRowsPerItem, per = nseg * ng;
+  // the two row blocks at either pole, whose x-fluxes cross up to hw whole
+  // cells, go first, one workgroup after the other on all XCDs
+  const int edge = min(2, nrb / 2), e = b - npole;
+  int L, rb;
+  if (e < 2 * edge * per) {
+    L = e % per;
+    rb = e / per;
+    rb = rb & 1 ? nrb - 1 - rb / 2 : rb / 2;
+  } else {
+    L = xcd_item(e - 2 * edge * per, gridDim.x - npole - 2 * edge * per);
+    rb = L / per + edge;
+    L = L % per;
+  }
+  it.t = L % ng * group;
+  it.nt = min(group, ntr - it.t);
   it.r = 1 + kRowsPerItem * rb;
-  it.c0 = s * kSeg;
+  it.c0 = L / ng * kSeg;
   return it;
 }
-int flux_blocks(const AdvGrid &g, int ntr) {
+int flux_blocks(const AdvGrid &g, int ntr, int group) {
   const int npole = (2 * ntr + kNumXcd - 1) / kNumXcd * kNumXcd;
-  return npole + ((g.nlat - 2 + kRowsPerItem - 1) / kRowsPerItem) * ((g.nlon + kSeg - 1) / kSeg) * ntr;
+  return npole + flux_items(g) * ((ntr + group - 1) / group);
+}
+
+// The y-fluxes of a group's V row h through column i into f[t][i's lane].
+template <bool VL, int LIM>
+__device__ __forceinline__ void group_yflux(const AdvGrid &g, int nt, double c, double v, int h, int i,
+                                            const double *my, int64_t tstride, double (*f)[NF]) {
+  if (h < 3 || h > g.nhalf - 4) {   // mirrored rows in reach
+    for (int t = 0; t < nt; t++) f[t][threadIdx.x] = yflux_any<VL>(g, LIM, c, v, h, i, my + t * tstride);
+    return;
+  }
+  const YFace face = y_face<VL>(g, c, v, i);
+  for (int t = 0; t < nt; t++) f[t][threadIdx.x] = y_flux<VL>(g, LIM, face, h, my + t * tstride);
 }
 
 // Sum over the columns of f(i) in wave_zonal_sum's order (lane l adds f(l),
@@ -245,15 +287,12 @@ __device__ __forceinline__ double wave_row_sum(int n, F f) {
 
 // ffsl_calc_tracer_hflx_cell, inner part (ffsl_mod.F90:350-407): the
 // advective half-steps qx, qy of every cell
-// (NF, 8): eight wavefronts per SIMD (four workgroups per CU); without the
-// bound the kernel argument and row registers take more scalar registers
-// than that occupancy allows
 template <bool VL, int LIM>
-__global__ void __launch_bounds__(NF, 8) k_adv_inner(AdvGrid g, Mesh M, int ntr, InnerPtrs p) {
+__global__ void __launch_bounds__(NF, 4) k_adv_inner(AdvGrid g, Mesh M, int ntr, int group, InnerPtrs p) {
   constexpr int lim = LIM;   // the limiter's branches fold at compile time
-  __shared__ double sfy[NF / kWave][kWave];
+  __shared__ double sfy[kGroup][NF];
   __shared__ double bcast;
-  const FluxItem it = flux_item(g, ntr);
+  const FluxItem it = flux_item(g, ntr, group);
   const int n = g.nlon;
   const int64_t toff = it.t * p.tstride, P = g.pitch;
   const double *q = p.q + toff;
@@ -279,32 +318,38 @@ __global__ void __launch_bounds__(NF, 8) k_adv_inner(AdvGrid g, Mesh M, int ntr,
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), l = threadIdx.x % kWave;
   // rows h and r are uniform over the wavefront: row pointers are scalar and
   // the lanes index them with unsigned column offsets
-  const int iw = wrap(it.c0 - 1 + l, n);   // column of the lane
+  const int iw = min(wrap(it.c0 - 1 + l, n), n - 1);   // column of the lane
   const unsigned uiw = iw;
   const int h = it.r - 1 + w, r = it.r + w;
   const bool row = w < kRowsPerItem && r <= g.nlat - 2;   // uniform over the wavefront
-  const int i = it.c0 - 1 + l;   // cell of the lane
-  const bool upd = row && l >= 1 && i < n;
-  const unsigned ui = i;
   const int64_t ro = r * P;
-  // the update's own loads, issued ahead of the fluxes
-  double qc = 0.0, dvx = 0.0, dvy = 0.0;
-  if (upd) {
-    qc = ldu(q + ro, ui);
-    dvx = ldu(p.divx + ro, ui);
-    dvy = ldu(p.divy + ro, ui);
+  // the x faces' and the update's wind, on their way during the y-fluxes
+  double cx = 0.0, ux = 0.0, dvx = 0.0, dvy = 0.0;
+  if (row) {
+    cx = ldu(p.cflx + ro, uiw);
+    ux = ldu(p.u + ro, uiw);
+    dvx = ldu(p.divx + ro, uiw);
+    dvy = ldu(p.divy + ro, uiw);
   }
   if (h <= g.nhalf - 1)
-    sfy[w][l] = yflux_any<VL>(g, lim, ldu(p.cfly + h * P, uiw), ldu(p.v + h * P, uiw), h, iw, q);
-  const double fx = row ? xflux<VL>(g, lim, ldu(p.cflx + ro, uiw), ldu(p.u + ro, uiw), iw, q + ro) : 0.0;
-  const double fxw = __shfl_up(fx, 1, kWave);
+    group_yflux<VL, LIM>(g, it.nt, ldu(p.cfly + h * P, uiw), ldu(p.v + h * P, uiw), h, iw, q, p.tstride, sfy);
   __syncthreads();
-  if (upd) {
-    const double lel = M(GMC_LE_LON, r), ac = M(GMC_AREA_CELL, r);
-    const double ls = M(GMC_LE_LAT, r - 1), ln = M(GMC_LE_LAT, r);
-    const double fs = sfy[w][l], fn = sfy[w + 1][l];
-    stu(p.qx + toff + ro, ui, qc - 0.5 * ((fx - fxw) * lel / ac - dvx * qc) * dt);
-    stu(p.qy + toff + ro, ui, qc - 0.5 * ((fn * ln - fs * ls) / ac - dvy * qc) * dt);
+  if (!row) return;
+  const bool upd = l >= 1 && it.c0 - 1 + l < n;
+  const double lel = M(GMC_LE_LON, r), ac = M(GMC_AREA_CELL, r), rac = 1.0 / ac;
+  const double ls = M(GMC_LE_LAT, r - 1), ln = M(GMC_LE_LAT, r);
+  const XFace face = x_face<VL>(g, cx, ux, iw);
+  for (int t = 0; t < it.nt; t++) {
+    const double *qt = q + t * p.tstride + ro;
+    const double qc = ldu(qt, uiw);
+    const double fx = x_flux<VL>(g, lim, face, qt);
+    const double fxw = __shfl_up(fx, 1, kWave);
+    const double fs = sfy[t][threadIdx.x], fn = sfy[t][threadIdx.x + kWave];
+    if (upd) {
+      const int64_t o = toff + t * p.tstride + ro;
+      stu(p.qx + o, uiw, qc - 0.5 * (div_rn((fx - fxw) * lel, ac, rac) - dvx * qc) * dt);
+      stu(p.qy + o, uiw, qc - 0.5 * (div_rn(fn * ln - fs * ls, ac, rac) - dvy * qc) * dt);
+    }
   }
 }
 
@@ -319,11 +364,11 @@ struct OuterPtrs {
 // outer fluxes (ffsl_mod.F90:410) and adv_run's flux-form update and /m
 // (adv_mod.F90:183-235) of every cell, into qp
 template <bool VL, int LIM>
-__global__ void __launch_bounds__(NF, 8) k_adv_flux(AdvGrid g, Mesh M, int ntr, OuterPtrs p) {
+__global__ void __launch_bounds__(NF, 4) k_adv_flux(AdvGrid g, Mesh M, int ntr, int group, OuterPtrs p) {
   constexpr int lim = LIM;
-  __shared__ double sfy[NF / kWave][kWave];
+  __shared__ double sfy[kGroup][NF];
   __shared__ double bcast;
-  const FluxItem it = flux_item(g, ntr);
+  const FluxItem it = flux_item(g, ntr, group);
   const int n = g.nlon;
   const int64_t toff = it.t * p.tstride, P = g.pitch;
   const double *qx = p.qx + toff, *qy = p.qy + toff, *q = p.q + toff;
@@ -346,50 +391,54 @@ __global__ void __launch_bounds__(NF, 8) k_adv_flux(AdvGrid g, Mesh M, int ntr, 
   }
   if (it.r < 0) return;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), l = threadIdx.x % kWave;
-  const int iw = wrap(it.c0 - 1 + l, n);
+  const int iw = min(wrap(it.c0 - 1 + l, n), n - 1);
   const unsigned uiw = iw;
   const int h = it.r - 1 + w, r = it.r + w;
   const bool row = w < kRowsPerItem && r <= g.nlat - 2;
-  const int i = it.c0 - 1 + l;
-  const bool upd = row && l >= 1 && i < n;
-  const unsigned ui = i;
   const int64_t ro = r * P;
-  // the update's own loads, issued ahead of the fluxes
-  double om = 0.0, qo = 0.0, mn = 1.0;
-  if (upd) {
-    om = ldu(p.old_m + ro, ui);
-    qo = ldu(q + ro, ui);
-    mn = ldu(p.m + ro, ui);
+  double cx = 0.0, ux = 0.0, om = 0.0, mn = 1.0;
+  if (row) {
+    cx = ldu(p.cflx + ro, uiw);
+    ux = ldu(p.mfx + ro, uiw);
+    om = ldu(p.old_m + ro, uiw);
+    mn = ldu(p.m + ro, uiw);
   }
   if (h <= g.nhalf - 1)
-    sfy[w][l] = yflux_any<VL>(g, lim, ldu(p.cfly + h * P, uiw), ldu(p.mfy + h * P, uiw), h, iw, qx);
-  const double fx = row ? xflux<VL>(g, lim, ldu(p.cflx + ro, uiw), ldu(p.mfx + ro, uiw), iw, qy + ro) : 0.0;
-  const double fxw = __shfl_up(fx, 1, kWave);
+    group_yflux<VL, LIM>(g, it.nt, ldu(p.cfly + h * P, uiw), ldu(p.mfy + h * P, uiw), h, iw, qx, p.tstride, sfy);
   __syncthreads();
-  if (upd) {
-    const double lel = M(GMC_LE_LON, r), ac = M(GMC_AREA_CELL, r);
-    const double ls = M(GMC_LE_LAT, r - 1), ln = M(GMC_LE_LAT, r);
-    const double fs = sfy[w][l], fn = sfy[w + 1][l];
-    const double qv = om * qo - ((fx - fxw) * lel + (fn * ln - fs * ls)) / ac * dt;
-    stu(qp + ro, ui, qv / mn);
+  if (!row) return;
+  const bool upd = l >= 1 && it.c0 - 1 + l < n;
+  const double lel = M(GMC_LE_LON, r), ac = M(GMC_AREA_CELL, r), rac = 1.0 / ac, rmn = 1.0 / mn;
+  const double ls = M(GMC_LE_LAT, r - 1), ln = M(GMC_LE_LAT, r);
+  const XFace face = x_face<VL>(g, cx, ux, iw);
+  for (int t = 0; t < it.nt; t++) {
+    const int64_t o = t * p.tstride + ro;
+    const double qo = ldu(q + o, uiw);
+    const double fx = x_flux<VL>(g, lim, face, qy + o);
+    const double fxw = __shfl_up(fx, 1, kWave);
+    const double fs = sfy[t][threadIdx.x], fn = sfy[t][threadIdx.x + kWave];
+    if (upd) {
+      const double qv = om * qo - div_rn((fx - fxw) * lel + (fn * ln - fs * ls), ac, rac) * dt;
+      stu(qp + o, uiw, div_rn(qv, mn, rmn));
+    }
   }
 }
 
 // the instances of the flux kernels for a run's flux type and limiter
 template <bool VL>
-void (*inner_kernel_lim(int lim))(AdvGrid, Mesh, int, InnerPtrs) {
+void (*inner_kernel_lim(int lim))(AdvGrid, Mesh, int, int, InnerPtrs) {
   return lim == GMC_LIMITER_PD ? k_adv_inner<VL, GMC_LIMITER_PD>
        : lim == GMC_LIMITER_NONE ? k_adv_inner<VL, GMC_LIMITER_NONE> : k_adv_inner<VL, GMC_LIMITER_MONO>;
 }
-void (*inner_kernel(bool vl, int lim))(AdvGrid, Mesh, int, InnerPtrs) {
+void (*inner_kernel(bool vl, int lim))(AdvGrid, Mesh, int, int, InnerPtrs) {
   return vl ? inner_kernel_lim<true>(lim) : inner_kernel_lim<false>(lim);
 }
 template <bool VL>
-void (*outer_kernel_lim(int lim))(AdvGrid, Mesh, int, OuterPtrs) {
+void (*outer_kernel_lim(int lim))(AdvGrid, Mesh, int, int, OuterPtrs) {
   return lim == GMC_LIMITER_PD ? k_adv_flux<VL, GMC_LIMITER_PD>
        : lim == GMC_LIMITER_NONE ? k_adv_flux<VL, GMC_LIMITER_NONE> : k_adv_flux<VL, GMC_LIMITER_MONO>;
 }
-void (*outer_kernel(bool vl, int lim))(AdvGrid, Mesh, int, OuterPtrs) {
+void (*outer_kernel(bool vl, int lim))(AdvGrid, Mesh, int, int, OuterPtrs) {
   return vl ? outer_kernel_lim<true>(lim) : outer_kernel_lim<false>(lim);
 }
 
@@ -619,15 +668,15 @@ int run_once(gmc_adv *a, int64_t time_step, bool basis, double scale, char *tape
   }
   if (time_step > 0 && time_step % ns == 0) {
     const int64_t ts = (int64_t)g.nlat * g.pitch;
-    const int ntr = a->cfg.ntracers;
-    const dim3 grid(flux_blocks(g, ntr));
+    const int ntr = a->cfg.ntracers, grp = flux_group(g, ntr);
+    const dim3 grid(flux_blocks(g, ntr, grp));
     // when taping, qx, qy and qp go straight to the tape slot's copies
     auto T = [&](double *p) { return tape ? (double *)(tape + ((char *)p - (char *)a->sm)) : p; };
     double *qx = T(a->qx), *qy = T(a->qy), *qp = T(a->qp);
     InnerPtrs ip{tracer_ptr(a, a->old, 0), qx, qy, a->u, a->v, a->cflx, a->cfly, a->divx, a->divy, ts};
-    adv_launch(a, KA_INNER, inner_kernel(vl, a->cfg.limiter), grid, dim3(NF), 0, g, M, ntr, ip);
+    adv_launch(a, KA_INNER, inner_kernel(vl, a->cfg.limiter), grid, dim3(NF), 0, g, M, ntr, grp, ip);
     OuterPtrs op{qx, qy, tracer_ptr(a, a->old, 0), qp, a->mfx, a->mfy, a->cflx, a->cfly, a->old_m, a->sm, ts};
-    adv_launch(a, KA_FLUX, outer_kernel(vl, a->cfg.limiter), grid, dim3(NF), 0, g, M, ntr, op);
+    adv_launch(a, KA_FLUX, outer_kernel(vl, a->cfg.limiter), grid, dim3(NF), 0, g, M, ntr, grp, op);
     if (tape) {
       // the rest of the step's base state: m, the winds, CFL numbers, split
       // divergences and old_m, and q of both levels (the new level's seams)
@@ -1260,7 +1309,7 @@ __global__ void __launch_bounds__(NA) k_adv_psum2(AdvGrid g, const double *f, in
 __global__ void __launch_bounds__(NF) t_adv_inner(AdvGrid g, Mesh M, int lim, int ntr, TBase b, TWork w) {
   __shared__ double sfy[NF / kWave][kWave];
   __shared__ double bcast;
-  const FluxItem it = flux_item(g, ntr);
+  const FluxItem it = flux_item(g, ntr, 1);
   const int n = g.nlon;
   const int64_t to = it.t * w.ts, P = g.pitch;
   const double *q = b.q + to, *d = w.in + to;
@@ -1307,7 +1356,7 @@ __global__ void __launch_bounds__(NF) t_adv_inner(AdvGrid g, Mesh M, int lim, in
 __global__ void __launch_bounds__(NF) t_adv_outer(AdvGrid g, Mesh M, int lim, int ntr, TBase b, TWork w) {
   __shared__ double sfy[NF / kWave][kWave];
   __shared__ double bcast;
-  const FluxItem it = flux_item(g, ntr);
+  const FluxItem it = flux_item(g, ntr, 1);
   const int n = g.nlon;
   const int64_t to = it.t * w.ts, P = g.pitch;
   const double *qx = b.qx + to, *qy = b.qy + to, *dqx = w.dqx + to, *dqy = w.dqy + to, *d = w.in + to;
@@ -1660,7 +1709,7 @@ void tl_step(gmc_adv *a, const char *slot, int old, const double *in, double *ou
   const size_t F = tl_fields(a);
   double *dqx = a->tl_f + 2 * F, *dqy = a->tl_f + 3 * F, *dqp = a->tl_f + 4 * F, *ps = a->tl_f + 5 * F;
   const TBase b = tape_base(a, slot, old);
-  const dim3 items(flux_blocks(g, ntr));
+  const dim3 items(flux_blocks(g, ntr, 1));
   hipLaunchKernelGGL(t_adv_inner, items, dim3(NF), 0, a->stream, g, M, lim, ntr, b, TWork{in, dqx, dqy, dqp, out, ps, ts});
   hipLaunchKernelGGL(t_adv_outer, items, dim3(NF), 0, a->stream, g, M, lim, ntr, b, TWork{in, dqx, dqy, dqp, out, ps, ts});
   hipLaunchKernelGGL(t_adv_fix, dim3(g.nlat, ntr), dim3(NA), 4 * (size_t)g.nlon * sizeof(double), a->stream, g, b,

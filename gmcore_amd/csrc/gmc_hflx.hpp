@@ -159,6 +159,103 @@ __device__ __forceinline__ double yflux_vl(const AdvGrid &g, int lim, double c, 
   const double dm = slope(lim, up ? f[0] : f[1], fu, up ? f[2] : f[3]);
   return v * (fu + dm * 0.5 * (copysign(1.0, c) - c));
 }
+// ---- the same fluxes with what depends on the wind alone formed once for
+// several tracers: a face's direction, its parabola weights, the reciprocal of
+// its Courant number (the flux's division by c is then div_rn's three
+// operations a tracer) and the address of its stencil, which starts at the
+// upwind cell of each lane instead of being selected from the cells of both
+// directions.
+struct YFace {
+  double s, c, y, ds1, ds2, k3;   // PPM; van Leer: s = v, c
+  unsigned off;                   // columns from row h - 2 (PPM), h - 1 (van Leer), upwind row's first
+  bool up, zero;
+};
+template <bool VL>
+__device__ __forceinline__ YFace y_face(const AdvGrid &g, double c, double v, unsigned i) {
+  YFace f;
+  f.up = c > 0;
+  f.zero = c == 0;
+  f.c = c;
+  f.s = VL || f.up ? v : -v;
+  f.off = i + (f.up ? 0u : (unsigned)g.pitch);
+  if (!VL) {
+    const double s1 = f.up ? 1 - c : 0, s2 = f.up ? 1 : -c;
+    const double ds3 = s2 * s2 * s2 - s1 * s1 * s1;
+    f.ds1 = s2 - s1;
+    f.ds2 = s2 * s2 - s1 * s1;
+    f.k3 = f.ds2 / 2.0 - div_rn(ds3, 3.0, 1.0 / 3.0);
+    f.y = 1.0 / c;
+  }
+  return f;
+}
+// y-flux through V point (h, i) of my, h uniform and at least three rows from
+// either pole (no mirrored rows: those are yflux_any's)
+template <bool VL>
+__device__ __forceinline__ double y_flux(const AdvGrid &g, int lim, const YFace &f, int h, const double *my) {
+  const double *row = my + (h - (VL ? 1 : 2)) * g.pitch;
+  double w[5];
+#pragma unroll
+  for (int k = 0; k < (VL ? 3 : 5); k++) w[k] = ldu(row + k * g.pitch, f.off);
+  if (VL) {
+    const double dm = slope(lim, w[0], w[1], w[2]);
+    return f.s * (w[1] + dm * 0.5 * (copysign(1.0, f.c) - f.c));
+  }
+  const Ppm p = ppm(lim, w[0], w[1], w[2], w[3], w[4]);
+  const double fy = div_rn(f.s * (p.fl * f.ds1 + 0.5 * p.df * f.ds2 + p.f6 * f.k3), f.c, f.y);
+  return f.zero ? 0 : fy;
+}
+
+struct XFace {
+  double s, c, y, cf, ds1, ds2, k3;   // van Leer: s = u, c, y, cf
+  int first, k0, cnt;                 // first stencil column; the whole cells crossed
+  bool up, zero, plain;               // plain (uniform): no lane's stencil wraps around the circle
+};
+template <bool VL> __device__ __forceinline__ XFace x_face(const AdvGrid &g, double c, double u, int i) {
+  XFace f;
+  int ci = (int)c;
+  f.cf = c - ci;
+  ci = ci > g.hw ? g.hw : (ci < -g.hw ? -g.hw : ci);
+  f.up = c > 0;
+  f.zero = c == 0;
+  f.c = c;
+  f.y = 1.0 / c;
+  f.s = VL || f.up ? u : -u;
+  f.first = (f.up ? i - ci : i - ci + 1) - (VL ? 1 : 2);
+  f.k0 = f.up ? i + 1 - ci : i + 1;
+  f.cnt = f.up ? ci : -ci;
+  f.plain = __all(f.first >= 0 && f.first + (VL ? 2 : 4) < g.nlon);
+  if (!VL) {
+    const double s1 = f.up ? 1 - f.cf : 0, s2 = f.up ? 1 : -f.cf;
+    const double ds3 = s2 * s2 * s2 - s1 * s1 * s1;
+    f.ds1 = s2 - s1;
+    f.ds2 = s2 * s2 - s1 * s1;
+    f.k3 = f.ds2 / 2.0 - div_rn(ds3, 3.0, 1.0 / 3.0);
+  }
+  return f;
+}
+template <bool VL>
+__device__ __forceinline__ double x_flux(const AdvGrid &g, int lim, const XFace &f, const double *row) {
+  constexpr int N = VL ? 3 : 5;
+  double w[5];
+  if (f.plain) {
+#pragma unroll
+    for (int k = 0; k < N; k++) w[k] = ldu(row + k, f.first);
+  } else {
+#pragma unroll
+    for (int k = 0; k < N; k++) w[k] = ldu(row, wrap(f.first + k, g.nlon));
+  }
+  const double sum = run_sum(row, f.k0, f.cnt, g.nlon);
+  if (VL) {
+    const double dm = slope(lim, w[0], w[1], w[2]);
+    const double a = f.up ? w[1] + dm * 0.5 * (1 - f.cf) : w[1] - dm * 0.5 * (1 + f.cf);
+    const double fx = div_rn(f.s * (f.up ? f.cf * a + sum : f.cf * a - sum), f.c, f.y);
+    return f.zero ? 0 : fx;
+  }
+  const Ppm p = ppm(lim, w[0], w[1], w[2], w[3], w[4]);
+  const double fx = div_rn(f.s * (sum + p.fl * f.ds1 + 0.5 * p.df * f.ds2 + p.f6 * f.k3), f.c, f.y);
+  return f.zero ? 0 : fx;
+}
+
 template <bool VL>
 __device__ __forceinline__ double xflux(const AdvGrid &g, int lim, double c, double u, int i, const double *row) {
   return VL ? xflux_vl(g, lim, c, u, i, row) : xflux_g(g, lim, c, u, i, row);

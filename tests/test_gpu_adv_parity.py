@@ -202,3 +202,32 @@ def test_half_degree_workload_properties():
             m0, m1 = _fsum_mass(qs[l], ac), _fsum_mass(q, ac)
             assert abs(m1 - m0) <= 1e-12 * m0, (l, (m1 - m0) / m0)
     assert g.fixes >= fix_cpu
+
+
+# tracers in groups of four (more than four workgroups per compute unit) with
+# every remainder, and one by one; segments of 63 columns filled exactly and by
+# one pair more; winds that cross several whole cells and none
+GROUPS = [(630, 120, 900.0, 7, 200, "mono", "ppm", 60.0), (632, 121, 900.0, 6, 200, "pd", "ppm", 60.0),
+          (630, 126, 900.0, 5, 200, "none", "ppm", 1.0), (632, 120, 900.0, 6, 200, "mono", "van_leer", 60.0),
+          (126, 15, 900.0, 2, 50, "mono", "ppm", 40.0), (12, 9, 900.0, 1, 2, "mono", "ppm", 10.0)]
+
+
+@pytest.mark.parametrize("case", GROUPS, ids=lambda c: f"{c[0]}x{c[1]}x{c[3]}-{c[5]}-{c[6]}")
+def test_tracer_groups_bitwise(case):
+    nlon, nlat, dt, ntr, hw, lim, flux, vmax = case
+    nl = Namelist(num_lon=nlon, num_lat=nlat, dt_adv=dt, dt_dyn=dt, limiter_type=lim, ffsl_flux_type=flux)
+    st = AdvSetup(nl, ntr, lon_halo_width=hw)
+    m = st.mesh.metrics
+    ub, vb = init_cond.deform_wind_basis(nlon, nlat, m, 3, 7, vmax)
+    qs = init_cond.tracer_set(nlon, nlat, m, 3, ntr)
+    o, g = _pair(st, qs)
+    g.set_wind_basis(ub, vb)
+    sc = init_cond.wind_scales(3, dt)
+    ones = np.ones((nlat, nlon))
+    for n in range(3):
+        u, v = ub * sc[n], vb * sc[n]
+        o.set_wind(u, v, u, v, ones)
+        assert o.run(n) == 0
+        g.drive(n, sc[n:n + 1])
+        _compare(o, g, ntr, f"step {n}")
+    assert g.fixes == o.fixes
