@@ -213,45 +213,50 @@ struct FluxItem {
   int c0;      // first cell of the segment
   int nt;      // tracers of the group
 };
-int flux_items(const AdvGrid &g) {
-  return ((g.nlat - 2 + kRowsPerItem - 1) / kRowsPerItem) * ((g.nlon + kSeg - 1) / kSeg);
-}
+// How a launch numbers its items: ng groups of `group` tracers, nseg segments,
+// nrb row blocks, the first and last `edge` of them first (below); the two
+// divisions of an item's number as products with 2^32 / n rounded up (exact
+// for the less than 2^16 items of a row block and 2^20 of a launch there are;
+// integer divisions were 0.4 us of a 4.5 us kernel).
+struct FluxMap {
+  int ntr, group, ng, per, nrb, edge, npole;
+  uint64_t div_ng, div_per;
+  __host__ __device__ FluxMap(const AdvGrid &g, int ntr_, int group_) : ntr(ntr_), group(group_) {
+    ng = (ntr + group - 1) / group;
+    per = (g.nlon + kSeg - 1) / kSeg * ng;
+    nrb = (g.nlat - 2 + kRowsPerItem - 1) / kRowsPerItem;
+    edge = nrb / 2 < 2 ? nrb / 2 : 2;
+    npole = (2 * ntr + kNumXcd - 1) / kNumXcd * kNumXcd;
+    div_ng = (0x100000000ull + ng - 1) / ng;
+    div_per = (0x100000000ull + per - 1) / per;
+  }
+  __host__ __device__ int blocks() const { return npole + nrb * per; }
+};
 // Tracers per item: one where that does not even give every compute unit four
-// workgroups (then the group's serial loop would be the kernel's time), else
-// kGroup.
-int flux_group(const AdvGrid &g, int ntr) { return flux_items(g) * ntr <= 4 * 256 ? 1 : kGroup; }
-__device__ __forceinline__ FluxItem flux_item(const AdvGrid &g, int ntr, int group) {
-  const int npole = (2 * ntr + kNumXcd - 1) / kNumXcd * kNumXcd;
+// workgroups, else kGroup.  There the kernels' time is one workgroup's chain of
+// loads, which a face formed in one piece keeps shorter: its stencil covers
+// both wind directions, so it is on its way together with the Courant number
+// (154 x 79 x 3 tracers, van Leer: 4.5 us a kernel against 5.6 grouped).
+int flux_group(const AdvGrid &g, int ntr) { return FluxMap(g, ntr, 1).blocks() <= 4 * 256 ? 1 : kGroup; }
+__device__ __forceinline__ FluxItem flux_item(const AdvGrid &g, const FluxMap &m) {
   const int b = blockIdx.x;
   FluxItem it{0, -1, 0, 0, 1};
-  if (b < npole) {
-    if (b < 2 * ntr) { it.pole = 1; it.r = b % 2 ? g.nlat - 1 : 0; it.t = b / 2; }
+  if (b < m.npole) {
+    if (b < 2 * m.ntr) { it.pole = 1; it.r = b % 2 ? g.nlat - 1 : 0; it.t = b / 2; }
     return it;
   }
-  const int nseg = (g.nlon + kSeg - 1) / kSeg, ng = (ntr + group - 1) / group;
-  const int nrb = (g.nlat - 2 + kRowsPerItem - 1) / kRowsPerItem, per = nseg * ng;
-  // the two row blocks at either pole, whose x-fluxes cross up to hw whole
+  // the `edge` row blocks at either pole, whose x-fluxes cross up to hw whole
   // cells, go first, one workgroup after the other on all XCDs
-  const int edge = min(2, nrb / 2), e = b - npole;
-  int L, rb;
-  if (e < 2 * edge * per) {
-    L = e % per;
-    rb = e / per;
-    rb = rb & 1 ? nrb - 1 - rb / 2 : rb / 2;
-  } else {
-    L = xcd_item(e - 2 * edge * per, gridDim.x - npole - 2 * edge * per);
-    rb = L / per + edge;
-    L = L % per;
-  }
-  it.t = L % ng * group;
-  it.nt = min(group, ntr - it.t);
+  const int e = b - m.npole, first = 2 * m.edge * m.per;
+  const int L = e < first ? e : xcd_item(e - first, m.nrb * m.per - first);
+  int rb = (int)((uint64_t)(unsigned)L * m.div_per >> 32);
+  const int rest = L - rb * m.per, seg = (int)((uint64_t)(unsigned)rest * m.div_ng >> 32);
+  rb = e >= first ? rb + m.edge : rb & 1 ? m.nrb - 1 - rb / 2 : rb / 2;
+  it.t = (rest - seg * m.ng) * m.group;
+  it.nt = min(m.group, m.ntr - it.t);
   it.r = 1 + kRowsPerItem * rb;
-  it.c0 = L / ng * kSeg;
+  it.c0 = seg * kSeg;
   return it;
-}
-int flux_blocks(const AdvGrid &g, int ntr, int group) {
-  const int npole = (2 * ntr + kNumXcd - 1) / kNumXcd * kNumXcd;
-  return npole + flux_items(g) * ((ntr + group - 1) / group);
 }
 
 // The y-fluxes of a group's V row h through column i into f[t][i's lane].
@@ -287,12 +292,12 @@ __device__ __forceinline__ double wave_row_sum(int n, F f) {
 
 // ffsl_calc_tracer_hflx_cell, inner part (ffsl_mod.F90:350-407): the
 // advective half-steps qx, qy of every cell
-template <bool VL, int LIM>
-__global__ void __launch_bounds__(NF, 4) k_adv_inner(AdvGrid g, Mesh M, int ntr, int group, InnerPtrs p) {
+template <bool VL, int LIM, bool GROUPED>
+__global__ void __launch_bounds__(NF, GROUPED ? 4 : 8) k_adv_inner(AdvGrid g, Mesh M, FluxMap map, InnerPtrs p) {
   constexpr int lim = LIM;   // the limiter's branches fold at compile time
-  __shared__ double sfy[kGroup][NF];
+  __shared__ double sfy[GROUPED ? kGroup : 1][NF];
   __shared__ double bcast;
-  const FluxItem it = flux_item(g, ntr, group);
+  const FluxItem it = flux_item(g, map);
   const int n = g.nlon;
   const int64_t toff = it.t * p.tstride, P = g.pitch;
   const double *q = p.q + toff;
@@ -323,6 +328,28 @@ __global__ void __launch_bounds__(NF, 4) k_adv_inner(AdvGrid g, Mesh M, int ntr,
   const int h = it.r - 1 + w, r = it.r + w;
   const bool row = w < kRowsPerItem && r <= g.nlat - 2;   // uniform over the wavefront
   const int64_t ro = r * P;
+  const bool upd = row && l >= 1 && it.c0 - 1 + l < n;
+  if constexpr (!GROUPED) {   // the update's own loads, issued ahead of the fluxes
+    double qc = 0.0, dvx = 0.0, dvy = 0.0;
+    if (upd) {
+      qc = ldu(q + ro, uiw);
+      dvx = ldu(p.divx + ro, uiw);
+      dvy = ldu(p.divy + ro, uiw);
+    }
+    if (h <= g.nhalf - 1)
+      sfy[0][threadIdx.x] = yflux_any<VL>(g, lim, ldu(p.cfly + h * P, uiw), ldu(p.v + h * P, uiw), h, iw, q);
+    const double fx = row ? xflux<VL>(g, lim, ldu(p.cflx + ro, uiw), ldu(p.u + ro, uiw), iw, q + ro) : 0.0;
+    const double fxw = __shfl_up(fx, 1, kWave);
+    __syncthreads();
+    if (upd) {
+      const double lel = M(GMC_LE_LON, r), ac = M(GMC_AREA_CELL, r);
+      const double ls = M(GMC_LE_LAT, r - 1), ln = M(GMC_LE_LAT, r);
+      const double fs = sfy[0][threadIdx.x], fn = sfy[0][threadIdx.x + kWave];
+      stu(p.qx + toff + ro, uiw, qc - 0.5 * ((fx - fxw) * lel / ac - dvx * qc) * dt);
+      stu(p.qy + toff + ro, uiw, qc - 0.5 * ((fn * ln - fs * ls) / ac - dvy * qc) * dt);
+    }
+    return;
+  }
   // the x faces' and the update's wind, on their way during the y-fluxes
   double cx = 0.0, ux = 0.0, dvx = 0.0, dvy = 0.0;
   if (row) {
@@ -335,7 +362,6 @@ __global__ void __launch_bounds__(NF, 4) k_adv_inner(AdvGrid g, Mesh M, int ntr,
     group_yflux<VL, LIM>(g, it.nt, ldu(p.cfly + h * P, uiw), ldu(p.v + h * P, uiw), h, iw, q, p.tstride, sfy);
   __syncthreads();
   if (!row) return;
-  const bool upd = l >= 1 && it.c0 - 1 + l < n;
   const double lel = M(GMC_LE_LON, r), ac = M(GMC_AREA_CELL, r), rac = 1.0 / ac;
   const double ls = M(GMC_LE_LAT, r - 1), ln = M(GMC_LE_LAT, r);
   const XFace face = x_face<VL>(g, cx, ux, iw);
@@ -363,12 +389,12 @@ struct OuterPtrs {
 
 // outer fluxes (ffsl_mod.F90:410) and adv_run's flux-form update and /m
 // (adv_mod.F90:183-235) of every cell, into qp
-template <bool VL, int LIM>
-__global__ void __launch_bounds__(NF, 4) k_adv_flux(AdvGrid g, Mesh M, int ntr, int group, OuterPtrs p) {
+template <bool VL, int LIM, bool GROUPED>
+__global__ void __launch_bounds__(NF, GROUPED ? 4 : 8) k_adv_flux(AdvGrid g, Mesh M, FluxMap map, OuterPtrs p) {
   constexpr int lim = LIM;
-  __shared__ double sfy[kGroup][NF];
+  __shared__ double sfy[GROUPED ? kGroup : 1][NF];
   __shared__ double bcast;
-  const FluxItem it = flux_item(g, ntr, group);
+  const FluxItem it = flux_item(g, map);
   const int n = g.nlon;
   const int64_t toff = it.t * p.tstride, P = g.pitch;
   const double *qx = p.qx + toff, *qy = p.qy + toff, *q = p.q + toff;
@@ -396,6 +422,28 @@ __global__ void __launch_bounds__(NF, 4) k_adv_flux(AdvGrid g, Mesh M, int ntr, 
   const int h = it.r - 1 + w, r = it.r + w;
   const bool row = w < kRowsPerItem && r <= g.nlat - 2;
   const int64_t ro = r * P;
+  const bool upd = row && l >= 1 && it.c0 - 1 + l < n;
+  if constexpr (!GROUPED) {
+    double om = 0.0, qo = 0.0, mn = 1.0;
+    if (upd) {
+      om = ldu(p.old_m + ro, uiw);
+      qo = ldu(q + ro, uiw);
+      mn = ldu(p.m + ro, uiw);
+    }
+    if (h <= g.nhalf - 1)
+      sfy[0][threadIdx.x] = yflux_any<VL>(g, lim, ldu(p.cfly + h * P, uiw), ldu(p.mfy + h * P, uiw), h, iw, qx);
+    const double fx = row ? xflux<VL>(g, lim, ldu(p.cflx + ro, uiw), ldu(p.mfx + ro, uiw), iw, qy + ro) : 0.0;
+    const double fxw = __shfl_up(fx, 1, kWave);
+    __syncthreads();
+    if (upd) {
+      const double lel = M(GMC_LE_LON, r), ac = M(GMC_AREA_CELL, r);
+      const double ls = M(GMC_LE_LAT, r - 1), ln = M(GMC_LE_LAT, r);
+      const double fs = sfy[0][threadIdx.x], fn = sfy[0][threadIdx.x + kWave];
+      const double qv = om * qo - ((fx - fxw) * lel + (fn * ln - fs * ls)) / ac * dt;
+      stu(qp + ro, uiw, qv / mn);
+    }
+    return;
+  }
   double cx = 0.0, ux = 0.0, om = 0.0, mn = 1.0;
   if (row) {
     cx = ldu(p.cflx + ro, uiw);
@@ -407,7 +455,6 @@ __global__ void __launch_bounds__(NF, 4) k_adv_flux(AdvGrid g, Mesh M, int ntr, 
     group_yflux<VL, LIM>(g, it.nt, ldu(p.cfly + h * P, uiw), ldu(p.mfy + h * P, uiw), h, iw, qx, p.tstride, sfy);
   __syncthreads();
   if (!row) return;
-  const bool upd = l >= 1 && it.c0 - 1 + l < n;
   const double lel = M(GMC_LE_LON, r), ac = M(GMC_AREA_CELL, r), rac = 1.0 / ac, rmn = 1.0 / mn;
   const double ls = M(GMC_LE_LAT, r - 1), ln = M(GMC_LE_LAT, r);
   const XFace face = x_face<VL>(g, cx, ux, iw);
@@ -424,22 +471,24 @@ __global__ void __launch_bounds__(NF, 4) k_adv_flux(AdvGrid g, Mesh M, int ntr, 
   }
 }
 
-// the instances of the flux kernels for a run's flux type and limiter
-template <bool VL>
-void (*inner_kernel_lim(int lim))(AdvGrid, Mesh, int, int, InnerPtrs) {
-  return lim == GMC_LIMITER_PD ? k_adv_inner<VL, GMC_LIMITER_PD>
-       : lim == GMC_LIMITER_NONE ? k_adv_inner<VL, GMC_LIMITER_NONE> : k_adv_inner<VL, GMC_LIMITER_MONO>;
+// the instances of the flux kernels for a run's flux type, limiter and items
+typedef void (*InnerKernel)(AdvGrid, Mesh, FluxMap, InnerPtrs);
+typedef void (*OuterKernel)(AdvGrid, Mesh, FluxMap, OuterPtrs);
+template <bool VL, bool GROUPED> InnerKernel inner_kernel_lim(int lim) {
+  return lim == GMC_LIMITER_PD ? k_adv_inner<VL, GMC_LIMITER_PD, GROUPED>
+       : lim == GMC_LIMITER_NONE ? k_adv_inner<VL, GMC_LIMITER_NONE, GROUPED> : k_adv_inner<VL, GMC_LIMITER_MONO, GROUPED>;
 }
-void (*inner_kernel(bool vl, int lim))(AdvGrid, Mesh, int, int, InnerPtrs) {
-  return vl ? inner_kernel_lim<true>(lim) : inner_kernel_lim<false>(lim);
+InnerKernel inner_kernel(bool vl, int lim, bool grouped) {
+  return vl ? (grouped ? inner_kernel_lim<true, true>(lim) : inner_kernel_lim<true, false>(lim))
+            : (grouped ? inner_kernel_lim<false, true>(lim) : inner_kernel_lim<false, false>(lim));
 }
-template <bool VL>
-void (*outer_kernel_lim(int lim))(AdvGrid, Mesh, int, int, OuterPtrs) {
-  return lim == GMC_LIMITER_PD ? k_adv_flux<VL, GMC_LIMITER_PD>
-       : lim == GMC_LIMITER_NONE ? k_adv_flux<VL, GMC_LIMITER_NONE> : k_adv_flux<VL, GMC_LIMITER_MONO>;
+template <bool VL, bool GROUPED> OuterKernel outer_kernel_lim(int lim) {
+  return lim == GMC_LIMITER_PD ? k_adv_flux<VL, GMC_LIMITER_PD, GROUPED>
+       : lim == GMC_LIMITER_NONE ? k_adv_flux<VL, GMC_LIMITER_NONE, GROUPED> : k_adv_flux<VL, GMC_LIMITER_MONO, GROUPED>;
 }
-void (*outer_kernel(bool vl, int lim))(AdvGrid, Mesh, int, int, OuterPtrs) {
-  return vl ? outer_kernel_lim<true>(lim) : outer_kernel_lim<false>(lim);
+OuterKernel outer_kernel(bool vl, int lim, bool grouped) {
+  return vl ? (grouped ? outer_kernel_lim<true, true>(lim) : outer_kernel_lim<true, false>(lim))
+            : (grouped ? outer_kernel_lim<false, true>(lim) : outer_kernel_lim<false, false>(lim));
 }
 
 struct FixPtrs {
@@ -669,14 +718,15 @@ int run_once(gmc_adv *a, int64_t time_step, bool basis, double scale, char *tape
   if (time_step > 0 && time_step % ns == 0) {
     const int64_t ts = (int64_t)g.nlat * g.pitch;
     const int ntr = a->cfg.ntracers, grp = flux_group(g, ntr);
-    const dim3 grid(flux_blocks(g, ntr, grp));
+    const FluxMap map(g, ntr, grp);
+    const dim3 grid(map.blocks());
     // when taping, qx, qy and qp go straight to the tape slot's copies
     auto T = [&](double *p) { return tape ? (double *)(tape + ((char *)p - (char *)a->sm)) : p; };
     double *qx = T(a->qx), *qy = T(a->qy), *qp = T(a->qp);
     InnerPtrs ip{tracer_ptr(a, a->old, 0), qx, qy, a->u, a->v, a->cflx, a->cfly, a->divx, a->divy, ts};
-    adv_launch(a, KA_INNER, inner_kernel(vl, a->cfg.limiter), grid, dim3(NF), 0, g, M, ntr, grp, ip);
+    adv_launch(a, KA_INNER, inner_kernel(vl, a->cfg.limiter, grp > 1), grid, dim3(NF), 0, g, M, map, ip);
     OuterPtrs op{qx, qy, tracer_ptr(a, a->old, 0), qp, a->mfx, a->mfy, a->cflx, a->cfly, a->old_m, a->sm, ts};
-    adv_launch(a, KA_FLUX, outer_kernel(vl, a->cfg.limiter), grid, dim3(NF), 0, g, M, ntr, grp, op);
+    adv_launch(a, KA_FLUX, outer_kernel(vl, a->cfg.limiter, grp > 1), grid, dim3(NF), 0, g, M, map, op);
     if (tape) {
       // the rest of the step's base state: m, the winds, CFL numbers, split
       // divergences and old_m, and q of both levels (the new level's seams)
@@ -1309,7 +1359,7 @@ __global__ void __launch_bounds__(NA) k_adv_psum2(AdvGrid g, const double *f, in
 __global__ void __launch_bounds__(NF) t_adv_inner(AdvGrid g, Mesh M, int lim, int ntr, TBase b, TWork w) {
   __shared__ double sfy[NF / kWave][kWave];
   __shared__ double bcast;
-  const FluxItem it = flux_item(g, ntr, 1);
+  const FluxItem it = flux_item(g, FluxMap(g, ntr, 1));
   const int n = g.nlon;
   const int64_t to = it.t * w.ts, P = g.pitch;
   const double *q = b.q + to, *d = w.in + to;
@@ -1356,7 +1406,7 @@ __global__ void __launch_bounds__(NF) t_adv_inner(AdvGrid g, Mesh M, int lim, in
 __global__ void __launch_bounds__(NF) t_adv_outer(AdvGrid g, Mesh M, int lim, int ntr, TBase b, TWork w) {
   __shared__ double sfy[NF / kWave][kWave];
   __shared__ double bcast;
-  const FluxItem it = flux_item(g, ntr, 1);
+  const FluxItem it = flux_item(g, FluxMap(g, ntr, 1));
   const int n = g.nlon;
   const int64_t to = it.t * w.ts, P = g.pitch;
   const double *qx = b.qx + to, *qy = b.qy + to, *dqx = w.dqx + to, *dqy = w.dqy + to, *d = w.in + to;
@@ -1709,7 +1759,7 @@ void tl_step(gmc_adv *a, const char *slot, int old, const double *in, double *ou
   const size_t F = tl_fields(a);
   double *dqx = a->tl_f + 2 * F, *dqy = a->tl_f + 3 * F, *dqp = a->tl_f + 4 * F, *ps = a->tl_f + 5 * F;
   const TBase b = tape_base(a, slot, old);
-  const dim3 items(flux_blocks(g, ntr, 1));
+  const dim3 items(FluxMap(g, ntr, 1).blocks());
   hipLaunchKernelGGL(t_adv_inner, items, dim3(NF), 0, a->stream, g, M, lim, ntr, b, TWork{in, dqx, dqy, dqp, out, ps, ts});
   hipLaunchKernelGGL(t_adv_outer, items, dim3(NF), 0, a->stream, g, M, lim, ntr, b, TWork{in, dqx, dqy, dqp, out, ps, ts});
   hipLaunchKernelGGL(t_adv_fix, dim3(g.nlat, ntr), dim3(NA), 4 * (size_t)g.nlon * sizeof(double), a->stream, g, b,
