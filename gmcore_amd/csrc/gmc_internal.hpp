@@ -102,6 +102,7 @@ struct FilterDev {
 struct HostStage {
   double *p = nullptr;
   size_t cap = 0;   // doubles
+  std::vector<hipEvent_t> ev;   // the ends of a download's pieces
 };
 // rows x nlon doubles between dev (row pitch `pitch`) and host (leading
 // dimension ld), through s; returns once the copy is complete.
