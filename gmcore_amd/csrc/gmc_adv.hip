@@ -225,7 +225,8 @@ struct FluxMap {
     ng = (ntr + group - 1) / group;
     per = (g.nlon + kSeg - 1) / kSeg * ng;
     nrb = (g.nlat - 2 + kRowsPerItem - 1) / kRowsPerItem;
-    edge = nrb / 2 < 2 ? nrb / 2 : 2;
+    // one tracer an item: all items run at once, in the order that shares L2s
+    edge = group == 1 ? 0 : nrb / 2 < 2 ? nrb / 2 : 2;
     npole = (2 * ntr + kNumXcd - 1) / kNumXcd * kNumXcd;
     div_ng = (0x100000000ull + ng - 1) / ng;
     div_per = (0x100000000ull + per - 1) / per;
