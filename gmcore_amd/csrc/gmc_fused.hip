@@ -1166,24 +1166,24 @@ struct StageArgs {
 using StageTile = Tile<11>;
 constexpr int kItemsPerWg = StageTile::NT / NF;
 
-__device__ __forceinline__ TileGeo short_tile(const StageMap &S, int nlon, int t) {
+template <int TY> __device__ __forceinline__ TileGeo short_tile(const StageMap &S, int nlon, int t) {
   TileSeg s = S.seg[0];
 #pragma unroll
   for (int k = 1; k < kMaxSegs; k++)
     if (k < S.nseg && t >= S.seg[k].t0) s = S.seg[k];
   const int e = t - s.t0, b = (int)(((uint64_t)(uint32_t)e * s.div) >> 32), x = e - b * s.nx;
-  const int r0 = S.ra + (s.b0 + b) * StageTile::TY, c0 = x * s.w;
-  return TileGeo{c0, min(s.w, nlon - c0), s.hl, r0, min(r0 + StageTile::TY, S.rb)};
+  const int r0 = S.ra + (s.b0 + b) * TY, c0 = x * s.w;
+  return TileGeo{c0, min(s.w, nlon - c0), s.hl, r0, min(r0 + TY, S.rb)};
 }
 
 // Tile e of the polar tendencies: bands from the south pole to row ra, then
 // from row rb to the north pole.
-__device__ __forceinline__ TileGeo polar_tile(const StageMap &S, const Grid &g, int e) {
+template <int TY> __device__ __forceinline__ TileGeo polar_tile(const StageMap &S, const Grid &g, int e) {
   const bool north = e >= S.tiles_s;
   if (north) e -= S.tiles_s;
   const int b = (int)(((uint64_t)(uint32_t)e * S.div_p) >> 32), x = e - b * S.nx_p;
-  const int r0 = (north ? S.rb : 0) + b * StageTile::TY, c0 = x * TX;
-  return TileGeo{c0, min(TX, g.nlon - c0), HXL, r0, min(r0 + StageTile::TY, north ? g.nlat : S.ra)};
+  const int r0 = (north ? S.rb : 0) + b * TY, c0 = x * TX;
+  return TileGeo{c0, min(TX, g.nlon - c0), HXL, r0, min(r0 + TY, north ? g.nlat : S.ra)};
 }
 
 // The work of polar workgroup e: kPoleParts workgroups for the band at each
@@ -1209,14 +1209,14 @@ __global__ void __launch_bounds__(StageTile::NT, PHASE == kStageOne ? 4 : 8) k_s
   if (b >= A.polar) {
     int t = A.tile0 + xcd_item(b - A.polar, A.tiles);
     t = t >= A.S.ntiles ? t - A.S.ntiles : t;
-    const TileGeo geo = short_tile(A.S, A.g.nlon, t);
+    const TileGeo geo = short_tile<S::TY>(A.S, A.g.nlon, t);
     const TileRest<FilterDev, const double *, double *> rest{A.big,  A.small, A.U.u_old, A.U.v_old, A.U.u,
                                                              A.U.v,  A.U.u_f, A.U.v_f,   A.G.gz_f,  A.G.gz};
     const TileIn io = tile_fetch<S>(A.g, A.P, geo);
     tend_tile<S, TAPE, true>(A.g, A.M, (RecPtr)A.mrows, A.grav, A.rgrav, A.dt, A.stokes, A.pv_scheme, A.order, A.wgt,
                              A.coriolis, A.P, geo, xs, io, &A.tape, rest);
   } else if constexpr (PHASE == kStageTend) {
-    const TileGeo geo = polar_tile(A.S, A.g, b);
+    const TileGeo geo = polar_tile<S::TY>(A.S, A.g, b);
     const TileIn io = tile_fetch<S>(A.g, A.P, geo);
     tile_poles<S>(A.g, A.M, A.grav, A.rgrav, A.P, geo.r0, xs);
     tend_tile<S, TAPE, false>(A.g, A.M, (RecPtr)A.mrows, A.grav, A.rgrav, A.dt, A.stokes, A.pv_scheme, A.order, A.wgt,
@@ -1241,7 +1241,12 @@ __global__ void __launch_bounds__(StageTile::NT, PHASE == kStageOne ? 4 : 8) k_s
 // A member's descriptor for one stage holds its geometry, tables, options,
 // stage dt and field pointers; tiles and filter items of all members are
 // numbered consecutively and each workgroup finds its member by the tile
-// offset (k_tend) or the item's member index (filters).
+// offset (k_tend) or the item's member index (filters).  The rows of short
+// filters go through their tiles whole, as in k_stage, and only the polar rows
+// through the filter kernels: bound by the passes over memory between the
+// kernels and by the number of filter workgroups.  At 16 members (8 of 180 x
+// 91, 6 of 360 x 181, 2 of 720 x 361) a stage's kernels took 38.5, 23.5 and
+// 12.7 us with every row in all three and 49.4, 7.7 and 11.3 us so.
 struct EnsMember {
   Grid g;
   Mesh M;
@@ -1253,7 +1258,8 @@ struct EnsMember {
   UVPtrs up;
   double *gz_f_out;    // gz_f of the new state (big filter output)
   double *gz_out;      // gz of the new state (small filter output)
-  int tile0, nx;       // first tile of the member, tiles per tile row
+  int tile0;           // first tile of the member: map.tiles_p of the polar rows, then map.ntiles
+  StageMap map;
 };
 
 // Field pointers read from a descriptor in memory are generic (FLAT) to the
@@ -1313,12 +1319,21 @@ __global__ void __launch_bounds__(S::NT, 8) k_tend_ens(const EnsMember *__restri
     }
     const EnsMember d = mem[lo];   // a private copy: no aliasing with the stores of the tile
     const int lt = t - d.tile0;
-    const TileGeo G = tile_geo<S>(d.g, lt % d.nx, lt / d.nx);
     const StagePtrsG sp = glb(d.sp);
-    const TileIn io = tile_fetch<S>(d.g, sp, G);
-    tile_poles<S>(d.g, glb(d.M), d.grav, d.rgrav, sp, G.r0, sh);
-    tend_tile<S, false, false>(d.g, glb(d.M), (RecPtr)d.mrows, d.grav, d.rgrav, d.dt, d.stokes, d.pv_scheme, d.order,
-                               d.wgt, d.coriolis, sp, G, sh, io, nullptr, NoRest{});
+    if (lt < d.map.tiles_p) {
+      const TileGeo G = polar_tile<S::TY>(d.map, d.g, lt);
+      const TileIn io = tile_fetch<S>(d.g, sp, G);
+      tile_poles<S>(d.g, glb(d.M), d.grav, d.rgrav, sp, G.r0, sh);
+      tend_tile<S, false, false>(d.g, glb(d.M), (RecPtr)d.mrows, d.grav, d.rgrav, d.dt, d.stokes, d.pv_scheme,
+                                 d.order, d.wgt, d.coriolis, sp, G, sh, io, nullptr, NoRest{});
+    } else {
+      const TileGeo G = short_tile<S::TY>(d.map, d.g.nlon, lt - d.map.tiles_p);
+      const TileRest<FilterDev, const double *, double *> rest{d.big,  d.small1, d.up.u_old, d.up.v_old, d.up.u,
+                                                               d.up.v, d.up.u_f, d.up.v_f,   d.gz_f_out, d.gz_out};
+      const TileIn io = tile_fetch<S>(d.g, sp, G);
+      tend_tile<S, false, true>(d.g, glb(d.M), (RecPtr)d.mrows, d.grav, d.rgrav, d.dt, d.stokes, d.pv_scheme, d.order,
+                                d.wgt, d.coriolis, sp, G, sh, io, nullptr, rest);
+    }
     __syncthreads();
   }
 }
@@ -1464,27 +1479,30 @@ static void short_rows(int nlat, const std::vector<int32_t> &nb, const std::vect
   while (rb < nhalf - 3 && cell(rb) && nbv[rb] <= kLaneTaps && cell(rb + 1)) rb++;
 }
 
-// The launches of the stage.  Grids of at least 64 columns and 24 rows (below
-// that the polar zones are most of the grid) whose short rows are at least
-// half of all take it.
-static int build_stage(gmc_ctx *c, FusedPlan *P, const std::vector<int32_t> &nb, const std::vector<int32_t> &ns,
-                       const std::vector<int32_t> &nbv) {
-  using S = StageTile;
-  const Grid &g = c->grid;
-  const int nlon = g.nlon, nlat = g.nlat, nhalf = g.nhalf;
-  if (nlon < kWave || nlat < 24) return GMC_OK;
-  StageMap &m = P->map;
-  short_rows(nlat, nb, ns, nbv, m.ra, m.rb);
-  if (2 * (m.rb - m.ra) < nlat) return GMC_OK;
-  constexpr size_t kLds = 160 * 1024, kTileLds = sizeof(double) * S::SH_ALL;
+// The rows of a grid that tiles of height ty take through the whole stage, and
+// those tiles: bands of like width in segments (the last segment takes what
+// does not fit the table at its widest filters); the tiles of the other rows'
+// tendencies.  Grids of at least 64 columns and 24 rows (below that the polar
+// zones are most of the grid) whose short rows are at least half of all have
+// such rows; false, and every row among the others, elsewhere.
+static bool stage_map(int nlon, int nlat, const std::vector<int32_t> &nb, const std::vector<int32_t> &ns,
+                      const std::vector<int32_t> &nbv, int ty, StageMap &m) {
+  m = StageMap{};
   auto half_width = [](int n) { return n > 1 ? (n - 1) / 2 : 0; };
   auto divisor = [](int n) { return (uint32_t)((0xffffffffull + n) / n); };
-  // the short rows' tiles: bands of like width in segments (the last segment
-  // takes what does not fit the table at its widest filters)
-  const int nbands = (m.rb - m.ra + S::TY - 1) / S::TY;
+  m.ra = m.rb = nlat;
+  if (nlon >= kWave && nlat >= 24) short_rows(nlat, nb, ns, nbv, m.ra, m.rb);
+  const bool has = 2 * (m.rb - m.ra) >= nlat;
+  if (!has) m.ra = m.rb = nlat;
+  m.nx_p = (nlon + TX - 1) / TX;
+  m.div_p = divisor(m.nx_p);
+  m.tiles_s = m.nx_p * ((m.ra + ty - 1) / ty);
+  m.tiles_p = m.tiles_s + m.nx_p * ((nlat - m.rb + ty - 1) / ty);
+  if (!has) return false;
+  const int nbands = (m.rb - m.ra + ty - 1) / ty;
   std::vector<std::pair<int, int>> h(nbands);   // half widths of the filters of gz, and of u and v
   for (int b = 0; b < nbands; b++) {
-    const int r0 = m.ra + S::TY * b, r1 = std::min(r0 + S::TY, m.rb);
+    const int r0 = m.ra + ty * b, r1 = std::min(r0 + ty, m.rb);
     for (int r = r0; r <= r1; r++) h[b].first = std::max({h[b].first, half_width(nb[r]), half_width(ns[r])});
     for (int r = r0; r < r1; r++) h[b].second = std::max({h[b].second, half_width(nb[r]), half_width(nbv[r])});
   }
@@ -1506,6 +1524,18 @@ static int build_stage(gmc_ctx *c, FusedPlan *P, const std::vector<int32_t> &nb,
     m.ntiles += s.nx * (e - b);
     b = e;
   }
+  return true;
+}
+
+// The launches of the stage.
+static int build_stage(gmc_ctx *c, FusedPlan *P, const std::vector<int32_t> &nb, const std::vector<int32_t> &ns,
+                       const std::vector<int32_t> &nbv) {
+  using S = StageTile;
+  const Grid &g = c->grid;
+  const int nlon = g.nlon, nlat = g.nlat, nhalf = g.nhalf;
+  StageMap &m = P->map;
+  if (!stage_map(nlon, nlat, nb, ns, nbv, S::TY, m)) return GMC_OK;
+  constexpr size_t kLds = 160 * 1024, kTileLds = sizeof(double) * S::SH_ALL;
   auto big_lds = [&](std::initializer_list<const void *> fs) {
     int rc = GMC_OK;
     for (const void *f : fs)
@@ -1535,10 +1565,6 @@ static int build_stage(gmc_ctx *c, FusedPlan *P, const std::vector<int32_t> &nb,
     return rc;
   }
   // three launches
-  m.nx_p = (nlon + TX - 1) / TX;
-  m.div_p = divisor(m.nx_p);
-  m.tiles_s = m.nx_p * ((m.ra + S::TY - 1) / S::TY);
-  m.tiles_p = m.tiles_s + m.nx_p * ((nlat - m.rb + S::TY - 1) / S::TY);
   // filter items of at most kStageWork tap-outputs: four share a workgroup's LDS
   constexpr int kStageWork = 8192;
   std::vector<Item> items[3];
@@ -1845,6 +1871,7 @@ struct gmc_ens {
   int n_gz = 0, n_uv = 0;
   size_t lds_gz = 0, lds_uv = 0;
   int total_tiles = 0;
+  std::vector<std::vector<int32_t>> nb_lon, nb_lat, ns_lon;   // taps of the members' rows
   std::vector<double> dt;           // dt the tables were built for
   int built_shape = -1;
   // graphs of one step and of kEnsBlock steps, by the parity they start from
@@ -1875,12 +1902,13 @@ int build_tables(gmc_ens *e) {
   const int nm = (int)e->m.size(), ty = kEnsShapes[e->shape].ty;
   std::vector<EnsMember> tab((size_t)2 * e->nstage * nm);
   int tiles = 0;
-  std::vector<int> tile0(nm), nx(nm);
+  std::vector<int> tile0(nm);
+  std::vector<StageMap> map(nm);
   for (int k = 0; k < nm; k++) {
     const Grid &g = e->m[k]->grid;
-    nx[k] = (g.nlon + TX - 1) / TX;
+    stage_map(g.nlon, g.nlat, e->nb_lon[k], e->ns_lon[k], e->nb_lat[k], ty, map[k]);
     tile0[k] = tiles;
-    tiles += nx[k] * ((g.nlat + ty - 1) / ty);
+    tiles += map[k].tiles_p + map[k].ntiles;
   }
   e->total_tiles = tiles;
   for (int par = 0; par < 2; par++)
@@ -1912,7 +1940,7 @@ int build_tables(gmc_ens *e) {
         d.gz_f_out = N[S_GZ_F];
         d.gz_out = N[S_GZ];
         d.tile0 = tile0[k];
-        d.nx = nx[k];
+        d.map = map[k];
       }
   int rc = ehip(e, hipMemcpy(e->d_mem, tab.data(), sizeof(EnsMember) * tab.size(), hipMemcpyHostToDevice), "tables");
   if (rc) return rc;
@@ -2028,6 +2056,7 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
   e->nstage = stage_count(e->scheme);
   e->dt.assign(n, 0.0);
   // filter work items of every member, tagged with the member index
+  constexpr int kEnsWork = 8192;   // tap-outputs of an item, as the stage's own
   std::vector<Item> gz, uv;
   size_t lgz = 0, luv = 0;
   int maxb = 1, maxs = 1;
@@ -2039,11 +2068,21 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
         hipMemcpy(nb_lat.data(), c->big.ngrid_lat, sizeof(int32_t) * g.nhalf, hipMemcpyDeviceToHost) != hipSuccess ||
         hipMemcpy(ns_lon.data(), c->small1.ngrid_lon, sizeof(int32_t) * g.nlat, hipMemcpyDeviceToHost) != hipSuccess)
       return fail(GMC_EDEVICE, "filter tables");
+    // the rows that the tiles do not take through the whole stage
+    StageMap sm;
+    stage_map(g.nlon, g.nlat, nb_lon, ns_lon, nb_lat, StageTile::TY, sm);
+    auto polar = [&](int r) { return r < sm.ra || r >= sm.rb; };
     std::vector<Item> a, b;
     for (int r = 0; r < g.nlat; r++)
-      add_row(a, r, 0, nb_lon[r] + std::max(1, nb_lon[r] / 2), g.nlon, lgz, std::max(nb_lon[r], ns_lon[r]));
-    for (int r = 0; r < g.nlat; r++) add_row(b, r, 1, nb_lon[r], g.nlon, luv, nb_lon[r]);
-    for (int r = 0; r < g.nhalf; r++) add_row(b, r, 2, nb_lat[r], g.nlon, luv, nb_lat[r]);
+      if (polar(r))
+        add_row(a, r, 0, nb_lon[r] + std::max(1, nb_lon[r] / 2), g.nlon, lgz, std::max(nb_lon[r], ns_lon[r]), 0, kEnsWork);
+    for (int r = 0; r < g.nlat; r++)
+      if (polar(r)) add_row(b, r, 1, nb_lon[r], g.nlon, luv, nb_lon[r], 0, kEnsWork);
+    for (int r = 0; r < g.nhalf; r++)
+      if (polar(r)) add_row(b, r, 2, nb_lat[r], g.nlon, luv, nb_lat[r], 0, kEnsWork);
+    e->nb_lon.push_back(nb_lon);
+    e->nb_lat.push_back(nb_lat);
+    e->ns_lon.push_back(ns_lon);
     for (auto &it : a) {
       it.n = nb_lon[it.row];
       it.n2 = ns_lon[it.row];

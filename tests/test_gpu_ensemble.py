@@ -89,3 +89,25 @@ def test_autotune_keeps_state():
         m.step(3)
     _assert_same(ens_m, plain, f"after autotune (shape {choice})")
     ens.close()
+
+
+# members whose rows all go through the filter kernels (narrow or low grids)
+# beside members whose tiles take their short rows whole: the first sizes that
+# do, odd and even zones, wide and hardly any filters, one and several segments
+# of tile widths
+ODD = [(62, 30, 1.0), (64, 23, 1.0), (64, 24, 1.0), (66, 25, 3.0), (108, 61, 1.0), (180, 91, 5.0), (502, 64, 1.0),
+       (560, 65, 4.0), (722, 100, 0.2), (8, 5, 1.0)]
+
+
+@pytest.mark.parametrize("shape", range(0, 9, 4))
+def test_uneven_members_bitwise(shape):
+    specs = [(nlon, nlat, 20000.0 * long / max(nlon, nlat)) for nlon, nlat, long in ODD]
+    ens_m, plain = ([_member(*s, k) for k, s in enumerate(specs)] for _ in range(2))
+    ens = Ensemble(ens_m)
+    ens.set_shape(shape)
+    for n in (1, 8):
+        ens.step(n)
+        for m in plain:
+            m.step(n)
+        _assert_same(ens_m, plain, f"{n} steps, shape {shape}")
+    ens.close()
