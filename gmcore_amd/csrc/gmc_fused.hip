@@ -1237,16 +1237,19 @@ __global__ void __launch_bounds__(StageTile::NT, PHASE == kStageOne ? 4 : 8) k_s
 }
 
 // ---------------------------------------------------------------------------
-// Batched ensembles: the same stage kernels over many contexts in one launch.
-// A member's descriptor for one stage holds its geometry, tables, options,
-// stage dt and field pointers; tiles and filter items of all members are
-// numbered consecutively and each workgroup finds its member by the tile
-// offset (k_tend) or the item's member index (filters).  The rows of short
-// filters go through their tiles whole, as in k_stage, and only the polar rows
-// through the filter kernels: bound by the passes over memory between the
-// kernels and by the number of filter workgroups.  At 16 members (8 of 180 x
-// 91, 6 of 360 x 181, 2 of 720 x 361) a stage's kernels took 38.5, 23.5 and
-// 12.7 us with every row in all three and 49.4, 7.7 and 11.3 us so.
+// Batched ensembles: the launches of a stage over many contexts at once.  A
+// member's descriptor for one stage holds its geometry, tables, options, stage
+// dt and field pointers; a list gives each tile its member (one trip to memory
+// where a search over the members' first tiles took four), and an item holds
+// its member's index.
+//
+// The tendency launch takes the polar rows' tiles; the filter launches, bound
+// by the latency of their widest rows, also take as many of the tiles that do
+// a whole stage as make two workgroups a compute unit, and the tendency launch
+// the rest.  At 16 members (8 of 180 x 91, 6 of 360 x 181, 2 of 720 x 361) a
+// stage's three launches took 38.5 + 23.5 + 12.7 us with every row in all
+// three, 49.4 + 7.7 + 11.3 us with all tiles in the first and 38.0 + 13.5 +
+// 12.6 us so.
 struct EnsMember {
   Grid g;
   Mesh M;
@@ -1258,8 +1261,11 @@ struct EnsMember {
   UVPtrs up;
   double *gz_f_out;    // gz_f of the new state (big filter output)
   double *gz_out;      // gz of the new state (small filter output)
-  int tile0;           // first tile of the member: map.tiles_p of the polar rows, then map.ntiles
-  StageMap map;
+};
+// Tile `tile` of member `member`: map.tiles_p of the polar rows, then
+// map.ntiles that do a whole stage.
+struct EnsTile {
+  int member, tile;
 };
 
 // Field pointers read from a descriptor in memory are generic (FLAT) to the
@@ -1297,71 +1303,71 @@ __device__ __forceinline__ UVPtrsG glb(const UVPtrs &p) {
   return UVPtrsG{glb(p.u_old), glb(p.v_old), glb(p.du), glb(p.dv), glb(p.gz_f), glb(p.u), glb(p.v), glb(p.u_f), glb(p.v_f)};
 }
 
-// The tiles of all members, numbered member by member and row-major within a
-// member, are cut into NXCD contiguous runs, one per XCD (workgroup b runs on
-// XCD b % NXCD), so vertically adjacent tiles share that XCD's L2.  The
-// workgroups of one XCD stride over its run: gridDim.x may be smaller than
+// A tile of an ensemble's member.
+template <class S, bool POLAR>
+__device__ __forceinline__ void ens_tile(const EnsMember *__restrict__ mem, const StageMap *__restrict__ maps,
+                                         EnsTile e, double *sh) {
+  const EnsMember d = mem[e.member];   // private copies: no aliasing with the stores of the tile
+  const StageMap m = maps[e.member];
+  const StagePtrsG sp = glb(d.sp);
+  if (POLAR && e.tile < m.tiles_p) {
+    const TileGeo G = polar_tile<S::TY>(m, d.g, e.tile);
+    const TileIn io = tile_fetch<S>(d.g, sp, G);
+    tile_poles<S>(d.g, glb(d.M), d.grav, d.rgrav, sp, G.r0, sh);
+    tend_tile<S, false, false>(d.g, glb(d.M), (RecPtr)d.mrows, d.grav, d.rgrav, d.dt, d.stokes, d.pv_scheme, d.order,
+                               d.wgt, d.coriolis, sp, G, sh, io, nullptr, NoRest{});
+  } else {
+    const TileGeo G = short_tile<S::TY>(m, d.g.nlon, e.tile - m.tiles_p);
+    const UVPtrsG up = glb(d.up);
+    const TileRest<FilterDevG, gptr<const double>, gptr<double>> rest{
+        glb(d.big), glb(d.small1), up.u_old, up.v_old, up.u, up.v, up.u_f, up.v_f, glb(d.gz_f_out), glb(d.gz_out)};
+    const TileIn io = tile_fetch<S>(d.g, sp, G);
+    tend_tile<S, false, true>(d.g, glb(d.M), (RecPtr)d.mrows, d.grav, d.rgrav, d.dt, d.stokes, d.pv_scheme, d.order,
+                              d.wgt, d.coriolis, sp, G, sh, io, nullptr, rest);
+  }
+}
+
+// The listed tiles are cut into NXCD contiguous runs, one per XCD (workgroup b
+// runs on XCD b % NXCD), so vertically adjacent tiles share that XCD's L2.
+// The workgroups of one XCD stride over its run: gridDim.x may be smaller than
 // the tile count (a persistent launch sized by the tuner).
 template <class S>
-__global__ void __launch_bounds__(S::NT, 8) k_tend_ens(const EnsMember *__restrict__ mem, int nmem, int total) {
+__global__ void __launch_bounds__(S::NT, 8) k_tend_ens(const EnsMember *__restrict__ mem,
+                                                       const StageMap *__restrict__ maps,
+                                                       const EnsTile *__restrict__ tiles, int total) {
   __shared__ double sh[S::SH_ALL];
   const int G = gridDim.x, x = blockIdx.x % NXCD;
-  int start = 0;
-  for (int y = 0; y < x; y++) start += (total - y + NXCD - 1) / NXCD;
-  const int cnt = (total - x + NXCD - 1) / NXCD;    // tiles of this XCD's run
-  const int per = (G - x + NXCD - 1) / NXCD;        // workgroups on this XCD
+  const int q = total / NXCD, rem = total % NXCD;
+  const int start = x * q + min(x, rem), cnt = q + (x < rem);   // this XCD's run
+  const int per = (G - x + NXCD - 1) / NXCD;                    // workgroups on this XCD
   for (int s = blockIdx.x / NXCD; s < cnt; s += per) {
-    const int t = start + s;
-    int lo = 0, hi = nmem - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (mem[mid].tile0 <= t) lo = mid; else hi = mid - 1;
-    }
-    const EnsMember d = mem[lo];   // a private copy: no aliasing with the stores of the tile
-    const int lt = t - d.tile0;
-    const StagePtrsG sp = glb(d.sp);
-    if (lt < d.map.tiles_p) {
-      const TileGeo G = polar_tile<S::TY>(d.map, d.g, lt);
-      const TileIn io = tile_fetch<S>(d.g, sp, G);
-      tile_poles<S>(d.g, glb(d.M), d.grav, d.rgrav, sp, G.r0, sh);
-      tend_tile<S, false, false>(d.g, glb(d.M), (RecPtr)d.mrows, d.grav, d.rgrav, d.dt, d.stokes, d.pv_scheme,
-                                 d.order, d.wgt, d.coriolis, sp, G, sh, io, nullptr, NoRest{});
-    } else {
-      const TileGeo G = short_tile<S::TY>(d.map, d.g.nlon, lt - d.map.tiles_p);
-      const TileRest<FilterDev, const double *, double *> rest{d.big,  d.small1, d.up.u_old, d.up.v_old, d.up.u,
-                                                               d.up.v, d.up.u_f, d.up.v_f,   d.gz_f_out, d.gz_out};
-      const TileIn io = tile_fetch<S>(d.g, sp, G);
-      tend_tile<S, false, true>(d.g, glb(d.M), (RecPtr)d.mrows, d.grav, d.rgrav, d.dt, d.stokes, d.pv_scheme, d.order,
-                                d.wgt, d.coriolis, sp, G, sh, io, nullptr, rest);
-    }
+    ens_tile<S, true>(mem, maps, tiles[start + s], sh);
     __syncthreads();
   }
 }
 
-__global__ void __launch_bounds__(NF) k_gzf_ens(const EnsMember *__restrict__ mem, const Item *__restrict__ items,
-                                                int nitems) {
-  extern __shared__ double xs[];
-  for (int b = blockIdx.x; b < nitems; b += gridDim.x) {
-    const Item it = items[b];
-    const EnsMember d = mem[it.member];
-    gzf_item(d.g, glb(d.big), glb(d.small1), it, glb(d.sp.gz_new), glb(d.gz_f_out), glb(d.gz_out), xs, threadIdx.x);
-    __syncthreads();
+// Workgroups [0, groups): an item per group of NF threads (the list is padded
+// with empty items); then the listed tiles.
+template <bool GZ>
+__global__ void __launch_bounds__(StageTile::NT, 8) k_filter_ens(const EnsMember *__restrict__ mem,
+                                                                 const StageMap *__restrict__ maps,
+                                                                 const EnsTile *__restrict__ tiles, int ntiles,
+                                                                 const Item *__restrict__ items, int groups,
+                                                                 int item_lds) {
+  extern __shared__ __attribute__((aligned(16))) double xs[];
+  const int b = blockIdx.x;
+  if (b >= groups) {
+    ens_tile<StageTile, false>(mem, maps, tiles[xcd_item(b - groups, ntiles)], xs);
+    return;
   }
-}
-
-__global__ void __launch_bounds__(NF) k_uvf_ens(const EnsMember *__restrict__ mem, const Item *__restrict__ items,
-                                                int nitems) {
-  extern __shared__ double xs[];
-  for (int b = blockIdx.x; b < nitems; b += gridDim.x) {
-    const Item it = items[b];
-    const EnsMember *d = mem + it.member;
-    const Grid g = d->g;
-    const MeshG M = glb(d->M);
-    const FilterDevG big = glb(d->big);
-    const UVPtrsG up = glb(d->up);
-    uvf_item(g, M, d->dt, big, it, up, xs, threadIdx.x);
-    __syncthreads();
-  }
+  const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x / NF), tid = threadIdx.x % NF;
+  const Item &it = items[b * kItemsPerWg + grp];
+  const EnsMember *d = mem + it.member;
+  double *x = xs + grp * item_lds;
+  if constexpr (GZ)
+    gzf_item(d->g, glb(d->big), glb(d->small1), it, glb(d->sp.gz_new), glb(d->gz_f_out), glb(d->gz_out), x, tid);
+  else
+    uvf_item(d->g, glb(d->M), d->dt, glb(d->big), it, glb(d->up), x, tid);
 }
 
 }  // namespace
@@ -1527,6 +1533,23 @@ static bool stage_map(int nlon, int nlat, const std::vector<int32_t> &nb, const 
   return true;
 }
 
+// The tap-outputs of a filter item of the launches that also take tiles (four
+// items share a workgroup's LDS), and the workgroups those launches are filled
+// up to with tiles: two on each compute unit.
+static constexpr int kStageWork = 8192, kStageSlots = 2 * 256;
+
+// Heavy and light items share a workgroup: item i of the order by work goes to
+// workgroup i mod the number of workgroups.
+static void deal_items(std::vector<Item> &v) {
+  auto taps = [](const Item &it) { return (int64_t)(it.c1 - it.c0) * std::max(it.n + it.n2, 1); };
+  std::stable_sort(v.begin(), v.end(), [&](const Item &a, const Item &b) { return taps(a) > taps(b); });
+  while (v.size() % kItemsPerWg) v.push_back(Item{1, 0, 0, 1, 0, 0, 0, 0});   // no columns
+  const int n = (int)v.size() / kItemsPerWg;
+  std::vector<Item> dealt(v.size());
+  for (int i = 0; i < (int)v.size(); i++) dealt[i % n * kItemsPerWg + i / n] = v[i];
+  v = dealt;
+}
+
 // The launches of the stage.
 static int build_stage(gmc_ctx *c, FusedPlan *P, const std::vector<int32_t> &nb, const std::vector<int32_t> &ns,
                        const std::vector<int32_t> &nbv) {
@@ -1565,8 +1588,6 @@ static int build_stage(gmc_ctx *c, FusedPlan *P, const std::vector<int32_t> &nb,
     return rc;
   }
   // three launches
-  // filter items of at most kStageWork tap-outputs: four share a workgroup's LDS
-  constexpr int kStageWork = 8192;
   std::vector<Item> items[3];
   size_t lgz = 0, luv = 0;
   for (int r = 0; r < nlat; r++) {
@@ -1576,29 +1597,17 @@ static int build_stage(gmc_ctx *c, FusedPlan *P, const std::vector<int32_t> &nb,
     if (r < nhalf) add_row(items[2], r, 2, nbv[r], nlon, luv, nbv[r], 0, kStageWork);
   }
   for (auto &it : items[1]) { it.n = nb[it.row]; it.n2 = ns[it.row]; }
-  for (int k = 1; k < 3; k++) {
-    // heavy and light items share a workgroup: item i of the order by work
-    // goes to workgroup i mod the number of workgroups
-    std::vector<Item> &v = items[k];
-    auto taps = [](const Item &it) { return (int64_t)(it.c1 - it.c0) * std::max(it.n + it.n2, 1); };
-    std::stable_sort(v.begin(), v.end(), [&](const Item &a, const Item &b) { return taps(a) > taps(b); });
-    while (v.size() % kItemsPerWg) v.push_back(Item{1, 0, 0, 1, 0, 0, 0, 0});   // no columns
-    const int n = (int)v.size() / kItemsPerWg;
-    std::vector<Item> dealt(v.size());
-    for (int i = 0; i < (int)v.size(); i++) dealt[i % n * kItemsPerWg + i / n] = v[i];
-    v = dealt;
-  }
+  for (int k = 1; k < 3; k++) deal_items(items[k]);
   const size_t item[3] = {0, lgz + sizeof(double) * (c->big.max_taps + c->small1.max_taps),
                           luv + sizeof(double) * c->big.max_taps};
   if (kItemsPerWg * std::max(item[1], item[2]) > kLds) return GMC_OK;
   // the short rows' tiles: what fills the second and third launch up to two
   // workgroups a compute unit, the two bands beside the polar rows (first and
   // last in the numbering) in the first
-  constexpr int slots = 2 * 256;
   const int keep = std::min(m.ntiles, m.seg[0].nx + m.seg[m.nseg - 1].nx);
   int left = m.ntiles - keep;
   for (int k = 1; k < 3; k++) {
-    const int polar = (int)items[k].size() / kItemsPerWg, take = std::min(left, std::max(0, slots - polar));
+    const int polar = (int)items[k].size() / kItemsPerWg, take = std::min(left, std::max(0, kStageSlots - polar));
     P->stage[k] = {polar, 0, take, (int)(item[k] / sizeof(double)), nullptr, std::max(kTileLds, kItemsPerWg * item[k])};
     left -= take;
   }
@@ -1866,11 +1875,13 @@ struct gmc_ens {
   std::vector<gmc_ctx *> m;
   int scheme = 0, nstage = 3;
   int shape = 0;
-  gmc::EnsMember *d_mem = nullptr;  // [2 parities][nstage][members]
+  gmc::EnsMember *d_mem = nullptr;  // [2 parities][nstage][members]; then, in the same allocation,
+  gmc::StageMap *d_maps = nullptr;  // [members],
+  gmc::EnsTile *d_tiles = nullptr;  // the tiles of the three launches
   gmc::Item *d_items = nullptr;
-  int n_gz = 0, n_uv = 0;
-  size_t lds_gz = 0, lds_uv = 0;
-  int total_tiles = 0;
+  int n_gz = 0, n_uv = 0;           // workgroups of filter items
+  size_t lds_gz = 0, lds_uv = 0;    // LDS of an item
+  int tiles[3] = {0, 0, 0};
   std::vector<std::vector<int32_t>> nb_lon, nb_lat, ns_lon;   // taps of the members' rows
   std::vector<double> dt;           // dt the tables were built for
   int built_shape = -1;
@@ -1897,20 +1908,45 @@ void drop_graphs(gmc_ens *e) {
     if (*g) { hip_note(hipGraphExecDestroy(*g), "ensemble graph destroy"); *g = nullptr; }
 }
 
+// the members' rows for tiles of height ty; returns the number of their tiles
+int ens_maps(gmc_ens *e, int ty, std::vector<StageMap> &maps) {
+  int tiles = 0;
+  maps.resize(e->m.size());
+  for (size_t k = 0; k < e->m.size(); k++) {
+    const Grid &g = e->m[k]->grid;
+    stage_map(g.nlon, g.nlat, e->nb_lon[k], e->ns_lon[k], e->nb_lat[k], ty, maps[k]);
+    tiles += maps[k].tiles_p + maps[k].ntiles;
+  }
+  return tiles;
+}
+
 // descriptor tables for the current shape and dts
 int build_tables(gmc_ens *e) {
   const int nm = (int)e->m.size(), ty = kEnsShapes[e->shape].ty;
   std::vector<EnsMember> tab((size_t)2 * e->nstage * nm);
-  int tiles = 0;
-  std::vector<int> tile0(nm);
-  std::vector<StageMap> map(nm);
+  std::vector<StageMap> maps;
+  ens_maps(e, ty, maps);
+  // The tiles of each launch, member by member.  The filter launches take tiles
+  // of their own workgroups' height only, and none of the two bands beside the
+  // polar rows, whose gz_f the last launch's polar rows read.
+  std::vector<EnsTile> tiles[3];
+  const int room[2] = {std::max(0, kStageSlots - e->n_gz), std::max(0, kStageSlots - e->n_uv)};
   for (int k = 0; k < nm; k++) {
-    const Grid &g = e->m[k]->grid;
-    stage_map(g.nlon, g.nlat, e->nb_lon[k], e->ns_lon[k], e->nb_lat[k], ty, map[k]);
-    tile0[k] = tiles;
-    tiles += map[k].tiles_p + map[k].ntiles;
+    const StageMap &m = maps[k];
+    const int first = m.nseg ? m.seg[0].nx : 0, last = m.nseg ? m.ntiles - m.seg[m.nseg - 1].nx : 0;
+    for (int t = 0; t < m.tiles_p + m.ntiles; t++) {
+      const int s = t - m.tiles_p;
+      int l = 0;
+      if (ty == StageTile::TY && s >= first && s < last)
+        l = (int)tiles[1].size() < room[0] ? 1 : (int)tiles[2].size() < room[1] ? 2 : 0;
+      tiles[l].push_back(EnsTile{k, t});
+    }
   }
-  e->total_tiles = tiles;
+  std::vector<EnsTile> list;
+  for (int l = 0; l < 3; l++) {
+    e->tiles[l] = (int)tiles[l].size();
+    list.insert(list.end(), tiles[l].begin(), tiles[l].end());
+  }
   for (int par = 0; par < 2; par++)
     for (int st = 0; st < e->nstage; st++)
       for (int k = 0; k < nm; k++) {
@@ -1939,10 +1975,13 @@ int build_tables(gmc_ens *e) {
         d.up = UVPtrs{O[S_U_LON], O[S_V_LAT], du, dv, N[S_GZ_F], N[S_U_LON], N[S_V_LAT], N[S_U_F], N[S_V_F]};
         d.gz_f_out = N[S_GZ_F];
         d.gz_out = N[S_GZ];
-        d.tile0 = tile0[k];
-        d.map = map[k];
       }
-  int rc = ehip(e, hipMemcpy(e->d_mem, tab.data(), sizeof(EnsMember) * tab.size(), hipMemcpyHostToDevice), "tables");
+  std::vector<char> all;
+  auto put = [&](const void *x, size_t n) { all.insert(all.end(), (const char *)x, (const char *)x + n); };
+  put(tab.data(), sizeof(EnsMember) * tab.size());
+  put(maps.data(), sizeof(StageMap) * maps.size());
+  put(list.data(), sizeof(EnsTile) * list.size());
+  int rc = ehip(e, hipMemcpy(e->d_mem, all.data(), all.size(), hipMemcpyHostToDevice), "tables");
   if (rc) return rc;
   drop_graphs(e);
   e->built_shape = e->shape;
@@ -1952,7 +1991,7 @@ int build_tables(gmc_ens *e) {
 template <int TY>
 void launch_tend(gmc_ens *e, const EnsMember *mem, int grid) {
   using S = Tile<TY>;
-  hipLaunchKernelGGL(k_tend_ens<S>, dim3(grid), dim3(S::NT), 0, e->stream, mem, (int)e->m.size(), e->total_tiles);
+  hipLaunchKernelGGL(k_tend_ens<S>, dim3(grid), dim3(S::NT), 0, e->stream, mem, e->d_maps, e->d_tiles, e->tiles[0]);
 }
 
 // the launches of one ensemble step for parity par (0: old 1 -> new 2)
@@ -1960,7 +1999,11 @@ void ens_launch_step(gmc_ens *e, int par) {
   const int nm = (int)e->m.size();
   const EnsShape &sh = kEnsShapes[e->shape];
   // k_tend_ens covers every tile when grid == total or grid >= NXCD
-  const int grid = sh.mult ? std::min(e->total_tiles, sh.mult * 256) : e->total_tiles;
+  const int grid = sh.mult ? std::min(e->tiles[0], sh.mult * 256) : e->tiles[0];
+  const EnsTile *t1 = e->d_tiles + e->tiles[0], *t2 = t1 + e->tiles[1];
+  auto lds = [](size_t item, int tiles) {
+    return (uint32_t)std::max(kItemsPerWg * item, tiles ? sizeof(double) * StageTile::SH_ALL : 0);
+  };
   for (int st = 0; st < e->nstage; st++) {
     const EnsMember *mem = e->d_mem + ((size_t)par * e->nstage + st) * nm;
     switch (sh.ty) {
@@ -1968,8 +2011,12 @@ void ens_launch_step(gmc_ens *e, int par) {
     case 7: launch_tend<7>(e, mem, grid); break;
     default: launch_tend<11>(e, mem, grid);
     }
-    hipLaunchKernelGGL(k_gzf_ens, dim3(e->n_gz), dim3(NF), e->lds_gz, e->stream, mem, e->d_items, e->n_gz);
-    hipLaunchKernelGGL(k_uvf_ens, dim3(e->n_uv), dim3(NF), e->lds_uv, e->stream, mem, e->d_items + e->n_gz, e->n_uv);
+    hipLaunchKernelGGL(k_filter_ens<true>, dim3(e->n_gz + e->tiles[1]), dim3(StageTile::NT),
+                       lds(e->lds_gz, e->tiles[1]), e->stream, mem, e->d_maps, t1, e->tiles[1], e->d_items, e->n_gz,
+                       (int)(e->lds_gz / sizeof(double)));
+    hipLaunchKernelGGL(k_filter_ens<false>, dim3(e->n_uv + e->tiles[2]), dim3(StageTile::NT),
+                       lds(e->lds_uv, e->tiles[2]), e->stream, mem, e->d_maps, t2, e->tiles[2],
+                       e->d_items + kItemsPerWg * e->n_gz, e->n_uv, (int)(e->lds_uv / sizeof(double)));
   }
 }
 
@@ -2056,7 +2103,6 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
   e->nstage = stage_count(e->scheme);
   e->dt.assign(n, 0.0);
   // filter work items of every member, tagged with the member index
-  constexpr int kEnsWork = 8192;   // tap-outputs of an item, as the stage's own
   std::vector<Item> gz, uv;
   size_t lgz = 0, luv = 0;
   int maxb = 1, maxs = 1;
@@ -2075,11 +2121,11 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
     std::vector<Item> a, b;
     for (int r = 0; r < g.nlat; r++)
       if (polar(r))
-        add_row(a, r, 0, nb_lon[r] + std::max(1, nb_lon[r] / 2), g.nlon, lgz, std::max(nb_lon[r], ns_lon[r]), 0, kEnsWork);
+        add_row(a, r, 0, nb_lon[r] + std::max(1, nb_lon[r] / 2), g.nlon, lgz, std::max(nb_lon[r], ns_lon[r]), 0, kStageWork);
     for (int r = 0; r < g.nlat; r++)
-      if (polar(r)) add_row(b, r, 1, nb_lon[r], g.nlon, luv, nb_lon[r], 0, kEnsWork);
+      if (polar(r)) add_row(b, r, 1, nb_lon[r], g.nlon, luv, nb_lon[r], 0, kStageWork);
     for (int r = 0; r < g.nhalf; r++)
-      if (polar(r)) add_row(b, r, 2, nb_lat[r], g.nlon, luv, nb_lat[r], 0, kEnsWork);
+      if (polar(r)) add_row(b, r, 2, nb_lat[r], g.nlon, luv, nb_lat[r], 0, kStageWork);
     e->nb_lon.push_back(nb_lon);
     e->nb_lat.push_back(nb_lat);
     e->ns_lon.push_back(ns_lon);
@@ -2096,20 +2142,32 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
     maxb = std::max(maxb, c->big.max_taps);
     maxs = std::max(maxs, c->small1.max_taps);
   }
-  e->n_gz = (int)gz.size();
-  e->n_uv = (int)uv.size();
+  deal_items(gz);
+  deal_items(uv);
+  e->n_gz = (int)gz.size() / kItemsPerWg;
+  e->n_uv = (int)uv.size() / kItemsPerWg;
   e->lds_gz = lgz + sizeof(double) * (maxb + maxs);
   e->lds_uv = luv + sizeof(double) * maxb;
+  int most = 0;
+  for (const EnsShape &sh : kEnsShapes) {
+    std::vector<StageMap> maps;
+    most = std::max(most, ens_maps(e, sh.ty, maps));
+  }
   gz.insert(gz.end(), uv.begin(), uv.end());
   int rc = ehip(e, hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking), "stream");
   if (!rc) rc = ehip(e, hipMalloc((void **)&e->d_items, sizeof(Item) * gz.size()), "items");
   if (!rc) rc = ehip(e, hipMemcpy(e->d_items, gz.data(), sizeof(Item) * gz.size(), hipMemcpyHostToDevice), "items");
-  if (!rc) rc = ehip(e, hipMalloc((void **)&e->d_mem, sizeof(EnsMember) * 2 * e->nstage * n), "tables");
-  if (!rc && e->lds_gz > 65536)
-    rc = ehip(e, hipFuncSetAttribute((const void *)k_gzf_ens, hipFuncAttributeMaxDynamicSharedMemorySize, (int)e->lds_gz), "lds");
-  if (!rc && e->lds_uv > 65536)
-    rc = ehip(e, hipFuncSetAttribute((const void *)k_uvf_ens, hipFuncAttributeMaxDynamicSharedMemorySize, (int)e->lds_uv), "lds");
-  if (!rc && std::max(e->lds_gz, e->lds_uv) > 160 * 1024) rc = eerr(e, GMC_EINVAL, "filter window exceeds LDS");
+  if (!rc)
+    rc = ehip(e, hipMalloc((void **)&e->d_mem, (sizeof(EnsMember) * 2 * e->nstage + sizeof(StageMap)) * n +
+                                                   sizeof(EnsTile) * most), "tables");
+  e->d_maps = (StageMap *)(e->d_mem + (size_t)2 * e->nstage * n);
+  e->d_tiles = (EnsTile *)(e->d_maps + n);
+  // an item's window and taps are at most about three circles of the widest
+  // member's (k_tend's limit): four of them fit
+  constexpr size_t kLds = 160 * 1024;
+  if (!rc && kItemsPerWg * std::max(e->lds_gz, e->lds_uv) > kLds) rc = eerr(e, GMC_EINVAL, "filter window exceeds LDS");
+  for (const void *f : {(const void *)k_filter_ens<true>, (const void *)k_filter_ens<false>})
+    if (!rc) rc = ehip(e, hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds), "lds");
   if (rc) {
     gmc_ens_destroy(e);
     return rc;

@@ -111,3 +111,17 @@ def test_uneven_members_bitwise(shape):
             m.step(n)
         _assert_same(ens_m, plain, f"{n} steps, shape {shape}")
     ens.close()
+
+
+@pytest.mark.parametrize("shape", [0, 1])
+def test_tiles_of_every_launch_bitwise(shape):
+    # more tiles than the filter launches have room for
+    specs = [(180, 91, 600.0), (1440, 721, 60.0), (360, 181, 300.0)]
+    ens_m, plain = ([_member(*s, k) for k, s in enumerate(specs)] for _ in range(2))
+    ens = Ensemble(ens_m)
+    ens.set_shape(shape)
+    ens.step(2)
+    for m in plain:
+        m.step(2)
+    _assert_same(ens_m, plain, f"shape {shape}")
+    ens.close()
