@@ -36,8 +36,10 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
 BYTES_PER_GP_STEP = 280.0          # 35 FP64 field passes per pc2 step
-# compulsory bytes per grid point of one launch of each kernel class, mean
-# over the three stages (k_tend reads 4 fields in stage 1 and 5 in stages
+# compulsory bytes per grid point of one launch of each kernel class of the
+# three-kernel stage (which gmc_kernel_times runs on every grid; gmc_step at
+# 1440 x 721 spreads a stage over k_stage's three launches), mean over the
+# three stages (k_tend reads 4 fields in stage 1 and 5 in stages
 # 2-3 and writes 3; k_gzf reads 1, writes 2; k_uvf reads 5, writes 4)
 KERNEL_BYTES_PER_GP = {"k_tend": 8.0 * (7 + 8 + 8) / 3, "k_gzf": 24.0, "k_uvf": 72.0}
 PROFILES = os.path.join(ROOT, "profiles")

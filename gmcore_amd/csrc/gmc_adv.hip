@@ -14,11 +14,13 @@
 //                 (adv_mod.F90:183-235) into qp
 //   k_adv_fix     per (row, tracer): the positivity fixer and the longitude
 //                 damping of the row (adv_mod.F90:236-301), qp -> new level
-// The flux kernels read every stencil from global memory (L2): one lane per
-// cell, no LDS and no barrier, so many wavefronts hide the latency of the
-// data-dependent loads (the upwind cells).  The pole rows, whose y-flux is a
-// zonal sum, are one workgroup each.  Only the fixer and the damping, which
-// walk a row, keep the row in LDS.
+// The flux kernels read every stencil from global memory (L2), one lane per
+// cell, so many wavefronts hide the latency of the data-dependent loads (the
+// upwind cells); only the y-fluxes pass through LDS, to the two cells either
+// side.  An item is a block of cells for a group of tracers, for which what
+// depends on the wind alone is formed once.  The pole rows, whose y-flux is a
+// zonal sum, are one workgroup each.  The fixer and the damping, which walk a
+// row, keep the row in LDS.
 //
 // Layout in HBM: dense row-major [rows][pitch] doubles per field, no halo;
 // tracer l of level k at q + ((k-1) * ntracers + l) * nlat * pitch.
