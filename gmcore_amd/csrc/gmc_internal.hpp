@@ -129,6 +129,19 @@ __device__ __forceinline__ int xcd_item(int b, int total) {
   return x * q + (x < m ? x : m) + s;
 }
 
+// x / d and x % d of 0 <= x < 2^31, d >= 1 without a division, mul =
+// div_mul(d) = floor((2^32 - 1) / d): x mul / 2^32 is below x / d by at most
+// x / 2^32 < 1, so its integer part is the quotient or one less.
+inline uint32_t div_mul(int d) { return 0xffffffffu / (uint32_t)d; }
+__host__ __device__ __forceinline__ void div_mod(int x, int d, uint32_t mul, int &q, int &r) {
+  q = (int)(((uint64_t)(uint32_t)x * mul) >> 32);
+  r = x - q * d;
+  if (r >= d) {
+    q++;
+    r -= d;
+  }
+}
+
 // Column i+d, periodic.
 __device__ __forceinline__ int wrap(int i, int n) {
   return i < 0 ? i + n : (i >= n ? i - n : i);

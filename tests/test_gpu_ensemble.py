@@ -113,6 +113,24 @@ def test_uneven_members_bitwise(shape):
     ens.close()
 
 
+# members of one tile across (at most 60 columns) and several tiles high at
+# every tile height, beside one two tiles across
+NARROW = [(8, 30), (16, 40), (58, 30), (60, 31), (60, 12), (62, 30)]
+
+
+@pytest.mark.parametrize("shape", range(9))
+def test_narrow_members_bitwise(shape):
+    specs = [(nlon, nlat, 20000.0 / max(nlon, nlat)) for nlon, nlat in NARROW]
+    ens_m, plain = ([_member(*s, k) for k, s in enumerate(specs)] for _ in range(2))
+    ens = Ensemble(ens_m)
+    ens.set_shape(shape)
+    ens.step(3)
+    for m in plain:
+        m.step(3)
+    _assert_same(ens_m, plain, f"shape {shape}")
+    ens.close()
+
+
 @pytest.mark.parametrize("shape", [0, 1])
 def test_tiles_of_every_launch_bitwise(shape):
     # more tiles than the filter launches have room for
