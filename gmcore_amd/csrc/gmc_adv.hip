@@ -1359,10 +1359,10 @@ __global__ void __launch_bounds__(NA) k_adv_psum2(AdvGrid g, const double *f, in
 // LDS, shared by the cells either side) and the x-flux tangents of one cell
 // row, the west face's from the lane below; a pole row's item sums the
 // tangents of its V row's fluxes itself
-__global__ void __launch_bounds__(NF) t_adv_inner(AdvGrid g, Mesh M, int lim, int ntr, TBase b, TWork w) {
+__global__ void __launch_bounds__(NF) t_adv_inner(AdvGrid g, Mesh M, int lim, FluxMap map, TBase b, TWork w) {
   __shared__ double sfy[NF / kWave][kWave];
   __shared__ double bcast;
-  const FluxItem it = flux_item(g, FluxMap(g, ntr, 1));
+  const FluxItem it = flux_item(g, map);
   const int n = g.nlon;
   const int64_t to = it.t * w.ts, P = g.pitch;
   const double *q = b.q + to, *d = w.in + to;
@@ -1406,10 +1406,10 @@ __global__ void __launch_bounds__(NF) t_adv_inner(AdvGrid g, Mesh M, int lim, in
 
 // tangent of the outer fluxes and the update (adv_mod.F90:183-235) into
 // dqp, on the work items of k_adv_flux
-__global__ void __launch_bounds__(NF) t_adv_outer(AdvGrid g, Mesh M, int lim, int ntr, TBase b, TWork w) {
+__global__ void __launch_bounds__(NF) t_adv_outer(AdvGrid g, Mesh M, int lim, FluxMap map, TBase b, TWork w) {
   __shared__ double sfy[NF / kWave][kWave];
   __shared__ double bcast;
-  const FluxItem it = flux_item(g, FluxMap(g, ntr, 1));
+  const FluxItem it = flux_item(g, map);
   const int n = g.nlon;
   const int64_t to = it.t * w.ts, P = g.pitch;
   const double *qx = b.qx + to, *qy = b.qy + to, *dqx = w.dqx + to, *dqy = w.dqy + to, *d = w.in + to;
@@ -1762,9 +1762,10 @@ void tl_step(gmc_adv *a, const char *slot, int old, const double *in, double *ou
   const size_t F = tl_fields(a);
   double *dqx = a->tl_f + 2 * F, *dqy = a->tl_f + 3 * F, *dqp = a->tl_f + 4 * F, *ps = a->tl_f + 5 * F;
   const TBase b = tape_base(a, slot, old);
-  const dim3 items(FluxMap(g, ntr, 1).blocks());
-  hipLaunchKernelGGL(t_adv_inner, items, dim3(NF), 0, a->stream, g, M, lim, ntr, b, TWork{in, dqx, dqy, dqp, out, ps, ts});
-  hipLaunchKernelGGL(t_adv_outer, items, dim3(NF), 0, a->stream, g, M, lim, ntr, b, TWork{in, dqx, dqy, dqp, out, ps, ts});
+  const FluxMap map(g, ntr, 1);
+  const dim3 items(map.blocks());
+  hipLaunchKernelGGL(t_adv_inner, items, dim3(NF), 0, a->stream, g, M, lim, map, b, TWork{in, dqx, dqy, dqp, out, ps, ts});
+  hipLaunchKernelGGL(t_adv_outer, items, dim3(NF), 0, a->stream, g, M, lim, map, b, TWork{in, dqx, dqy, dqp, out, ps, ts});
   hipLaunchKernelGGL(t_adv_fix, dim3(g.nlat, ntr), dim3(NA), 4 * (size_t)g.nlon * sizeof(double), a->stream, g, b,
                      TWork{in, dqx, dqy, dqp, out, ps, ts}, a->d_wgt, a->cfg.lon_damp_passes);
 }
