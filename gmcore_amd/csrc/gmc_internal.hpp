@@ -124,7 +124,7 @@ struct Grid {
 // kNumXcd, m = total % kNumXcd, in order.  Items that share rows then share
 // an L2.
 constexpr int kNumXcd = 8;
-__device__ __forceinline__ int xcd_item(int b, int total) {
+__host__ __device__ __forceinline__ int xcd_item(int b, int total) {
   const int x = b % kNumXcd, s = b / kNumXcd, q = total / kNumXcd, m = total % kNumXcd;
   return x * q + (x < m ? x : m) + s;
 }

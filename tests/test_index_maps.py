@@ -12,7 +12,7 @@ HIPCC = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "bin", "hipcc")
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not found")
-@pytest.mark.parametrize("name", ["stage_map"])
+@pytest.mark.parametrize("name", ["stage_map", "flux_items"])
 def test_every_point_has_one_owner(name, tmp_path):
     exe = tmp_path / name
     subprocess.run([HIPCC, "-x", "hip", "--offload-host-only", "-O1", "-std=c++17",
