@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/gmcore_hip.h"
+#include "gmc_arith.hpp"
 
 namespace gmc {
 
@@ -33,45 +34,6 @@ enum TendField {
   T_DU, T_DV, T_DGZ, T_QHU, T_QHV, T_DKEDLON, T_DKEDLAT, T_DMFDLON, T_DMFDLAT,
   T_PGF_LON, T_PGF_LAT, T_NFIELDS
 };
-
-// a / d correctly rounded, from y = 1 / d correctly rounded: q0 = a y, the
-// exact remainder e = a - d q0 (one fma), q = q0 + e y rounded once
-// (Markstein's correction step, P. W. Markstein, IBM J. Res. Dev. 34 (1990)
-// 111-119).  Gives the value of the IEEE quotient for normal a, d and a / d
-// (a zero numerator gives +0).  Three FP64 operations instead of the scale /
-// reciprocal / Newton / fixup sequence of a division, for denominators shared
-// by a wavefront (metric terms of one row).
-__device__ __forceinline__ double div_rn(double a, double d, double y) {
-  const double q0 = a * y;
-  return __builtin_fma(__builtin_fma(-q0, d, a), y, q0);
-}
-
-// a / d correctly rounded for a, d and a / d well inside the normal range
-// (layer depths, wind speeds and their ratios): the hardware's reciprocal
-// estimate, two Newton steps and Markstein's correction, 8 instructions.  The
-// compiler's division adds the scaling and fixup of subnormal and overflowing
-// operands, 11.
-__device__ __forceinline__ double div_mid(double a, double d) {
-  double y = __builtin_amdgcn_rcp(d);
-  y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
-  y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
-  return div_rn(a, d, y);
-}
-
-// sqrt(x) correctly rounded for x = 0 and x >= 1e-290: the hardware's
-// reciprocal square root estimate and the coupled Newton iteration of
-// (sqrt, 1 / 2 sqrt) with two corrections of the root, without the
-// compiler's scaling of subnormal operands and its zero / infinity select.
-// Smaller x gives a root below 1e-140, of no account where it is added to kEps.
-__device__ __forceinline__ double sqrt_mid(double x) {
-  const double y = __builtin_amdgcn_rsq(__builtin_fmax(x, 1e-290));
-  double g = x * y, h = 0.5 * y;
-  const double r = __builtin_fma(-h, g, 0.5);
-  g = __builtin_fma(g, r, g);
-  h = __builtin_fma(h, r, h);
-  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
-  return __builtin_fma(__builtin_fma(-g, g, x), h, g);
-}
 
 // Metric fields whose reciprocals the row records also hold (slot order).
 constexpr int kRecipFields[] = {GMC_AREA_VTX, GMC_AREA_CELL, GMC_DE_LON, GMC_DE_LAT};

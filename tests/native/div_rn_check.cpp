@@ -1,7 +1,10 @@
-/* Exhaustive-by-sampling check of the reciprocal division used by the fused
- * stage kernels (div_rn in gmcore_amd/csrc/gmc_internal.hpp):
- *     q0 = a * y,  e = fma(-q0, d, a),  q = e == 0 ? q0 : fma(e, y, q0)
- * with y = 1 / d correctly rounded must equal the IEEE quotient a / d.
+/* Exhaustive-by-sampling check of the kernels' divisions and square roots
+ * (gmcore_amd/csrc/gmc_arith.hpp, the code itself):
+ *   div_rn     from y = 1 / d correctly rounded must equal the IEEE quotient
+ *              (a zero numerator gives a zero; -0 / d may be +0);
+ *   div_from   the same from an estimate of 1 / d up to 2^-22 off;
+ *   sqrt_from  the IEEE square root for 0 and x >= 1e-290 from an estimate of
+ *              1 / sqrt(x) up to 2^-22 off.
  *
  * usage: div_rn_check DENOMS_FILE SAMPLES_PER_DENOM SEED
  * DENOMS_FILE holds raw doubles (the divisor metric terms of real meshes);
@@ -10,12 +13,20 @@
  * doubles over 200 binades and, for the hard cases of rounding, a = RN(d m)
  * and its four nearest neighbours for random rounding midpoints m (d m is
  * exact in binary128), so that a / d lies within a few ulps of 2^-53 of a
- * midpoint.  Prints "checked N mismatches M" and exits 1 on a mismatch. */
+ * midpoint; square roots are taken of random doubles over 1800 binades and of
+ * the doubles around the squares of doubles and of midpoints.  Prints
+ * "checked N mismatches M" and exits 1 on a mismatch. */
 #include <math.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+
+#include "../../gmcore_amd/csrc/gmc_arith.hpp"
+
+using gmc::div_from;
+using gmc::div_rn;
+using gmc::sqrt_from;
 
 static uint64_t st;
 static uint64_t rnd(void) {
@@ -37,20 +48,26 @@ static uint64_t bits(double x) {
 static double rdbl(int e0, int span) {
   return from_bits((rnd() & 0x000fffffffffffffull) | ((uint64_t)(1023 + e0 + (int)(rnd() % (uint64_t)span)) << 52));
 }
-static double div_rn(double a, double d, double y) {
-  const double q0 = a * y;
-  const double e = fma(-q0, d, a);
-  return e == 0.0 ? q0 : fma(e, y, q0);
-}
-
 static long checked, bad;
-static void check(double a, double d, double y) {
-  const double want = a / d, got = div_rn(a, d, y);
+static void expect(const char *what, double a, double d, double want, double got) {
   checked++;
-  if (bits(want) != bits(got)) {
-    if (bad < 5) printf("mismatch a=%a d=%a want=%a got=%a\n", a, d, want, got);
+  if (bits(want) != bits(got) && !(want == 0.0 && got == 0.0)) {
+    if (bad < 5) printf("%s mismatch a=%a d=%a want=%a got=%a\n", what, a, d, want, got);
     bad++;
   }
+}
+/* an estimate of x as the hardware may give it */
+static double rough(double x) {
+  const double err = ldexp((double)(rnd() % 2001) / 1000.0 - 1.0, -22);
+  return x * (1.0 + err);
+}
+static void check(double a, double d, double y) {
+  const double want = a / d;
+  expect("div_rn", a, d, want, div_rn(a, d, y));
+  expect("div_from", a, d, want, div_from(a, d, rough(y)));
+}
+static void check_sqrt(double x) {
+  expect("sqrt_from", x, 0.0, sqrt(x), sqrt_from(x, rough(1.0 / sqrt(fmax(x, 1e-290)))));
 }
 
 static void one_divisor(double d, long n) {
@@ -86,6 +103,21 @@ int main(int argc, char **argv) {
     one_divisor(ldexp(1.0 + ldexp(1.0, -52), e), n);
     one_divisor(-ldexp(1.5, e), n);
     nd += 4;
+  }
+  check_sqrt(0.0);
+  for (long k = 0; k < 500 * n; k++) {
+    check_sqrt(rdbl(-960, 1900));
+    const double g = rdbl(-450, 900);
+    const __float128 m = (__float128)g + ((__float128)nextafter(g, INFINITY) - (__float128)g) / 2;
+    const double x0 = g * g, x1 = (double)(m * m);
+    for (int off = -2; off <= 2; off++) {
+      check_sqrt(from_bits(bits(x0) + (int64_t)off));
+      check_sqrt(from_bits(bits(x1) + (int64_t)off));
+    }
+    const double tiny = rdbl(-1022, 57);   /* below 1e-290 */
+    const double r = sqrt_from(tiny, rough(1.0 / sqrt(fmax(tiny, 1e-290))));
+    checked++;
+    if (tiny < 1e-290 && !(fabs(r) < 1e-140)) bad++;
   }
   printf("divisors %ld checked %ld mismatches %ld\n", nd, checked, bad);
   return bad != 0;
