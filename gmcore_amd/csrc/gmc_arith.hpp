@@ -31,10 +31,13 @@ __host__ __device__ __forceinline__ double div_from(double a, double d, double y
   y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
   return div_rn(a, d, y);
 }
-// ... from the hardware's estimate (2^29 units): 8 instructions, the compiler's
-// division of such operands without the scaling that leaves them as they are
-// and the fixup of exceptional ones, 11.
-__device__ __forceinline__ double div_mid(double a, double d) { return div_from(a, d, __builtin_amdgcn_rcp(d)); }
+// ... from the hardware's estimate (2^29 units), and the fixup of zero, infinite
+// and NaN operands (vanishing or overflowing depths and winds): 9 instructions.
+// The compiler's division adds the scaling, which leaves such operands as they
+// are, 11.
+__device__ __forceinline__ double div_mid(double a, double d) {
+  return __builtin_amdgcn_div_fixup(div_from(a, d, __builtin_amdgcn_rcp(d)), d, a);
+}
 
 // sqrt(x) correctly rounded for x = 0 and finite x >= 1e-290, from an estimate
 // y of 1 / sqrt(max(x, 1e-290)) within 2^-22: the coupled Newton iteration of
@@ -48,9 +51,13 @@ __host__ __device__ __forceinline__ double sqrt_from(double x, double y) {
   g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
   return __builtin_fma(__builtin_fma(-g, g, x), h, g);
 }
-// ... without the compiler's scaling of subnormal operands
-__device__ __forceinline__ double sqrt_mid(double x) {
-  return sqrt_from(x, __builtin_amdgcn_rsq(__builtin_fmax(x, 1e-290)));
+// a / (sqrt(x) + eps) of 0 <= a <= sqrt(x), eps^2 far above 1e-290: without the
+// compiler's scaling of subnormal operands, and with one fixup for root and
+// quotient, in which x stands for its root (an infinite x gives 0 or, with an
+// infinite a, NaN; an a below 2^-1075 x gives 0)
+__device__ __forceinline__ double div_root(double a, double x, double eps) {
+  const double xm = __builtin_fmax(x, 1e-290), d = sqrt_from(x, __builtin_amdgcn_rsq(xm)) + eps;
+  return __builtin_amdgcn_div_fixup(div_from(a, d, __builtin_amdgcn_rcp(d)), xm, a);
 }
 
 }  // namespace gmc

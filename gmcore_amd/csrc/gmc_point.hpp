@@ -67,7 +67,7 @@ __device__ __forceinline__ double pv_of(double vor, const MT &M, int r, double m
 __device__ __forceinline__ double pv_upwind_edge(int order, double wgt, double t, double n,
                                                  int lat_edge, double f1, double f2, double f3,
                                                  double f4) {
-  const double b = div_mid(fabs(t), sqrt_mid(lat_edge ? t * t + n * n : n * n + t * t) + kEps);
+  const double b = div_root(fabs(t), lat_edge ? t * t + n * n : n * n + t * t, kEps);
   const double dir = copysign(1.0, t);
   const double up = order == 1 ? upwind1(dir, wgt, f2, f3) : upwind3(dir, wgt, f1, f2, f3, f4);
   return b * up + (1 - b) * 0.5 * (f2 + f3);

@@ -28,6 +28,28 @@ def test_prepare_matches():
         assert rel_err(g.download(1, f), o.get(1, f)) <= TOL, f
 
 
+@pytest.mark.parametrize("depth", [0.0, np.inf])
+@pytest.mark.parametrize("nlon,nlat", [(180, 91), (60, 31)])
+def test_pv_of_exceptional_depths(nlon, nlat, depth):
+    # vorticity over no depth is an infinity of its sign, over an infinite one 0
+    st = Setup(namelist(nlon, nlat))
+    ic = list(seeded_ic(st, lmax=8))
+    ic[2] = ic[2].copy()
+    rows = slice(nlat // 2 - 3, nlat // 2 + 4)
+    ic[2][rows, 10:16] = ic[3][rows, 10:16] + depth
+    o, g = make_oracle(st, ic), make_gpu(st, ic)
+    o.prepare(1)
+    g.prepare(1)
+    want, got = o.get(1, "pv"), g.download(1, "pv")
+    assert np.isfinite(want).all() != (depth == 0.0)
+    with np.errstate(invalid="ignore"):
+        np.testing.assert_allclose(got, want, rtol=1e-12, atol=1e-12 * np.abs(want[np.isfinite(want)]).max())
+    if depth == 0.0:    # the fused stage's pv of the same state
+        g.keep_derived()
+        g.step(1)
+        np.testing.assert_array_equal(g.download(1, "pv"), got)
+
+
 @pytest.mark.parametrize("pass_,pv", [(0, "upwind"), (1, "upwind"), (1, "tvd")])
 def test_forward_pass(pass_, pv):
     st, o, g = _pair(namelist(pv_scheme=pv))
