@@ -193,6 +193,21 @@ struct InnerPtrs {
 // (154 x 79 x 3 tracers, van Leer: 4.5 us a kernel against 5.6 grouped).
 int flux_group(const AdvGrid &g, int ntr) { return FluxMap(g, ntr, 1).blocks() <= 4 * 256 ? 1 : kGroup; }
 
+// A group's quotients come from reciprocals (div_rn), which is no quotient where
+// the reciprocal overflows (a subnormal Courant number, no mass) or a numerator
+// is infinite: it is a NaN then, and so is what the cells either side make of it.
+// A wavefront that finds its cells' sum over the tracers not finite forms them
+// anew by divisions, fluxes included, as the items of one tracer do.  The sum is
+// one or two additions a cell and tracer (720 x 361 x 8 tracers: 79.2 -> 80.0 us
+// a step; a test of each value took 81.1).
+__device__ __forceinline__ bool any_not_finite(double x) { return __builtin_expect(__any(!__builtin_isfinite(x)), 0); }
+// The lane's column for that second loop, newly known in each round: addresses
+// kept ahead of the loop took the kernel from 85 to 126 registers, 83 us a step.
+__device__ __forceinline__ int own_column(int i) {
+  asm volatile("" : "+v"(i));
+  return i;
+}
+
 // The y-fluxes of a group's V row h through column i into f[t][i's lane].
 template <bool VL, int LIM>
 __device__ __forceinline__ void group_yflux(const AdvGrid &g, int nt, double c, double v, int h, int i,
@@ -299,16 +314,37 @@ __global__ void __launch_bounds__(NF, GROUPED ? 4 : 8) k_adv_inner(AdvGrid g, Me
   const double lel = M(GMC_LE_LON, r), ac = M(GMC_AREA_CELL, r), rac = 1.0 / ac;
   const double ls = M(GMC_LE_LAT, r - 1), ln = M(GMC_LE_LAT, r);
   const XFace face = x_face<VL>(g, cx, ux, iw);
+  double sum = 0.0;
   for (int t = 0; t < it.nt; t++) {
     const double *qt = q + t * p.tstride + ro;
     const double qc = ldu(qt, uiw);
     const double fx = x_flux<VL>(g, lim, face, qt);
     const double fxw = __shfl_up(fx, 1, kWave);
     const double fs = sfy[t][threadIdx.x], fn = sfy[t][threadIdx.x + kWave];
+    const double qx = qc - 0.5 * (div_rn((fx - fxw) * lel, ac, rac) - dvx * qc) * dt;
+    const double qy = qc - 0.5 * (div_rn(fn * ln - fs * ls, ac, rac) - dvy * qc) * dt;
+    sum += qx + qy;
     if (upd) {
       const int64_t o = toff + t * p.tstride + ro;
-      stu(p.qx + o, uiw, qc - 0.5 * (div_rn((fx - fxw) * lel, ac, rac) - dvx * qc) * dt);
-      stu(p.qy + o, uiw, qc - 0.5 * (div_rn(fn * ln - fs * ls, ac, rac) - dvy * qc) * dt);
+      stu(p.qx + o, uiw, qx);
+      stu(p.qy + o, uiw, qy);
+    }
+  }
+  if (any_not_finite(sum)) {
+#pragma unroll 1
+    for (int t = 0; t < it.nt; t++) {
+      const int64_t o = t * p.tstride;
+      const int i = own_column(iw);
+      const unsigned ui = i;
+      const double qc = ldu(q + o + ro, ui);
+      const double fx = xflux<VL>(g, lim, ldu(p.cflx + ro, ui), ldu(p.u + ro, ui), i, q + o + ro);
+      const double fxw = __shfl_up(fx, 1, kWave);
+      const double fs = yflux_any<VL>(g, lim, ldu(p.cfly + h * P, ui), ldu(p.v + h * P, ui), h, i, q + o);
+      const double fn = yflux_any<VL>(g, lim, ldu(p.cfly + ro, ui), ldu(p.v + ro, ui), r, i, q + o);
+      if (upd) {
+        stu(p.qx + toff + o + ro, ui, qc - 0.5 * ((fx - fxw) * lel / ac - dvx * qc) * dt);
+        stu(p.qy + toff + o + ro, ui, qc - 0.5 * ((fn * ln - fs * ls) / ac - dvy * qc) * dt);
+      }
     }
   }
 }
@@ -392,15 +428,31 @@ __global__ void __launch_bounds__(NF, GROUPED ? 4 : 8) k_adv_flux(AdvGrid g, Mes
   const double lel = M(GMC_LE_LON, r), ac = M(GMC_AREA_CELL, r), rac = 1.0 / ac, rmn = 1.0 / mn;
   const double ls = M(GMC_LE_LAT, r - 1), ln = M(GMC_LE_LAT, r);
   const XFace face = x_face<VL>(g, cx, ux, iw);
+  double sum = 0.0;
   for (int t = 0; t < it.nt; t++) {
     const int64_t o = t * p.tstride + ro;
     const double qo = ldu(q + o, uiw);
     const double fx = x_flux<VL>(g, lim, face, qy + o);
     const double fxw = __shfl_up(fx, 1, kWave);
     const double fs = sfy[t][threadIdx.x], fn = sfy[t][threadIdx.x + kWave];
-    if (upd) {
-      const double qv = om * qo - div_rn((fx - fxw) * lel + (fn * ln - fs * ls), ac, rac) * dt;
-      stu(qp + o, uiw, div_rn(qv, mn, rmn));
+    const double qv = om * qo - div_rn((fx - fxw) * lel + (fn * ln - fs * ls), ac, rac) * dt;
+    const double qn = div_rn(qv, mn, rmn);
+    sum += qn;
+    if (upd) stu(qp + o, uiw, qn);
+  }
+  if (any_not_finite(sum)) {
+#pragma unroll 1
+    for (int t = 0; t < it.nt; t++) {
+      const int64_t o = t * p.tstride;
+      const int i = own_column(iw);
+      const unsigned ui = i;
+      const double qo = ldu(q + o + ro, ui);
+      const double fx = xflux<VL>(g, lim, ldu(p.cflx + ro, ui), ldu(p.mfx + ro, ui), i, qy + o + ro);
+      const double fxw = __shfl_up(fx, 1, kWave);
+      const double fs = yflux_any<VL>(g, lim, ldu(p.cfly + h * P, ui), ldu(p.mfy + h * P, ui), h, i, qx + o);
+      const double fn = yflux_any<VL>(g, lim, ldu(p.cfly + ro, ui), ldu(p.mfy + ro, ui), r, i, qx + o);
+      const double qv = om * qo - ((fx - fxw) * lel + (fn * ln - fs * ls)) / ac * dt;
+      if (upd) stu(qp + o + ro, ui, qv / mn);
     }
   }
 }

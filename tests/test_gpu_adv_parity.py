@@ -231,3 +231,30 @@ def test_tracer_groups_bitwise(case):
         g.drive(n, sc[n:n + 1])
         _compare(o, g, ntr, f"step {n}")
     assert g.fixes == o.fixes
+
+
+# what the reciprocals of a group cannot divide by: Courant numbers whose
+# reciprocals overflow, and no mass.  630 x 120 takes groups of four tracers,
+# 126 x 15 one by one.
+@pytest.mark.parametrize("flux", ["ppm", "van_leer"])
+@pytest.mark.parametrize("nlon,nlat,ntr", [(630, 120, 7), (126, 15, 2)])
+def test_vanishing_winds_and_masses(nlon, nlat, ntr, flux):
+    st = _setup(nlon, nlat, 900.0, ntr, min(200, nlon // 2 - 4), flux=flux)
+    m = st.mesh.metrics
+    ub, vb = init_cond.deform_wind_basis(nlon, nlat, m, 3, 7, 40.0)
+    qs = [q + 1.0 for q in init_cond.tracer_set(nlon, nlat, m, 3, ntr)]
+    o, g = _pair(st, qs)
+    mass = np.ones((nlat, nlon))
+    for n, scale in enumerate((1.0, 1e-311, 1e-308, 1e-290, 1.0)):
+        u, v = ub * scale, vb * scale
+        if n == 4:      # the last step leaves two rows' cells without mass
+            mass = mass.copy()
+            mass[nlat // 2:nlat // 2 + 2, 5:9] = 0.0
+        o.set_wind(u, v, u, v, mass)
+        g.set_wind(u, v, u, v, mass)
+        assert o.run(n) == 0
+        g.run(n)
+        for l in range(ntr):
+            a, b = g.tracer(g.old, l), o.tracer(o.old, l)
+            np.testing.assert_array_equal(a, b, err_msg=f"step {n} tracer {l}")
+            assert np.isfinite(b).all() == (n < 4)
