@@ -522,7 +522,7 @@ __device__ __forceinline__ void gzf_item(const Grid &g, const FT &big, const FT 
   const int64_t o = r * g.pitch;
   const int nb = it.n, ns = it.n2;
   const int hb = nb > 1 ? (nb - 1) / 2 : 0, hs = ns > 1 ? (ns - 1) / 2 : 0, hw = hb > hs ? hb : hs;
-  double *wb = xs, *ws = xs + big.max_taps, *x0 = xs + big.max_taps + small.max_taps;
+  double *wb = xs, *ws = wb + max(nb, 0), *x0 = ws + max(ns, 0);
   const int len = it.c1 - it.c0 + 2 * hw;
   for (int k = tid; k < nb; k += NF) wb[k] = big.wgt_lon[(int64_t)r * big.max_taps + k];
   for (int k = tid; k < ns; k += NF) ws[k] = small.wgt_lon[(int64_t)r * small.max_taps + k];
@@ -563,9 +563,9 @@ __device__ __forceinline__ void uvf_item(const Grid &g, const MT &M, double dt, 
   const int r = it.row;
   const int64_t p = g.pitch, o = r * p;
   const int nl = g.nlon;
-  double *w = xs, *x0 = xs + big.max_taps;
   const bool pole_u = it.kind == 1 && (r == 0 || r == g.nlat - 1);   // not updated, copied to u_f
   const int n = pole_u ? 0 : it.n;
+  double *w = xs, *x0 = xs + max(n, 0);
   const int h = n > 1 ? (n - 1) / 2 : 0;
   const int len = it.c1 - it.c0 + 2 * h;
   const auto wg = (it.kind == 1 ? big.wgt_lon : big.wgt_lat) + (int64_t)r * big.max_taps;
@@ -1337,18 +1337,19 @@ static constexpr int kNarrowChunk = GMC_NARROW_CHUNK;
 
 // One row of a filter work list: `work` taps per output sets the chunk
 // width; n (and n2) are the taps of the row's filters, the window of a chunk
-// is its columns and (n - 1) / 2 on either side (lds: the largest window).
+// is its columns and (n - 1) / 2 of the wider filter's taps on either side
+// (lds: the most of weights and window).
 // Returns the number of chunks the row was cut into.
 static int add_row(std::vector<Item> &v, int row, int kind, int work, int nlon, size_t &lds, int n, int n2 = 0,
                    int chunk_work = kChunkWork) {
   int w = work <= 16 ? std::min(nlon, kNarrowChunk)
                      : std::min(nlon, std::max(64, (chunk_work / work + 63) / 64 * 64));
   const int parts = (nlon + w - 1) / w;
-  const int h = n > 1 ? (n - 1) / 2 : 0;
+  const int taps = std::max(n, 0) + std::max(n2, 0), widest = std::max(n, n2), h = widest > 1 ? (widest - 1) / 2 : 0;
   for (int k = 0; k < parts; k++) {
     const int c0 = (int)((int64_t)nlon * k / parts), c1 = (int)((int64_t)nlon * (k + 1) / parts);
     v.push_back(Item{row, c0, c1, kind, 0, n, n2, 0});
-    lds = std::max(lds, sizeof(double) * (size_t)(c1 - c0 + 2 * h));
+    lds = std::max(lds, sizeof(double) * (size_t)(taps + c1 - c0 + 2 * h));
   }
   return parts;
 }
@@ -1484,14 +1485,12 @@ static int build_stage(gmc_ctx *c, FusedPlan *P, const std::vector<int32_t> &nb,
   size_t lgz = 0, luv = 0;
   for (int r = 0; r < nlat; r++) {
     if (r >= m.ra && r < m.rb) continue;
-    add_row(items[1], r, 0, nb[r] + std::max(1, nb[r] / 2), nlon, lgz, std::max(nb[r], ns[r]), 0, kStageWork);
+    add_row(items[1], r, 0, nb[r] + std::max(1, nb[r] / 2), nlon, lgz, nb[r], ns[r], kStageWork);
     add_row(items[2], r, 1, nb[r], nlon, luv, nb[r], 0, kStageWork);
     if (r < nhalf) add_row(items[2], r, 2, nbv[r], nlon, luv, nbv[r], 0, kStageWork);
   }
-  for (auto &it : items[1]) { it.n = nb[it.row]; it.n2 = ns[it.row]; }
   for (int k = 1; k < 3; k++) deal_items(items[k]);
-  const size_t item[3] = {0, lgz + sizeof(double) * (c->big.max_taps + c->small1.max_taps),
-                          luv + sizeof(double) * c->big.max_taps};
+  const size_t item[3] = {0, lgz, luv};
   if (kItemsPerWg * std::max(item[1], item[2]) > kLds) return GMC_OK;
   // the short rows' tiles: what fills the second and third launch up to two
   // workgroups a compute unit, the two bands beside the polar rows (first and
@@ -1544,9 +1543,8 @@ static int build_plan(gmc_ctx *c) {
     };
     // gz items: the window is that of the wider of the two filters
     for (int r = 0; r < g.nlat; r++)
-      count(add_row(gz, r, 0, nb_lon[r] + std::max(1, nb_lon[r] / 2), g.nlon, P->lds_gz,
-                    std::max(nb_lon[r], ns_lon[r])), nb_lon[r]);
-    for (auto &it : gz) { it.n = nb_lon[it.row]; it.n2 = ns_lon[it.row]; }
+      count(add_row(gz, r, 0, nb_lon[r] + std::max(1, nb_lon[r] / 2), g.nlon, P->lds_gz, nb_lon[r], ns_lon[r]),
+            nb_lon[r]);
     // u row r next to v rows r - 1 and r: the three read gz_f row r
     for (int r = 0; r < g.nlat; r++) {
       count(add_row(uv, r, 1, nb_lon[r], g.nlon, P->lds_uv, nb_lon[r]), nb_lon[r]);
@@ -1562,8 +1560,6 @@ static int build_plan(gmc_ctx *c) {
     items.insert(items.end(), uv_d.begin(), uv_d.end());
     P->n_uv = (int)items.size() - P->n_gz;
   }
-  P->lds_gz += sizeof(double) * (c->big.max_taps + c->small1.max_taps);
-  P->lds_uv += sizeof(double) * c->big.max_taps;
   rc = check_hip(c, hipMalloc((void **)&P->d_items, sizeof(Item) * items.size()), "plan alloc");
   if (!rc) rc = check_hip(c, hipMemcpy(P->d_items, items.data(), sizeof(Item) * items.size(), hipMemcpyHostToDevice),
                           "plan copy");
@@ -1997,7 +1993,6 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
   // filter work items of every member, tagged with the member index
   std::vector<Item> gz, uv;
   size_t lgz = 0, luv = 0;
-  int maxb = 1, maxs = 1;
   for (int k = 0; k < n; k++) {
     gmc_ctx *c = e->m[k];
     const Grid &g = c->grid;
@@ -2013,7 +2008,7 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
     std::vector<Item> a, b;
     for (int r = 0; r < g.nlat; r++)
       if (polar(r))
-        add_row(a, r, 0, nb_lon[r] + std::max(1, nb_lon[r] / 2), g.nlon, lgz, std::max(nb_lon[r], ns_lon[r]), 0, kStageWork);
+        add_row(a, r, 0, nb_lon[r] + std::max(1, nb_lon[r] / 2), g.nlon, lgz, nb_lon[r], ns_lon[r], kStageWork);
     for (int r = 0; r < g.nlat; r++)
       if (polar(r)) add_row(b, r, 1, nb_lon[r], g.nlon, luv, nb_lon[r], 0, kStageWork);
     for (int r = 0; r < g.nhalf; r++)
@@ -2022,8 +2017,6 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
     e->nb_lat.push_back(nb_lat);
     e->ns_lon.push_back(ns_lon);
     for (auto &it : a) {
-      it.n = nb_lon[it.row];
-      it.n2 = ns_lon[it.row];
       it.member = k;
       gz.push_back(it);
     }
@@ -2031,15 +2024,13 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
       it.member = k;
       uv.push_back(it);
     }
-    maxb = std::max(maxb, c->big.max_taps);
-    maxs = std::max(maxs, c->small1.max_taps);
   }
   deal_items(gz);
   deal_items(uv);
   e->n_gz = (int)gz.size() / kItemsPerWg;
   e->n_uv = (int)uv.size() / kItemsPerWg;
-  e->lds_gz = lgz + sizeof(double) * (maxb + maxs);
-  e->lds_uv = luv + sizeof(double) * maxb;
+  e->lds_gz = lgz;
+  e->lds_uv = luv;
   int most = 0;
   for (const EnsShape &sh : kEnsShapes) {
     std::vector<StageMap> maps;

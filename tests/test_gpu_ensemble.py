@@ -9,7 +9,7 @@ import pytest
 
 from helpers import STATE
 from gmcore_amd import init_cond
-from gmcore_amd.host import Ensemble, Setup, ShallowWater
+from gmcore_amd.host import Ensemble, Setup, ShallowWater, make_config
 from gmcore_amd.namelist import Namelist
 
 pytestmark = pytest.mark.gpu
@@ -110,6 +110,37 @@ def test_uneven_members_bitwise(shape):
         for m in plain:
             m.step(n)
         _assert_same(ens_m, plain, f"{n} steps, shape {shape}")
+    ens.close()
+
+
+def test_wide_filter_tables_bitwise():
+    # tables of many more columns than any row has taps: what a launch keeps of
+    # a row's weights is the row's taps
+    def padded(nlon, nlat, dt, k):
+        st = Setup(Namelist(num_lon=nlon, num_lat=nlat, dt_dyn=dt, time_scheme="pc2"))
+        for f in (st.big, st.small):
+            for w in ("wgt_lon", "wgt_lat"):
+                a = getattr(f, w)
+                wide = np.zeros((a.shape[0], 3000))
+                wide[:, :a.shape[1]] = a
+                setattr(f, w, wide)
+            f.max_taps = 3000
+        st.cfg = make_config(st.nl, st.big, st.small)
+        ic = init_cond.seeded_state(nlon, nlat, st.mesh.metrics, 8, 0, perturb=(0.01, 100 + k),
+                                    omega=st.nl.omega, radius=st.nl.radius)
+        m = ShallowWater(st)
+        m.set_state(*ic)
+        m.prepare(1)
+        return m
+
+    specs = [(60, 31, 900.0), (72, 37, 1800.0), (180, 91, 600.0), (720, 361, 150.0)]
+    wide, alone, plain = ([make(*s, k) for k, s in enumerate(specs)] for make in (padded, padded, _member))
+    ens = Ensemble(wide)
+    ens.step(3)
+    for m in alone + plain:
+        m.step(3)
+    _assert_same(wide, plain, "ensemble")
+    _assert_same(alone, plain, "gmc_step")
     ens.close()
 
 
