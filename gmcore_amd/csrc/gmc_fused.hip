@@ -1493,19 +1493,17 @@ static int build_stage(gmc_ctx *c, FusedPlan *P, const std::vector<int32_t> &nb,
   const size_t item[3] = {0, lgz, luv};
   if (kItemsPerWg * std::max(item[1], item[2]) > kLds) return GMC_OK;
   // the short rows' tiles: what fills the second and third launch up to two
-  // workgroups a compute unit, the two bands beside the polar rows (first and
-  // last in the numbering) in the first
-  const int keep = std::min(m.ntiles, m.seg[0].nx + m.seg[m.nseg - 1].nx);
-  int left = m.ntiles - keep;
+  // workgroups a compute unit, from the middle of the numbering
+  int left = m.ntiles - beside_polar(m);
   for (int k = 1; k < 3; k++) {
     const int polar = (int)items[k].size() / kItemsPerWg, take = std::min(left, std::max(0, kStageSlots - polar));
     P->stage[k] = {polar, 0, take, (int)(item[k] / sizeof(double)), nullptr, std::max(kTileLds, kItemsPerWg * item[k])};
     left -= take;
   }
-  const int n0 = keep + left;   // the first launch's tiles, around the numbering's ends
-  P->stage[0] = {m.tiles_p, m.ntiles - (n0 + 1) / 2, n0, 0, nullptr, kTileLds};
-  P->stage[1].tile0 = n0 / 2;
-  P->stage[2].tile0 = n0 / 2 + P->stage[1].tiles;
+  const int n0 = beside_polar(m) + left, south = south_tiles(m, n0);
+  P->stage[0] = {m.tiles_p, m.ntiles - (n0 - south), n0, 0, nullptr, kTileLds};
+  P->stage[1].tile0 = south;
+  P->stage[2].tile0 = south + P->stage[1].tiles;
   rc = big_lds({(const void *)k_stage<kStageTend, false>, (const void *)k_stage<kStageTend, true>,
                 (const void *)k_stage<kStageGz, false>, (const void *)k_stage<kStageGz, true>,
                 (const void *)k_stage<kStageUv, false>, (const void *)k_stage<kStageUv, true>});

@@ -121,4 +121,14 @@ inline bool stage_map(int nlon, int nlat, const std::vector<int32_t> &nb, const 
   return true;
 }
 
+// Where the tiles of the short rows are shared out over three launches, the
+// first takes those of the bands next to the polar rows, whose gz_f the polar v
+// rows of the last launch read: beside_polar tiles at least.  Of n tiles it
+// takes, south_tiles are the first of the numbering and the rest the last.
+inline int beside_polar(const StageMap &m) { return std::min(m.ntiles, m.seg[0].nx + m.seg[m.nseg - 1].nx); }
+inline int south_tiles(const StageMap &m, int n) {
+  const int first = m.seg[0].nx, last = m.seg[m.nseg - 1].nx;
+  return n < first + last ? n : std::min(std::max(n / 2, first), n - last);
+}
+
 }  // namespace gmc

@@ -45,6 +45,13 @@ template <int TY> static void check(int nlon, int nlat, const std::vector<int32_
       fault("a whole-stage tile reads beyond its lanes", nlon, nlat, TY, t);
     if (G.r0 < 3 || G.r1 > nlat - 4) fault("a whole-stage tile next to a pole", nlon, nlat, TY, t);
   }
+  // the first launch's share, however many tiles it takes: the first `south` and
+  // the last of the numbering, with the bands beside the polar rows among them
+  for (int n = m.nseg ? beside_polar(m) : 0; n && n <= m.ntiles; n++) {
+    const int south = south_tiles(m, n), north = n - south;
+    if (south < 0 || north < 0 || (n < m.ntiles && (south < m.seg[0].nx || north < m.seg[m.nseg - 1].nx)))
+      fault("a band beside the polar rows not in the first launch", nlon, nlat, TY, n);
+  }
   for (char o : owned)
     if (o != 1) {
       fault("a point not owned exactly once", nlon, nlat, TY, -1);
@@ -79,6 +86,7 @@ int main() {
           nb[r] = taps();
           ns[r] = taps();
           nbv[r] = taps();
+          if (table == 2 && !polar && r > nlat / 2) nb[r] = ns[r] = nbv[r] = 1;   // no filters in the north
         }
         check<5>(nlon, nlat, nb, ns, nbv);
         check<7>(nlon, nlat, nb, ns, nbv);
