@@ -127,23 +127,25 @@ static void copy_packed(double *dst, int64_t dld, const double *src, int64_t sld
 // threads, since first touches of the caller's pages make one thread slower
 // than the link (16.6 MB: 0.30 ms on the link, 0.7 to 0.9 ms for the copy of
 // one thread into fresh pages, 0.3 of four).  The threads end with the call.
+// At most kMaxPieces pieces: each costs the link about 10 us.
 constexpr size_t kPiece = 512 * 1024, kThreadsFrom = 4 * 1024 * 1024;
-constexpr int kMaxPieces = 8, kHelpers = 3;   // each piece costs the link about 10 us
+constexpr int kHelpers = 3;
 static hipError_t stage_download(HostStage &s, hipStream_t stream, const double *dev, int64_t pitch, double *host,
                                  int64_t ld, int nlon, int rows) {
   const size_t row = sizeof(double) * nlon, bytes = row * rows;
-  const int pieces = std::max(1, (int)std::min({(size_t)kMaxPieces, (size_t)rows, bytes / kPiece}));
+  const int pieces = std::max(1, (int)std::min({(size_t)HostStage::kMaxPieces, (size_t)rows, bytes / kPiece}));
   if (pieces == 1) {
     hipError_t e = hipMemcpy2DAsync(s.p, row, dev, sizeof(double) * pitch, row, rows, hipMemcpyDeviceToHost, stream);
     if (e == hipSuccess) e = hipStreamSynchronize(stream);
     if (e == hipSuccess) copy_packed(host, ld, s.p, nlon, nlon, rows);
     return e;
   }
-  while ((int)s.ev.size() < pieces) {
-    hipEvent_t ev;
-    const hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-    if (e != hipSuccess) return e;
-    s.ev.push_back(ev);
+  for (int k = 0; k < pieces; k++) {
+    const hipError_t e = s.ev[k] ? hipSuccess : hipEventCreateWithFlags(&s.ev[k], hipEventDisableTiming);
+    if (e != hipSuccess) {
+      s.ev[k] = nullptr;
+      return e;
+    }
   }
   auto first = [&](int k) { return (int)((int64_t)rows * k / pieces); };
   for (int k = 0; k < pieces; k++) {
@@ -201,7 +203,8 @@ hipError_t stage_copy(HostStage &s, hipStream_t stream, bool to_device, double *
 
 void stage_free(HostStage &s) {
   if (s.p) (void)hipHostFree(s.p);
-  for (hipEvent_t e : s.ev) (void)hipEventDestroy(e);
+  for (hipEvent_t e : s.ev)
+    if (e) (void)hipEventDestroy(e);
   s = HostStage{};
 }
 

@@ -62,9 +62,10 @@ struct FilterDev {
 // 2D copies between pageable host memory and pitched device rows go row by
 // row, so a field passes through this buffer (packed rows) instead.
 struct HostStage {
+  static constexpr int kMaxPieces = 8;
   double *p = nullptr;
   size_t cap = 0;   // doubles
-  std::vector<hipEvent_t> ev;   // the ends of a download's pieces
+  hipEvent_t ev[kMaxPieces] = {};   // the ends of a download's pieces
 };
 // rows x nlon doubles between dev (row pitch `pitch`) and host (leading
 // dimension ld), through s; returns once the copy is complete.
