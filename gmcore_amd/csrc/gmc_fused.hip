@@ -1101,17 +1101,19 @@ __device__ __forceinline__ void band_stage(const Grid &g, RecPtr mrows, double g
 // part one after the other:
 //   one launch    (kStageOne) where their circles fit into LDS: bands of the
 //                 polar rows beside the tiles;
-//   three launches (kStageTend, kStageGz, kStageUv) elsewhere: tiles of the
-//                 polar tendencies, then four filter items a workgroup, with
-//                 the tiles of the other rows spread over the three so that
-//                 none of them leaves compute units idle.
+//   three launches (kStageTend, kStageGz, kStageUv) on wider grids of many
+//                 tiles (kSpreadTiles): tiles of the polar tendencies, then
+//                 four filter items a workgroup, with the tiles of the other
+//                 rows spread over the three so that none of them leaves
+//                 compute units idle;
+//   k_tend, k_gzf and k_uvf over all rows on the others.
 // A polar v row next to the tiles reads their gz_f row, so the tiles beside
 // the polar rows go into the first launch.
 //
 // Measured per step with three models in flight on three streams (and alone),
 // three kernels a stage against this: 180 x 91 wrfrk3 17.9 (50) -> 13.5 (39)
 // us, 360 x 181 24.1 (62) -> 19.4 (55), 502 x 253 with damping 35 (90) -> 31
-// (85), 1440 x 721 149 (164) -> 134 (163).  A full tile takes 5 us from its
+// (85); the wider grids at kSpreadTiles.  A full tile takes 5 us from its
 // start to its last store; the band at a pole, 17 us at 360 columns, bounds
 // the small grids, the vector instructions and the loads of the tiles (two
 // workgroups a compute unit, 45 % of the issue slots) the large ones.
@@ -1431,6 +1433,18 @@ template <class T> static int to_device(gmc_ctx *c, FusedPlan *P, const std::vec
 // up to with tiles: two on each compute unit.
 static constexpr int kStageWork = 8192, kStageSlots = 2 * 256;
 
+// Tiles of the whole grid from which a stage of wide circles goes in the three
+// launches that share its tiles out, two and a half a compute unit.  A filter
+// launch is as long as its widest rows' chains, 4 to 5 us longer beside tiles;
+// below, k_tend's tiles run at once or nearly so and spreading them saves less
+// than that.  us a step of one model (of three in flight), three launches and
+// three kernels: 560 x 281 (260 tiles) 82 (35) and 70 (29), 720 x 361 (396) 94
+// (41.5) and 76 (37.4), 900 x 451 (615) 104 (53) and 92 (53), 960 x 481 (704)
+// 106 (57) and 101 (59), 1024 x 513 (846) 109 (62) and 104 (69), 1440 x 721
+// (1584) 164 (134) and 147 to 154 (147), 2160 x 1081 (3564) 336 (289) and 348
+// (322).
+static constexpr int kSpreadTiles = 5 * 256 / 2;
+
 // Heavy and light items share a workgroup: item i of the order by work goes to
 // workgroup i mod the number of workgroups.
 static void deal_items(std::vector<Item> &v) {
@@ -1481,6 +1495,7 @@ static int build_stage(gmc_ctx *c, FusedPlan *P, const std::vector<int32_t> &nb,
     return rc;
   }
   // three launches
+  if (((nlon + TX - 1) / TX) * ((nlat + S::TY - 1) / S::TY) < kSpreadTiles) return GMC_OK;
   std::vector<Item> items[3];
   size_t lgz = 0, luv = 0;
   for (int r = 0; r < nlat; r++) {

@@ -41,7 +41,9 @@ def test_stage_on_tile_edges(nlon, nlat, scheme):
 # and even zones; the widest circles of the bands and the first beyond; wide
 # filters (long steps) and none (short ones)
 FORMS = [(62, 30, 1.0), (64, 23, 1.0), (64, 24, 1.0), (66, 25, 3.0), (108, 61, 1.0), (110, 60, 2.0), (180, 91, 5.0),
-         (502, 64, 1.0), (516, 65, 4.0), (560, 64, 1.0), (602, 127, 3.0), (722, 100, 0.2)]
+         (502, 64, 1.0), (516, 65, 4.0), (560, 64, 1.0), (602, 127, 3.0), (722, 100, 0.2),
+         # circles too wide for LDS: the tiles shared out from 640 tiles on
+         (602, 638, 1.0), (602, 640, 1.0), (722, 601, 0.2), (1442, 300, 3.0)]
 
 
 @pytest.mark.parametrize("nlon,nlat,long", FORMS)
