@@ -113,22 +113,31 @@ static int upload_filter(gmc_ctx *c, const gmc_filter &f, FilterDev &d, int slot
   return rc;
 }
 
-// rows x nlon packed doubles <-> rows of leading dimension ld
+// rows x nlon packed doubles <-> rows of leading dimension ld.  Packed ones are
+// copied in runs of 128 KB, up to 8 MB: a memcpy of a megabyte and more writes
+// past the caches, and the data is in them when a download's copy ends on the
+// link, and wanted there when an upload's begins (2.1 MB each way: 99 and 83 us
+// in one memcpy, 93 and 76 in runs; row by row 92 and 78).  Larger ones leave
+// the caches anyway (16.7 MB up: 510 us in one memcpy, 580 in runs, 700 by row).
 static void copy_packed(double *dst, int64_t dld, const double *src, int64_t sld, int nlon, int rows) {
-  if (dld == nlon && sld == nlon) {   // one run: 80 GB/s here against 32 row by row
-    std::memcpy(dst, src, sizeof(double) * (size_t)nlon * rows);
+  constexpr size_t kRun = 128 * 1024 / sizeof(double), kCached = 8 * 1024 * 1024 / sizeof(double);
+  if (dld == nlon && sld == nlon) {
+    const size_t n = (size_t)nlon * rows, run = n <= kCached ? kRun : n;
+    for (size_t k = 0; k < n; k += run) std::memcpy(dst + k, src + k, sizeof(double) * std::min(run, n - k));
     return;
   }
   for (int r = 0; r < rows; r++) std::memcpy(dst + (size_t)r * dld, src + (size_t)r * sld, sizeof(double) * nlon);
 }
 
 // A download of more than a piece passes through the stage in pieces, so that
-// the host copies one while the next is on the link; a large one with helper
-// threads, since first touches of the caller's pages make one thread slower
-// than the link (16.6 MB: 0.30 ms on the link, 0.7 to 0.9 ms for the copy of
-// one thread into fresh pages, 0.3 of four).  The threads end with the call.
-// At most kMaxPieces pieces: each costs the link about 10 us.
-constexpr size_t kPiece = 512 * 1024, kThreadsFrom = 4 * 1024 * 1024;
+// the host copies one while the next is on the link, with helper threads, since
+// first touches of the caller's pages make one thread slower than the link
+// (16.6 MB: 0.30 ms on the link, 0.7 to 0.9 ms for the copy of one thread into
+// fresh pages, 0.3 of four).  The threads end with the call.  At most kMaxPieces
+// pieces of at least 2 MB: each costs the link about 10 us, and the first can
+// only be copied when it is there (4.2 MB: 175 us in one piece, 165 in two, 240
+// in eight of 512 KB).
+constexpr size_t kPiece = 2 * 1024 * 1024;
 constexpr int kHelpers = 3;
 static hipError_t stage_download(HostStage &s, hipStream_t stream, const double *dev, int64_t pitch, double *host,
                                  int64_t ld, int nlon, int rows) {
@@ -167,14 +176,13 @@ static hipError_t stage_download(HostStage &s, hipStream_t stream, const double 
     }
   };
   std::thread helper[kHelpers];
-  if (bytes >= kThreadsFrom)
-    for (std::thread &t : helper) {
-      try {
-        t = std::thread(work);
-      } catch (...) {   // none to be had: the pieces are this thread's
-        break;
-      }
+  for (int k = 0; k < std::min(kHelpers, pieces - 1); k++) {
+    try {
+      helper[k] = std::thread(work);
+    } catch (...) {   // none to be had: the pieces are this thread's
+      break;
     }
+  }
   work();
   for (std::thread &t : helper)
     if (t.joinable()) t.join();

@@ -14,7 +14,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("nlon,nlat,nlev,pad", [(16, 9, 2, 0), (16, 9, 2, 5), (362, 181, 2, 0), (360, 181, 4, 0),
-                                                (360, 181, 10, 3), (360, 181, 32, 0)])
+                                                (360, 181, 10, 3), (360, 181, 32, 0),
+                                                # two pieces of 2 MB just not and just reached, three
+                                                (512, 256, 3, 0), (512, 257, 4, 0), (512, 257, 6, 0)])
 def test_fields_come_back(nlon, nlat, nlev, pad):
     mesh = Mesh(nlon, nlat, 6371220.0, 7.292e-5)
     b = Baroclinic(mesh, np.linspace(0.0, 1.0, nlev + 1) * 0.1, np.linspace(0.0, 0.9, nlev + 1))
