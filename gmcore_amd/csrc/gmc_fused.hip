@@ -1302,13 +1302,13 @@ __global__ void __launch_bounds__(S::NT, 8) k_tend_ens(const EnsMember *__restri
 }
 
 // Workgroups [0, groups): an item per group of NF threads (the list is padded
-// with empty items); then the listed tiles.
+// with empty items); then the listed tiles, where a workgroup has their size.
 template <bool GZ>
 __global__ void __launch_bounds__(StageTile::NT, 8) k_filter_ens(const EnsMember *__restrict__ mem,
                                                                  const StageMap *__restrict__ maps,
                                                                  const EnsTile *__restrict__ tiles, int ntiles,
                                                                  const Item *__restrict__ items, int groups,
-                                                                 int item_lds) {
+                                                                 int per_wg, int item_lds) {
   extern __shared__ __attribute__((aligned(16))) double xs[];
   const int b = blockIdx.x;
   if (b >= groups) {
@@ -1316,7 +1316,7 @@ __global__ void __launch_bounds__(StageTile::NT, 8) k_filter_ens(const EnsMember
     return;
   }
   const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x / NF), tid = threadIdx.x % NF;
-  const Item &it = items[b * kItemsPerWg + grp];
+  const Item &it = items[b * per_wg + grp];
   const EnsMember *d = mem + it.member;
   double *x = xs + grp * item_lds;
   if constexpr (GZ)
@@ -1445,15 +1445,27 @@ static constexpr int kStageWork = 8192, kStageSlots = 2 * 256;
 // (322).
 static constexpr int kSpreadTiles = 5 * 256 / 2;
 
-// Heavy and light items share a workgroup: item i of the order by work goes to
-// workgroup i mod the number of workgroups.
-static void deal_items(std::vector<Item> &v) {
+// Tiles of 60 x 11 over all rows of all members from which an ensemble's tiles
+// take the short rows whole: more than run at once.  Below, a launch is one
+// workgroup's chain, which a whole tile or four filter items in a workgroup only
+// make longer.  us a step, every row in three kernels with a filter item a
+// workgroup, and whole tiles: 2 members of 180 x 91 (54 tiles) 54.7 and 69, 2 of
+// 180 x 91 and one of 360 x 181 (156) 63.6 and 74.6, 4 of 360 x 181 (408) 87 and
+// 95, 16 of 180 x 91 (432) 90.3 and 92.2; 2 of 180 x 91, one of 360 x 181 and
+// one of 720 x 361 (552) 115 and 108, 3 and 6 of the first two (693) 114.6 and
+// 117, 2 of 720 x 361 (792) 131 and 122, 8, 6 and 2 of the three (1620) 202 and
+// 200.
+static constexpr int kWholeTiles = kStageSlots;
+
+// Heavy and light items share a workgroup of `per`: item i of the order by work
+// goes to workgroup i mod the number of workgroups.
+static void deal_items(std::vector<Item> &v, int per = kItemsPerWg) {
   auto taps = [](const Item &it) { return (int64_t)(it.c1 - it.c0) * std::max(it.n + it.n2, 1); };
   std::stable_sort(v.begin(), v.end(), [&](const Item &a, const Item &b) { return taps(a) > taps(b); });
-  while (v.size() % kItemsPerWg) v.push_back(Item{1, 0, 0, 1, 0, 0, 0, 0});   // no columns
-  const int n = (int)v.size() / kItemsPerWg;
+  while (v.size() % per) v.push_back(Item{1, 0, 0, 1, 0, 0, 0, 0});   // no columns
+  const int n = (int)v.size() / per;
   std::vector<Item> dealt(v.size());
-  for (int i = 0; i < (int)v.size(); i++) dealt[i % n * kItemsPerWg + i / n] = v[i];
+  for (int i = 0; i < (int)v.size(); i++) dealt[i % n * per + i / n] = v[i];
   v = dealt;
 }
 
@@ -1780,6 +1792,8 @@ struct gmc_ens {
   gmc::StageMap *d_maps = nullptr;  // [members],
   gmc::EnsTile *d_tiles = nullptr;  // the tiles of the three launches
   gmc::Item *d_items = nullptr;
+  bool whole = false;               // tiles take the rows of short filters through the whole stage
+  int per_wg = 1;                   // filter items of a workgroup
   int n_gz = 0, n_uv = 0;           // workgroups of filter items
   size_t lds_gz = 0, lds_uv = 0;    // LDS of an item
   int tiles[3] = {0, 0, 0};
@@ -1815,7 +1829,7 @@ int ens_maps(gmc_ens *e, int ty, std::vector<StageMap> &maps) {
   maps.resize(e->m.size());
   for (size_t k = 0; k < e->m.size(); k++) {
     const Grid &g = e->m[k]->grid;
-    stage_map(g.nlon, g.nlat, e->nb_lon[k], e->ns_lon[k], e->nb_lat[k], ty, maps[k]);
+    stage_map(g.nlon, g.nlat, e->nb_lon[k], e->ns_lon[k], e->nb_lat[k], ty, maps[k], e->whole);
     tiles += maps[k].tiles_p + maps[k].ntiles;
   }
   return tiles;
@@ -1902,9 +1916,10 @@ void ens_launch_step(gmc_ens *e, int par) {
   // k_tend_ens covers every tile when grid == total or grid >= NXCD
   const int grid = sh.mult ? std::min(e->tiles[0], sh.mult * 256) : e->tiles[0];
   const EnsTile *t1 = e->d_tiles + e->tiles[0], *t2 = t1 + e->tiles[1];
-  auto lds = [](size_t item, int tiles) {
-    return (uint32_t)std::max(kItemsPerWg * item, tiles ? sizeof(double) * StageTile::SH_ALL : 0);
+  auto lds = [&](size_t item, int tiles) {
+    return (uint32_t)std::max(e->per_wg * item, tiles ? sizeof(double) * StageTile::SH_ALL : 0);
   };
+  const dim3 block(e->per_wg * NF);
   for (int st = 0; st < e->nstage; st++) {
     const EnsMember *mem = e->d_mem + ((size_t)par * e->nstage + st) * nm;
     switch (sh.ty) {
@@ -1912,12 +1927,12 @@ void ens_launch_step(gmc_ens *e, int par) {
     case 7: launch_tend<7>(e, mem, grid); break;
     default: launch_tend<11>(e, mem, grid);
     }
-    hipLaunchKernelGGL(k_filter_ens<true>, dim3(e->n_gz + e->tiles[1]), dim3(StageTile::NT),
-                       lds(e->lds_gz, e->tiles[1]), e->stream, mem, e->d_maps, t1, e->tiles[1], e->d_items, e->n_gz,
+    hipLaunchKernelGGL(k_filter_ens<true>, dim3(e->n_gz + e->tiles[1]), block, lds(e->lds_gz, e->tiles[1]), e->stream,
+                       mem, e->d_maps, t1, e->tiles[1], e->d_items, e->n_gz, e->per_wg,
                        (int)(e->lds_gz / sizeof(double)));
-    hipLaunchKernelGGL(k_filter_ens<false>, dim3(e->n_uv + e->tiles[2]), dim3(StageTile::NT),
-                       lds(e->lds_uv, e->tiles[2]), e->stream, mem, e->d_maps, t2, e->tiles[2],
-                       e->d_items + kItemsPerWg * e->n_gz, e->n_uv, (int)(e->lds_uv / sizeof(double)));
+    hipLaunchKernelGGL(k_filter_ens<false>, dim3(e->n_uv + e->tiles[2]), block, lds(e->lds_uv, e->tiles[2]), e->stream,
+                       mem, e->d_maps, t2, e->tiles[2], e->d_items + e->per_wg * e->n_gz, e->n_uv, e->per_wg,
+                       (int)(e->lds_uv / sizeof(double)));
   }
 }
 
@@ -2003,6 +2018,12 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
   e->scheme = members[0]->cfg.time_scheme;
   e->nstage = stage_count(e->scheme);
   e->dt.assign(n, 0.0);
+  // few tiles: every row in the three kernels, a filter item a workgroup
+  int ntiles = 0;
+  for (const gmc_ctx *c : e->m)
+    ntiles += ((c->grid.nlon + TX - 1) / TX) * ((c->grid.nlat + StageTile::TY - 1) / StageTile::TY);
+  e->whole = ntiles >= kWholeTiles;
+  e->per_wg = e->whole ? kItemsPerWg : 1;
   // filter work items of every member, tagged with the member index
   std::vector<Item> gz, uv;
   size_t lgz = 0, luv = 0;
@@ -2016,7 +2037,7 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
       return fail(GMC_EDEVICE, "filter tables");
     // the rows that the tiles do not take through the whole stage
     StageMap sm;
-    stage_map(g.nlon, g.nlat, nb_lon, ns_lon, nb_lat, StageTile::TY, sm);
+    stage_map(g.nlon, g.nlat, nb_lon, ns_lon, nb_lat, StageTile::TY, sm, e->whole);
     auto polar = [&](int r) { return r < sm.ra || r >= sm.rb; };
     std::vector<Item> a, b;
     for (int r = 0; r < g.nlat; r++)
@@ -2038,10 +2059,10 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
       uv.push_back(it);
     }
   }
-  deal_items(gz);
-  deal_items(uv);
-  e->n_gz = (int)gz.size() / kItemsPerWg;
-  e->n_uv = (int)uv.size() / kItemsPerWg;
+  deal_items(gz, e->per_wg);
+  deal_items(uv, e->per_wg);
+  e->n_gz = (int)gz.size() / e->per_wg;
+  e->n_uv = (int)uv.size() / e->per_wg;
   e->lds_gz = lgz;
   e->lds_uv = luv;
   int most = 0;
@@ -2061,7 +2082,7 @@ int gmc_ens_create(gmc_ctx *const *members, int32_t n, gmc_ens **out) {
   // an item's window and taps are at most about three circles of the widest
   // member's (k_tend's limit): four of them fit
   constexpr size_t kLds = 160 * 1024;
-  if (!rc && kItemsPerWg * std::max(e->lds_gz, e->lds_uv) > kLds) rc = eerr(e, GMC_EINVAL, "filter window exceeds LDS");
+  if (!rc && e->per_wg * std::max(e->lds_gz, e->lds_uv) > kLds) rc = eerr(e, GMC_EINVAL, "filter window exceeds LDS");
   for (const void *f : {(const void *)k_filter_ens<true>, (const void *)k_filter_ens<false>})
     if (!rc) rc = ehip(e, hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds), "lds");
   if (rc) {

@@ -81,11 +81,11 @@ inline void short_rows(int nlat, const std::vector<int32_t> &nb, const std::vect
 // zones are most of the grid) whose short rows are at least half of all have
 // such rows; false, and every row among the others, elsewhere.
 inline bool stage_map(int nlon, int nlat, const std::vector<int32_t> &nb, const std::vector<int32_t> &ns,
-                      const std::vector<int32_t> &nbv, int ty, StageMap &m) {
+                      const std::vector<int32_t> &nbv, int ty, StageMap &m, bool whole = true) {
   m = StageMap{};
   auto half_width = [](int n) { return n > 1 ? (n - 1) / 2 : 0; };
   m.ra = m.rb = nlat;
-  if (nlon >= kWave && nlat >= 24) short_rows(nlat, nb, ns, nbv, m.ra, m.rb);
+  if (whole && nlon >= kWave && nlat >= 24) short_rows(nlat, nb, ns, nbv, m.ra, m.rb);
   const bool has = 2 * (m.rb - m.ra) >= nlat;
   if (!has) m.ra = m.rb = nlat;
   m.nx_p = (nlon + TX - 1) / TX;

@@ -113,6 +113,23 @@ def test_uneven_members_bitwise(shape):
     ens.close()
 
 
+# the same beside a member of so many tiles that all members' short rows go
+# through their tiles whole (512 tiles of 60 x 11 and more; the others above
+# are some 300, every row in three kernels), and either side of that number
+@pytest.mark.parametrize("more,shape", [((1440, 300, 1.0), 0), ((1440, 300, 1.0), 4), ((1440, 300, 1.0), 8),
+                                        ((602, 198, 1.0), 0), ((602, 209, 1.0), 0)])
+def test_uneven_members_whole_bitwise(more, shape):
+    specs = [(nlon, nlat, 20000.0 * long / max(nlon, nlat)) for nlon, nlat, long in ODD + [more]]
+    ens_m, plain = ([_member(*s, k) for k, s in enumerate(specs)] for _ in range(2))
+    ens = Ensemble(ens_m)
+    ens.set_shape(shape)
+    ens.step(3)
+    for m in plain:
+        m.step(3)
+    _assert_same(ens_m, plain, f"{more}, shape {shape}")
+    ens.close()
+
+
 def test_wide_filter_tables_bitwise():
     # tables of many more columns than any row has taps: what a launch keeps of
     # a row's weights is the row's taps
@@ -133,7 +150,7 @@ def test_wide_filter_tables_bitwise():
         m.prepare(1)
         return m
 
-    specs = [(60, 31, 900.0), (72, 37, 1800.0), (180, 91, 600.0), (720, 361, 150.0)]
+    specs = [(60, 31, 900.0), (180, 91, 600.0), (360, 181, 300.0), (720, 361, 150.0)]
     wide, alone, plain = ([make(*s, k) for k, s in enumerate(specs)] for make in (padded, padded, _member))
     ens = Ensemble(wide)
     ens.step(3)
