@@ -216,12 +216,13 @@ __device__ __forceinline__ void tile_poles(const Grid &g, const MT &Mg, double g
   if (R0 + S::TY + 3 >= g.nlat - 1) pole_sums<S::NT>(g, Mg, grav, rgrav, P, 1, sh, pole);
 }
 
-// the six upwind derivatives of one edge point into a tape
-__device__ __forceinline__ void tape_upwind(double *const *dst, int64_t o, const UpwD &d) {
-  dst[0][o] = d.dt;
-  dst[1][o] = d.dn;
+// the six upwind derivatives of an edge point, column i of the row at `row` of
+// the fields, into a tape
+__device__ __forceinline__ void tape_upwind(double *const *dst, int64_t row, unsigned i, const UpwD &d) {
+  row_st(dst[0] + row, i, d.dt);
+  row_st(dst[1] + row, i, d.dn);
 #pragma unroll
-  for (int j = 0; j < 4; j++) dst[2 + j][o] = d.df[j];
+  for (int j = 0; j < 4; j++) row_st(dst[2 + j] + row, i, d.df[j]);
 }
 
 // A short zonal filter (half width H) of a value held one column a lane, taps
@@ -300,7 +301,6 @@ __device__ __forceinline__ void tend_tile(const Grid &g, const MT &Mg, RecPtr mr
   const int kn = min(k + 1, S::LR - 1), ks = max(k - 1, 0), kss = max(k - 2, 0);
   const bool out_pt = k >= 2 && r < G.r1 && q >= G.hl && q < G.hl + G.nc;
   const bool u_row = r >= 1 && r <= nlat - 2, v_row = r >= 0 && r < nhalf;
-  const int64_t o = r * p + ic;
   const MeshRow M(mrows, nlat, r);
 
   // A: m, u_f, v_f of the row
@@ -314,8 +314,8 @@ __device__ __forceinline__ void tend_tile(const Grid &g, const MT &Mg, RecPtr mr
     svf[k][LC] = io.vf_x;
   }
   if (TAPE && out_pt && tape->u_f) {
-    tape->u_f[o] = uf;
-    if (v_row) tape->v_f[o] = vf;
+    row_st(tape->u_f + r * p, ic, uf);
+    if (v_row) row_st(tape->v_f + r * p, ic, vf);
   }
   __syncthreads();
 
@@ -351,10 +351,10 @@ __device__ __forceinline__ void tend_tile(const Grid &g, const MT &Mg, RecPtr mr
   spv[k][q] = pv;
   ske[k][q] = ke;
   if (TAPE && out_pt && v_row) {
-    tape->m_vtx[o] = mv;
-    tape->pv[o] = pv;
-    tape->mfy[o] = mfy;
-    tape->m_lat[o] = (m0 + m2) * 0.5;
+    row_st(tape->m_vtx + r * p, ic, mv);
+    row_st(tape->pv + r * p, ic, pv);
+    row_st(tape->mfy + r * p, ic, mfy);
+    row_st(tape->m_lat + r * p, ic, (m0 + m2) * 0.5);
   }
   __syncthreads();
 
@@ -366,38 +366,55 @@ __device__ __forceinline__ void tend_tile(const Grid &g, const MT &Mg, RecPtr mr
   const double mfy_s = smfy[ks][q], mfx_n = smfx[kn][q];
   double pl = 0.0, pt = 0.0;
   if (k >= 1 && k < S::TY + 3) {
-    const double pss = spv[kss][q], ps = spv[ks][q], pn = spv[kn][q];
-    const double pw = lane_west(pv), pww = lane_west(pw), pe = lane_east(pv);
-    const double tl = tangent_sum(M(GMC_FULL_TANGENT_WGT1, r), M(GMC_FULL_TANGENT_WGT2, r), mfy_s, lane_east(mfy_s),
-                                  mfy, lane_east(mfy));
-    const double tu = tangent_sum(M(GMC_HALF_TANGENT_WGT1, r), M(GMC_HALF_TANGENT_WGT2, r), lane_west(mfx), mfx,
-                                  lane_west(mfx_n), mfx_n);
-    const double vl = div_mid(tl, (m0 + m1) * 0.5);
-    const double ul = div_mid(tu, (m0 + m2) * 0.5);
-    if (pv_scheme == GMC_PV_UPWIND && order == 3) {   // both edges in one block
-      pl = pv_upwind_edge(3, wgt, vl, uf, 0, pss, ps, pv, pn);
-      pt = pv_upwind_edge(3, wgt, ul, vf, 1, pww, pw, pv, pe);
-    } else {
-      pl = pv_edge(pv_scheme, order, wgt, vl, uf, 0, dt, M(GMC_LE_LON, r), pss, ps, pv, pn);
+    auto lon_tangent = [&] {
+      return tangent_sum(M(GMC_FULL_TANGENT_WGT1, r), M(GMC_FULL_TANGENT_WGT2, r), mfy_s, lane_east(mfy_s), mfy,
+                         lane_east(mfy));
+    };
+    auto lat_tangent = [&] {
+      return tangent_sum(M(GMC_HALF_TANGENT_WGT1, r), M(GMC_HALF_TANGENT_WGT2, r), lane_west(mfx), mfx,
+                         lane_west(mfx_n), mfx_n);
+    };
+    if (TAPE) {   // an edge at a time: both with their tapes are more than the registers
+      {
+        const double pss = spv[kss][q], ps = spv[ks][q], pn = spv[kn][q];
+        const double t = lon_tangent(), ml = (m0 + m1) * 0.5, vl = div_mid(t, ml);
+        pl = pv_edge(pv_scheme, order, wgt, vl, uf, 0, dt, M(GMC_LE_LON, r), pss, ps, pv, pn);
+        if (!u_row) pl = 0.0;
+        if (out_pt && u_row) {
+          row_st(tape->m_lon + r * p, ic, ml);
+          row_st(tape->mfx + r * p, ic, mfx);
+          if (tape->mfy_lon) row_st(tape->mfy_lon + r * p, ic, t);
+          row_st(tape->v_lon + r * p, ic, vl);
+          row_st(tape->pv_lon + r * p, ic, pl);
+          if (tape->dlon[0])
+            tape_upwind(tape->dlon, r * p, ic, upwind_deriv(pv_scheme, order, wgt, vl, uf, 0, pss, ps, pv, pn));
+        }
+      }
+      const double pw = lane_west(pv), pww = lane_west(pw), pe = lane_east(pv);
+      const double t = lat_tangent(), ul = div_mid(t, (m0 + m2) * 0.5);
       pt = pv_edge(pv_scheme, order, wgt, ul, vf, 1, dt, M(GMC_LE_LAT, r), pww, pw, pv, pe);
-    }
-    if (!u_row) pl = 0.0;
-    if (!v_row) pt = 0.0;
-    if (TAPE && out_pt) {
-      if (u_row) {
-        tape->m_lon[o] = (m0 + m1) * 0.5;
-        tape->mfx[o] = mfx;
-        if (tape->mfy_lon) tape->mfy_lon[o] = tl;
-        tape->v_lon[o] = vl;
-        tape->pv_lon[o] = pl;
-        if (tape->dlon[0]) tape_upwind(tape->dlon, o, upwind_deriv(pv_scheme, order, wgt, vl, uf, 0, pss, ps, pv, pn));
+      if (!v_row) pt = 0.0;
+      if (out_pt && v_row) {
+        if (tape->mfx_lat) row_st(tape->mfx_lat + r * p, ic, t);
+        row_st(tape->u_lat + r * p, ic, ul);
+        row_st(tape->pv_lat + r * p, ic, pt);
+        if (tape->dlat[0])
+          tape_upwind(tape->dlat, r * p, ic, upwind_deriv(pv_scheme, order, wgt, ul, vf, 1, pww, pw, pv, pe));
       }
-      if (v_row) {
-        if (tape->mfx_lat) tape->mfx_lat[o] = tu;
-        tape->u_lat[o] = ul;
-        tape->pv_lat[o] = pt;
-        if (tape->dlat[0]) tape_upwind(tape->dlat, o, upwind_deriv(pv_scheme, order, wgt, ul, vf, 1, pww, pw, pv, pe));
+    } else {
+      const double pss = spv[kss][q], ps = spv[ks][q], pn = spv[kn][q];
+      const double pw = lane_west(pv), pww = lane_west(pw), pe = lane_east(pv);
+      const double vl = div_mid(lon_tangent(), (m0 + m1) * 0.5);
+      const double ul = div_mid(lat_tangent(), (m0 + m2) * 0.5);
+      if (pv_scheme == GMC_PV_UPWIND && order == 3) {   // both edges in one block
+        pl = pv_upwind_edge(3, wgt, vl, uf, 0, pss, ps, pv, pn);
+        pt = pv_upwind_edge(3, wgt, ul, vf, 1, pww, pw, pv, pe);
+      } else {
+        pl = pv_edge(pv_scheme, order, wgt, vl, uf, 0, dt, M(GMC_LE_LON, r), pss, ps, pv, pn);
+        pt = pv_edge(pv_scheme, order, wgt, ul, vf, 1, dt, M(GMC_LE_LAT, r), pww, pw, pv, pe);
       }
+      if (!u_row) pl = 0.0;
+      if (!v_row) pt = 0.0;
     }
   }
   spl[k][q] = pl;
@@ -961,7 +978,7 @@ __device__ __forceinline__ void band_stage(const Grid &g, RecPtr mrows, double g
         if (tape.mfy_lon) row_st(tape.mfy_lon + r * p, i, tl);
         row_st(tape.v_lon + r * p, i, vl);
         row_st(tape.pv_lon + r * p, i, pl);
-        if (tape.dlon[0]) tape_upwind(tape.dlon, r * p + i, upwind_deriv(pv_scheme, order, wgt, vl, uf, 0, a1, a2, a3, a4));
+        if (tape.dlon[0]) tape_upwind(tape.dlon, r * p, i, upwind_deriv(pv_scheme, order, wgt, vl, uf, 0, a1, a2, a3, a4));
       }
       spl[k * n + i] = pl;
     }
@@ -979,7 +996,7 @@ __device__ __forceinline__ void band_stage(const Grid &g, RecPtr mrows, double g
         if (tape.mfx_lat) row_st(tape.mfx_lat + r * p, i, tu);
         row_st(tape.u_lat + r * p, i, ul);
         row_st(tape.pv_lat + r * p, i, pt);
-        if (tape.dlat[0]) tape_upwind(tape.dlat, r * p + i, upwind_deriv(pv_scheme, order, wgt, ul, vf, 1, a1, a2, a3, a4));
+        if (tape.dlat[0]) tape_upwind(tape.dlat, r * p, i, upwind_deriv(pv_scheme, order, wgt, ul, vf, 1, a1, a2, a3, a4));
       }
       spt[k * n + i] = pt;
     }
