@@ -198,8 +198,8 @@ int flux_group(const AdvGrid &g, int ntr) { return FluxMap(g, ntr, 1).blocks() <
 // is infinite: it is a NaN then, and so is what the cells either side make of it.
 // A wavefront that finds its cells' sum over the tracers not finite forms them
 // anew by divisions, fluxes included, as the items of one tracer do.  The sum is
-// one or two additions a cell and tracer (720 x 361 x 8 tracers: 79.2 -> 80.0 us
-// a step; a test of each value took 81.1).
+// one operation a cell and tracer (720 x 361 x 8 tracers: 80.0 -> 80.6 us a
+// step; a test of each value took 81.1).
 __device__ __forceinline__ bool any_not_finite(double x) { return __builtin_expect(__any(!__builtin_isfinite(x)), 0); }
 // The lane's column for that second loop, newly known in each round: addresses
 // kept ahead of the loop took the kernel from 85 to 126 registers, 83 us a step.
@@ -323,7 +323,7 @@ __global__ void __launch_bounds__(NF, GROUPED ? 4 : 8) k_adv_inner(AdvGrid g, Me
     const double fs = sfy[t][threadIdx.x], fn = sfy[t][threadIdx.x + kWave];
     const double qx = qc - 0.5 * (div_rn((fx - fxw) * lel, ac, rac) - dvx * qc) * dt;
     const double qy = qc - 0.5 * (div_rn(fn * ln - fs * ls, ac, rac) - dvy * qc) * dt;
-    sum += qx + qy;
+    sum = __builtin_fma(qx, qy, sum);   // not finite unless both are
     if (upd) {
       const int64_t o = toff + t * p.tstride + ro;
       stu(p.qx + o, uiw, qx);
