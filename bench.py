@@ -9,11 +9,14 @@ rows), FP64, polar filter on, pc2, dt = 60 s, seeded balanced initial state
 captured HIP graph, inputs resident in HBM.
 
 Prints one JSON line.  value = grid-point-steps per second (nlon * nlat per
-step).  roofline: the dominant kernel's algorithmic bytes per launch over its
-mean launch time from gmc_kernel_times (a start and an end HIP event per
-launch on the library's stream, stamped by the dispatch) against 8 TB/s, with the HBM traffic per launch measured by
-rocprofv3 counters.  step_roofline: the algorithmic bytes of the whole step
-(35 FP64 field passes per grid point, 280 B/gp) over the step time.  cpu_baseline: the oracle (a scalar C
+step).  roofline: the algorithmic bytes of the step (35 FP64 field passes per
+grid point, 280 B/gp) over the step time against 8 TB/s, with the HBM traffic of
+a step's launches measured by rocprofv3 counters (profiles/); step_roofline is
+the same without the traffic.  three_kernel_form: each kernel's mean time from
+gmc_kernel_times (a start and an end HIP event per launch on the library's
+stream, stamped by the dispatch) with its algorithmic bytes; gmc_kernel_times
+runs the stage as three kernels on every grid, the timed step as k_stage
+launches, so these kernels are not part of the timed step.  cpu_baseline: the oracle (a scalar C
 restatement of the reference, gcc -O3, one thread as the reference runs) timed
 on a bounded sample of the same workload; cpu_baseline_all_cores: the same
 code with its row loops on OpenMP threads over the usable host CPUs.
@@ -36,11 +39,10 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
 BYTES_PER_GP_STEP = 280.0          # 35 FP64 field passes per pc2 step
-# compulsory bytes per grid point of one launch of each kernel class of the
-# three-kernel stage (which gmc_kernel_times runs on every grid; gmc_step at
-# 1440 x 721 spreads a stage over k_stage's three launches), mean over the
-# three stages (k_tend reads 4 fields in stage 1 and 5 in stages
-# 2-3 and writes 3; k_gzf reads 1, writes 2; k_uvf reads 5, writes 4)
+# compulsory bytes per grid point of one launch of each kernel of the
+# three-kernel stage, mean over the three stages (k_tend reads 4 fields in
+# stage 1 and 5 in stages 2-3 and writes 3; k_gzf reads 1, writes 2; k_uvf
+# reads 5, writes 4)
 KERNEL_BYTES_PER_GP = {"k_tend": 8.0 * (7 + 8 + 8) / 3, "k_gzf": 24.0, "k_uvf": 72.0}
 PROFILES = os.path.join(ROOT, "profiles")
 
@@ -768,7 +770,7 @@ def main():
     ms_step = ms.value / args.steps
     d1 = m.diagnose()
 
-    # per-kernel breakdown (launches one by one with events)
+    # the three kernels of the stage (launches one by one with events)
     kt = np.zeros(8)
     nk = C.c_int32()
     rc = m.lib.gmc_kernel_times(m.ctx, cfg["dt"], 3, capi.dptr(kt), 8, C.byref(nk))
@@ -781,9 +783,7 @@ def main():
         b = KERNEL_BYTES_PER_GP.get(name, 0.0) * gp
         kernels.append({"name": name, "avg_us": kt[k] * 1e3,
                         "bytes_per_launch": b, "gbs": b / (kt[k] * 1e-3) / 1e9 if kt[k] > 0 else 0.0})
-    dom = max(kernels, key=lambda x: x["avg_us"])
     step_gbs = BYTES_PER_GP_STEP * gp / (ms_step * 1e-3) / 1e9
-    traffic = profiled_traffic(args.config, dom["name"])
     result = {
         "metric": "grid-point-steps/s (FP64 SW pc2 step, 1 GPU)",
         "value": gp / (ms_step * 1e-3),
@@ -801,18 +801,18 @@ def main():
         "config": {"workload": f"shallow-water {args.config}: {cfg['nlon']}x{cfg['nlat']} C-grid, FP64, "
                                f"pc2, dt={cfg['dt']:g} s, polar filter on, seeded l<={cfg['lmax']}",
                    "nlon": cfg["nlon"], "nlat": cfg["nlat"], "dt": cfg["dt"], "time_scheme": "pc2"},
-        "roofline": {"bound": "hbm", "achieved": dom["gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": dom["gbs"] / HBM_PEAK_GBS,
-                     "traffic": traffic,
-                     "kernel": dom["name"],
-                     "scope": f"dominant kernel {dom['name']}: algorithmic bytes per launch "
-                              f"{KERNEL_BYTES_PER_GP[dom['name']]:.2f} B/grid point over its mean "
-                              "launch time (start and end HIP events of each launch on the library stream)"},
+        "roofline": {"bound": "hbm", "achieved": step_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                     "frac": step_gbs / HBM_PEAK_GBS,
+                     "traffic": profiled_traffic(args.config, "step"),
+                     "kernel": "the launches of a step",
+                     "scope": "whole pc2 step: 280 B/grid point algorithmic over the step time; traffic = HBM "
+                              "bytes of a step's launches from the profiler's counters"},
         "step_roofline": {"bound": "hbm", "achieved": step_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                           "frac": step_gbs / HBM_PEAK_GBS,
-                          "scope": "whole pc2 step (one graph launch): 280 B/grid point algorithmic"},
-        "dominant_kernel": dom,
-        "kernels": kernels,
+                          "scope": "whole pc2 step (graphs of 8 steps and of one): 280 B/grid point algorithmic"},
+        "three_kernel_form": {"kernels": kernels,
+                              "scope": "gmc_kernel_times: the stage as three kernels, which the timed step does "
+                                       "not launch where it runs k_stage"},
         "mass_rel_drift": float((d1[0] - d0[0]) / d0[0]),
     }
     if not args.no_cpu:

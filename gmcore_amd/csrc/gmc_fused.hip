@@ -1132,8 +1132,8 @@ __device__ __forceinline__ void band_stage(const Grid &g, RecPtr mrows, double g
 // us, 360 x 181 24.1 (62) -> 19.4 (55), 502 x 253 with damping 35 (90) -> 31
 // (85); the wider grids at kSpreadTiles.  A full tile takes 5 us from its
 // start to its last store; the band at a pole, 17 us at 360 columns, bounds
-// the small grids, the vector instructions and the loads of the tiles (two
-// workgroups a compute unit, 45 % of the issue slots) the large ones.
+// the small grids, the chains of the tiles (two workgroups a compute unit, the
+// VALU 34 % busy) and of the widest filter rows the large ones.
 //
 // A workgroup finds its work from its number and the kernel arguments alone: a
 // table would put one more trip to memory (about 1 us) before its first load.

@@ -139,7 +139,10 @@ int gmc_destroy(gmc_ctx *ctx);
 const char *gmc_last_error(const gmc_ctx *ctx);
 
 /* Copy one interior field between host and device state `level`
- * (1..3, block%state(level); tendencies use block%tend(level)). */
+ * (1..3, block%state(level); tendencies use block%tend(level)).  Both return
+ * when the copy is complete.  A download of 4 MB or more, here and in the other
+ * headers, is copied into the caller's array by up to three more host threads,
+ * which end before the call returns. */
 int gmc_upload(gmc_ctx *ctx, int32_t level, int32_t field, const double *host, int64_t ld);
 int gmc_download(gmc_ctx *ctx, int32_t level, int32_t field, double *host, int64_t ld);
 
@@ -163,7 +166,8 @@ int gmc_update_state(gmc_ctx *ctx, int32_t tend, int32_t old_level,
  * step_forward_backward, time_schemes_mod.F90:102-118, 244-288) followed by
  * damp_run (damp_mod.F90:49-63).  Level 3 is the intermediate state.  The
  * caller swaps old and new afterwards, as time_advance does.  Uses the fused
- * stage kernels. */
+ * stage kernels; the tendency levels are their scratch, and what they hold
+ * afterwards is undefined. */
 int gmc_time_integrate(gmc_ctx *ctx, int32_t old_level, int32_t new_level, double dt);
 
 /* `time_integrator` (time_schemes_mod.F90:244-288) with step =>

@@ -4,8 +4,8 @@ quotient from the correctly rounded reciprocal plus one fma correction.  The
 advection kernels divide by 3 and 6, and for several tracers by Courant numbers,
 areas and masses, the same way; pv and the tangential winds divide by depths
 through div_mid, whose reciprocal is two Newton steps from the hardware's
-estimate, and the upwind weights through div_root, with a root from an estimate as well.  The kernels stay
-bit-identical to the oracle only if these give the IEEE results.  This test
+estimate, and the upwind weights through div_root, with a root from an estimate
+as well.  The kernels stay bit-identical to the oracle only if these give the IEEE results.  This test
 compiles the header's own code for the host, the hardware's estimates replaced
 by exact ones with an error of up to 2^-22, and checks it against the host's
 quotients and roots: for every divisor of four real meshes (and adversarial

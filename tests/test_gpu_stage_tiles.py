@@ -56,7 +56,7 @@ def test_stage_forms_bitwise(nlon, nlat, long, option):
     a, b = make_gpu(st, ic), make_gpu(st, ic)
     for m in (a, b):
         m.prepare(1)
-        m.keep_derived()    # the taping variant: every intermediate of the star level
+        m.keep_derived()    # the taping variant (pv here, the others through the sums of diagnose)
     a.step(2)
     kt, nk = np.zeros(8), C.c_int32()
     assert b.lib.gmc_kernel_times(b.ctx, st.nl.dt_dyn, 2, dptr(kt), 8, C.byref(nk)) == 0

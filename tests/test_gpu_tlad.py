@@ -210,7 +210,9 @@ def _rand_at(nlon, nlat, seed, scale):
     return u, rng.standard_normal((nlat - 1, nlon)) * scale[1], rng.standard_normal((nlat, nlon)) * scale[2]
 
 
-@pytest.mark.parametrize("nlon,nlat,dt,coriolis", [(360, 181, 300.0, 1), (72, 37, 1800.0, 2)])
+@pytest.mark.parametrize("nlon,nlat,dt,coriolis", [(360, 181, 300.0, 1), (72, 37, 1800.0, 2),
+                                                   # taping stages of three launches, with whole tiles in each
+                                                   (722, 601, 100.0, 1)])
 def test_dot_product_chunked_rows_and_coriolis2(nlon, nlat, dt, coriolis):
     """At 360 x 181 the adjoint's row kernels cut the polar rows into
     column chunks that read each other's columns as halo; with Coriolis
